@@ -20,6 +20,32 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
+// D += A B over four records in the plan's own precision:
+// v_mfma_f32_16x16x4_f32 / v_mfma_f64_16x16x4_f64 (lane l holds A row l % 16,
+// B column l % 16, K element l / 16; D column l % 16, rows row(l, 0..3)).
+template <typename T>
+struct ExactMma;
+
+template <>
+struct ExactMma<float> {
+    using Acc = f32x4;
+    __device__ static Acc mma(float a, float b, const Acc &c)
+    {
+        return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+    }
+    __device__ static int row(int lane, int r) { return 4 * (lane >> 4) + r; }
+};
+
+template <>
+struct ExactMma<double> {
+    typedef double Acc __attribute__((ext_vector_type(4)));
+    __device__ static Acc mma(double a, double b, const Acc &c)
+    {
+        return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+    }
+    __device__ static int row(int lane, int r) { return 4 * r + (lane >> 4); }
+};
+
 // mma: v_mfma_f32_32x32x16 (lane l holds A row l % 32, B column l % 32, K
 // elements 8 (l / 32) .. +7); mma16: v_mfma_f32_16x16x32 (lane l holds A row
 // l % 16, B column l % 16, K elements 8 (l / 16) .. +7; D column l % 16, rows

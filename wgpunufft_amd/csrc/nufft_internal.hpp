@@ -66,6 +66,17 @@ struct EsKernel {
     double evaluate(double distance) const;
 };
 
+// Coefficients of the kernel's panel polynomials.  A support of w cells has
+// its weights at distances t - (w - 1) / 2 + x, t = 0 .. w - 1, x in
+// [-1/2, 1/2); cells t and w - 1 - t are E_t(x^2) + x O_t(x^2) and
+// E_t(x^2) - x O_t(x^2).  For t = 1 .. (w - 1) / 2: `even` coefficients of
+// E_t, then `odd` of O_t, lowest power first (the middle cell of an odd
+// width has O = 0).  The support's first and last cells, where the kernel's
+// square root ends, have no polynomial.
+constexpr int kPanelEven32 = 6, kPanelOdd32 = 5;
+constexpr int kPanelEven64 = 8, kPanelOdd64 = 7;
+std::vector<double> es_panel_coefficients(const EsKernel &k, int even, int odd);
+
 // Returns false (and sets the last error) for an unsupported tolerance.
 bool es_kernel_for_tolerance(double eps, double sigma, EsKernel *out);
 bool fft_length_supported(int64_t n);
@@ -125,6 +136,7 @@ struct GridParams {
     int width;
     double half_width;
     double beta;
+    const void *panels;  // the kernel's panel polynomials in the plan's type
     AxisParams ax[kMaxDims];
     int64_t nbins;
     int64_t fine_total;

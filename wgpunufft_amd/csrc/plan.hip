@@ -195,6 +195,18 @@ bool Plan::init_common()
         !validate_f32_rounding(std::vector<int64_t>(n_modes, n_modes + dim), eps, sigma, precision,
                                coeffs))
         return false;
+    // the kernel's panel polynomials behind the amplitudes, in the plan's type
+    panel_off = (int64_t)table.size();
+    if (precision == Precision::F32) {
+        const std::vector<double> pc =
+            es_panel_coefficients(kernel, kPanelEven32, kPanelOdd32);
+        const std::vector<float> pf(pc.begin(), pc.end());
+        table.resize(table.size() + (pf.size() + 1) / 2);
+        if (!pf.empty()) std::memcpy(table.data() + panel_off, pf.data(), 4 * pf.size());
+    } else {
+        for (double v : es_panel_coefficients(kernel, kPanelEven64, kPanelOdd64))
+            table.push_back(v);
+    }
     if (!hip_ok(hipMalloc(&d_inv_phihat, sizeof(double) * table.size()), "amplitude table"))
         return false;
     if (!hip_ok(hipMemcpy(d_inv_phihat, table.data(), sizeof(double) * table.size(),
@@ -233,6 +245,7 @@ GridParams Plan::grid_params(const int64_t *side) const
     g.width = kernel.width;
     g.half_width = kernel.half_width();
     g.beta = kernel.beta;
+    g.panels = d_inv_phihat + panel_off;
     g.nbins = 1;
     g.fine_total = fine_total;
     for (int a = 0; a < kMaxDims; ++a) {

@@ -42,6 +42,7 @@ struct Plan {
     int64_t fine_total = 1, mode_total = 1;
     int64_t phihat_off[kMaxDims] = {};
     double *d_inv_phihat = nullptr;
+    int64_t panel_off = 0;  // of the panel polynomials in d_inv_phihat, in doubles
     SpreadLayout layout;
     SpreadParams sp{};         // plain spread: the row tiles where `sweep`, else sp_generic
     SpreadParams sp_generic{};  // output-stationary blocks of the reference layout

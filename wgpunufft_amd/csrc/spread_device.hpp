@@ -22,6 +22,67 @@ __device__ inline T es_weight(T d, int w, T beta)
         return exp(beta * (sqrt(q) - 1.0));
 }
 
+// Coefficients read by scalar loads: the same address for every lane.
+template <typename T>
+using UniformPtr = const __attribute__((address_space(4))) T *;
+
+template <typename T>
+__device__ inline UniformPtr<T> panel_coefficients(const GridParams &g)
+{
+    return (UniformPtr<T>)(uintptr_t)g.panels;
+}
+
+// The weight of a support's first or last cell, at distance d: directly,
+// for W known (no division), FP32 as exp2 of -beta log2(e) s^2 / (1 + sqrt q)
+// on the hardware square root, reciprocal and exponential.  That form has no
+// cancellation near the centre, so its error (2e-7 of the exponent) stays
+// below the correctly rounded sqrt(q) - 1 form's.
+template <typename T, int W>
+__device__ inline T es_edge_weight(T d, T beta)
+{
+    const T s = d * (T)(2.0 / W);
+    const T q = (T)1 - s * s;
+    if constexpr (sizeof(T) == 4) {
+        const float r = __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_sqrtf(fmaxf(q, 0.0f)));
+        const float e = __builtin_amdgcn_exp2f(-1.44269504f * beta * (s * s) * r);
+        return q > 0.0f ? e : 0.0f;
+    } else {
+        return q > 0.0 ? exp(beta * (sqrt(q) - 1.0)) : 0.0;
+    }
+}
+
+// The W weights of one axis of a record, put(t, weight) for cell t of its
+// support, from its offset (start - position, in [-W/2, 1 - W/2)).  Inner
+// cells come in pairs from the panel polynomials (about 5 FMAs a weight in
+// FP32 and 8 in FP64, where sqrt and exp take 30 and 60 instructions),
+// accurate to the type's rounding; the end cells directly.
+template <typename T, int W, typename Put>
+__device__ __forceinline__ void es_axis_weights(T off, T beta, UniformPtr<T> c, Put put)
+{
+    constexpr int NE = sizeof(T) == 4 ? kPanelEven32 : kPanelEven64;
+    constexpr int NO = sizeof(T) == 4 ? kPanelOdd32 : kPanelOdd64;
+    const T x = off + (T)(0.5 * (W - 1));
+    const T x2 = x * x;
+    put(0, es_edge_weight<T, W>(off, beta));
+    put(W - 1, es_edge_weight<T, W>(off + (T)(W - 1), beta));
+#pragma unroll
+    for (int t = 1; t <= (W - 1) / 2; ++t) {
+        UniformPtr<T> e = c + (t - 1) * (NE + NO), o = e + NE;
+        T even = e[NE - 1];
+#pragma unroll
+        for (int i = NE - 2; i >= 0; --i) even = __builtin_elementwise_fma(even, x2, e[i]);
+        if (2 * t == W - 1) {
+            put(t, even);
+        } else {
+            T odd = o[NO - 1];
+#pragma unroll
+            for (int i = NO - 2; i >= 0; --i) odd = __builtin_elementwise_fma(odd, x2, o[i]);
+            put(t, __builtin_elementwise_fma(x, odd, even));
+            put(W - 1 - t, __builtin_elementwise_fma(-x, odd, even));
+        }
+    }
+}
+
 // The FP32 weight from the hardware square root and base-2 exponential
 // (v_sqrt_f32, v_exp_f32): a few ulp where the weight is near one and an
 // absolute error below 1e-12 at the support edges (weight about e^-beta),
