@@ -76,49 +76,48 @@ bool es_kernel_for_tolerance(double eps, double sigma, EsKernel *out)
 
 std::vector<double> es_panel_coefficients(const EsKernel &k, int even, int odd)
 {
-    // Chebyshev interpolation of every panel on 32 nodes in long double, cut
+    // Chebyshev interpolation of every panel on 20 nodes in long double, cut
     // at the degree kept (near-minimax: the series falls geometrically, the
     // kernel's singularities lying at least one panel away), then rewritten
     // in powers of x.
-    constexpr int nodes = 32;
-    struct Cosines {
-        long double v[4 * nodes];  // cos(pi i / (2 nodes))
-        Cosines()
+    constexpr int nodes = 20, terms = 16;
+    struct Tables {
+        long double cosine[4 * nodes];    // cos(pi i / (2 nodes))
+        long double power[terms][terms];  // T_j(2 x) = sum_i power[j][i] x^i
+        Tables()
         {
             for (int i = 0; i < 4 * nodes; ++i)
-                v[i] = cosl(3.141592653589793238462643383279502884L * i / (2 * nodes));
+                cosine[i] = cosl(3.141592653589793238462643383279502884L * i / (2 * nodes));
+            for (int j = 0; j < terms; ++j)
+                for (int i = 0; i < terms; ++i)
+                    power[j][i] = j < 2 ? (i == j ? (j ? 2.0L : 1.0L) : 0.0L)
+                                        : (i ? 4.0L * power[j - 1][i - 1] : 0.0L) - power[j - 2][i];
         }
     };
-    static const Cosines cosines;
-    const int degree = std::max(2 * even - 2, 2 * odd - 1);
+    static const Tables tab;
+    const int degree = std::min(terms - 1, std::max(2 * even - 2, 2 * odd - 1));
     std::vector<double> out;
+    out.reserve((size_t)std::max((k.width - 1) / 2, 0) * (even + odd));
     for (int t = 1; t <= (k.width - 1) / 2; ++t) {
-        std::vector<long double> cheb(degree + 1, 0.0L);
+        long double cheb[terms] = {};
         for (int i = 0; i < nodes; ++i) {
-            const long double d = t - 0.5L * (k.width - 1) + 0.5L * cosines.v[2 * i + 1];
+            const long double d = t - 0.5L * (k.width - 1) + 0.5L * tab.cosine[2 * i + 1];
             const long double s = 2.0L * d / k.width;
             const long double f =
-                expl((long double)k.beta * (sqrtl(std::max(1.0L - s * s, 0.0L)) - 1.0L));
+                expl((long double)k.beta * (sqrtl(std::max(1.0L - s * s, 0.0L)) - 1.0L)) *
+                (2.0L / nodes);
             for (int j = 0; j <= degree; ++j)
-                cheb[j] += f * cosines.v[j * (2 * i + 1) % (4 * nodes)] *
-                           (j == 0 ? 1.0L : 2.0L) / nodes;
+                cheb[j] += f * tab.cosine[j * (2 * i + 1) % (4 * nodes)];
         }
-        // T_j(u) in powers of u by the recurrence T_{j+1} = 2 u T_j - T_{j-1}
-        std::vector<long double> power(degree + 1, 0.0L), t0(degree + 1, 0.0L),
-            t1(degree + 1, 0.0L), t2(degree + 1, 0.0L);
-        t0[0] = 1.0L;
-        t1[1] = 1.0L;
-        for (int j = 0; j <= degree; ++j) {
-            for (int i = 0; i <= j; ++i) power[i] += cheb[j] * t0[i];
-            for (int i = 0; i <= degree; ++i) t2[i] = (i ? 2.0L * t1[i - 1] : 0.0L) - t0[i];
-            t0 = t1;
-            t1 = t2;
-        }
+        cheb[0] *= 0.5L;
+        const auto power = [&](int i) {
+            long double v = 0.0L;
+            for (int j = i; j <= degree; j += 2) v += cheb[j] * tab.power[j][i];
+            return (double)v;
+        };
         const bool middle = 2 * t == k.width - 1;
-        for (int i = 0; i < even; ++i) out.push_back((double)(power[2 * i] * powl(2.0L, 2 * i)));
-        for (int i = 0; i < odd; ++i)
-            out.push_back(middle ? 0.0
-                                 : (double)(power[2 * i + 1] * powl(2.0L, 2 * i + 1)));
+        for (int i = 0; i < even; ++i) out.push_back(power(2 * i));
+        for (int i = 0; i < odd; ++i) out.push_back(middle ? 0.0 : power(2 * i + 1));
     }
     return out;
 }

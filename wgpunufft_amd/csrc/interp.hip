@@ -294,6 +294,7 @@ __device__ __forceinline__ void interp_tile3(typename Complex2<T>::type *tile, c
     constexpr int RX = Shape::RX;
     const int64_t n0 = g.ax[0].n, n1 = g.ax[1].n, n2 = g.ax[2].n;
     const T beta = (T)g.beta;
+    const UniformPtr<T> panels = panel_coefficients<T>(g);
     // tile loads: every wavefront fills RPW rows of RX cells at a time, each
     // lane keeping its x cell
     constexpr int ROWS = EY * EZ;
@@ -333,24 +334,7 @@ __device__ __forceinline__ void interp_tile3(typename Complex2<T>::type *tile, c
             int64_t ws = wrapped_start(start, g.ax[a].n);
             int64_t o = a == 0 ? x0 : (a == 1 ? y0 : z0);
             l[a] = (int)(ws - o);
-            if constexpr (sizeof(T) == 4) {
-                // the kernel at distances j + off: scaled distance off * 2/w +
-                // j * 2/w, exponent as one FMA (hardware sqrt / exp2)
-                constexpr float two_over_w = 2.0f / (float)W;
-                const float u0 = (float)off * two_over_w;
-                const float bl = (float)beta * 1.44269504088896341f;
-#pragma unroll
-                for (int j = 0; j < W; ++j) {
-                    const float sv = u0 + (float)j * two_over_w;
-                    const float q = __builtin_fmaf(-sv, sv, 1.0f);
-                    const float e = __builtin_amdgcn_exp2f(
-                        __builtin_fmaf(__builtin_amdgcn_sqrtf(q), bl, -bl));
-                    wt[a][j] = q > 0.0f ? e : 0.0f;
-                }
-            } else {
-#pragma unroll
-                for (int j = 0; j < W; ++j) wt[a][j] = es_w<T>((T)j + (T)off, W, beta);
-            }
+            es_axis_weights<T, W>((T)off, beta, panels, [&](int j, T wj) { wt[a][j] = wj; });
         }
         T sre = (T)0, sim = (T)0;
         if constexpr (kPairs) {
@@ -478,6 +462,142 @@ __global__ __launch_bounds__(THREADS) void k_interp_tiled3_many(
 }
 
 // ---------------------------------------------------------------------
+// LDS-tiled 3D interpolation of wide FP64 kernels (widths 9..16).  Same tiles
+// and work items as above, four lanes (a quad) per point: lane a < 3 computes
+// the weights of axis a, the quad shares them by DPP moves, and lane j sums
+// the planes dz = j, j + 4, ... of the point's window, which are then added
+// in a fixed order.  The tile shrinks with the width so that tile and halo
+// leave room for two workgroups in a CU's LDS up to width 14.
+// Bound by the LDS: w^3 cells of 16 bytes a point (16 GB for 1e6 points at
+// width 10, 0.2 ms at 128 bytes a clock and CU).
+// ---------------------------------------------------------------------
+template <int W>
+struct WideTile3 {
+    static constexpr int TX = wide3_side(W, 0), TY = wide3_side(W, 1), TZ = wide3_side(W, 2);
+    static constexpr int EX = TX + W - 1, EY = TY + W - 1, EZ = TZ + W - 1;
+};
+
+constexpr int kWide3Threads = 256, kWide3Points = 1024;
+
+// The value of quad lane SEL of every lane's quad.
+template <int SEL>
+__device__ inline double quad_bcast(double v)
+{
+    constexpr int ctrl = SEL * 0x55;
+    const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), ctrl, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), ctrl, 0xf, 0xf, true);
+    return __hiloint2double(hi, lo);
+}
+
+// v plus the value of the quad lane whose index differs in the bits of X.
+template <int X>
+__device__ inline double quad_add_xor(double v)
+{
+    constexpr int ctrl = (0 ^ X) | ((1 ^ X) << 2) | ((2 ^ X) << 4) | ((3 ^ X) << 6);
+    const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), ctrl, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), ctrl, 0xf, 0xf, true);
+    return v + __hiloint2double(hi, lo);
+}
+
+template <int W>
+__global__ __launch_bounds__(kWide3Threads) void k_interp_wide3(
+    int64_t M, const uint32_t *__restrict__ sorted, const uint32_t *__restrict__ offsets,
+    const uint32_t *__restrict__ item_off, const double *__restrict__ coords, GridParams g,
+    const double *__restrict__ grid, double *__restrict__ out)
+{
+    using Shape = WideTile3<W>;
+    constexpr int TX = Shape::TX, TY = Shape::TY, TZ = Shape::TZ;
+    constexpr int EX = Shape::EX, EY = Shape::EY, EZ = Shape::EZ;
+    __shared__ double2 tile[EX * EY * EZ];
+    const int64_t n0 = g.ax[0].n, n1 = g.ax[1].n, n2 = g.ax[2].n;
+    const int64_t n_items = item_off[g.nbins];
+    const double *gv = grid + 2 * (int64_t)blockIdx.y * g.fine_total;
+    double *out_v = out + 2 * (int64_t)blockIdx.y * M;
+    const UniformPtr<double> panels = panel_coefficients<double>(g);
+    constexpr int RPW = 64 / EX;  // rows a wavefront loads at a time
+    const int lane = threadIdx.x & 63;
+    const int rsub = lane / EX, lx = lane % EX;
+    const int j = lane & 3, axis = j < 2 ? j : 2;
+    for (int64_t item = blockIdx.x; item < n_items; item += gridDim.x) {
+        const TileItem3 ti = tile_item3(item, item_off, g, TX, TY, TZ);
+        const int64_t first = (int64_t)offsets[ti.b] + ti.k * kWide3Points;
+        int64_t last = first + kWide3Points;
+        if (last > (int64_t)offsets[ti.b + 1]) last = offsets[ti.b + 1];
+        if (rsub < RPW) {
+            int64_t gx = ti.x0 + lx;
+            gx = gx >= n0 ? gx - n0 : gx;
+            for (int r = (int)(threadIdx.x >> 6) * RPW + rsub; r < EY * EZ;
+                 r += kWide3Threads / 64 * RPW) {
+                int64_t gy = ti.y0 + r % EY, gz = ti.z0 + r / EY;
+                gy = gy >= n1 ? gy - n1 : gy;
+                gz = gz >= n2 ? gz - n2 : gz;
+                tile[r * EX + lx] = *(const double2 *)(gv + 2 * (gx + n0 * (gy + n1 * gz)));
+            }
+        }
+        __syncthreads();
+        for (int64_t s = first + (threadIdx.x >> 2); s < last; s += kWide3Threads / 4) {
+            const uint32_t idx = sorted[s];
+            double x[3];
+#pragma unroll
+            for (int a = 0; a < 3; ++a) x[a] = coords[(int64_t)idx * 3 + a];
+            const bool reach = FoldTraits<double>::in_reach(x[0]) &&
+                               FoldTraits<double>::in_reach(x[1]) &&
+                               FoldTraits<double>::in_reach(x[2]);
+            int l[3];
+            double mine = 0.0;  // the offset of the lane's axis
+#pragma unroll
+            for (int a = 0; a < 3; ++a) {
+                int64_t start;
+                double off;
+                support_start<double>(x[a], reach, g, a, &start, &off);
+                const int64_t o = a == 0 ? ti.x0 : (a == 1 ? ti.y0 : ti.z0);
+                l[a] = (int)(wrapped_start(start, g.ax[a].n) - o);
+                if (a == axis) mine = off;
+            }
+            double wt[W], wx[W], wy[W];
+            es_axis_weights<double, W>(mine, g.beta, panels, [&](int t, double w) { wt[t] = w; });
+#pragma unroll
+            for (int t = 0; t < W; ++t) {
+                wx[t] = quad_bcast<0>(wt[t]);
+                wy[t] = quad_bcast<1>(wt[t]);
+                wt[t] = quad_bcast<2>(wt[t]);
+            }
+            double sre = 0.0, sim = 0.0;
+#pragma unroll
+            for (int k = 0; k < W; k += 4) {
+                // the lane's plane k + j; past the window its weight is zero
+                double wz = wt[k];
+                if (k + 1 < W) wz = j == 1 ? wt[k + 1] : wz;
+                if (k + 2 < W) wz = j == 2 ? wt[k + 2] : wz;
+                if (k + 3 < W) wz = j == 3 ? wt[k + 3] : wz;
+                const int dz = k + j < W ? k + j : W - 1;
+                wz = k + j < W ? wz : 0.0;
+                const double2 *plane = tile + ((l[2] + dz) * EY + l[1]) * EX + l[0];
+                double pre = 0.0, pim = 0.0;
+#pragma unroll
+                for (int dy = 0; dy < W; ++dy) {
+                    double rre = 0.0, rim = 0.0;
+#pragma unroll
+                    for (int dx = 0; dx < W; ++dx) {
+                        const double2 cv = plane[dy * EX + dx];
+                        rre += wx[dx] * cv.x;
+                        rim += wx[dx] * cv.y;
+                    }
+                    pre += wy[dy] * rre;
+                    pim += wy[dy] * rim;
+                }
+                sre += wz * pre;
+                sim += wz * pim;
+            }
+            sre = quad_add_xor<2>(quad_add_xor<1>(sre));
+            sim = quad_add_xor<2>(quad_add_xor<1>(sim));
+            if (j < 2) out_v[2 * (int64_t)idx + j] = j == 0 ? sre : sim;
+        }
+        __syncthreads();
+    }
+}
+
+// ---------------------------------------------------------------------
 // LDS-tiled 2D interpolation: type-2 bins are tiles of TX x TY cells of
 // support starts; workgroups take bins with a stride (a 2D tile holds a few
 // hundred points at most densities, so a bin is one unit of work).  The
@@ -538,6 +658,7 @@ __global__ __launch_bounds__(THREADS) void k_interp_tiled2(
             gv = grid0 + 2 * v * g0.fine_total;
             vo = v * M;
         }
+        const UniformPtr<T> panels = panel_coefficients<T>(g);
         const int64_t n0 = g.ax[0].n, n1 = g.ax[1].n;
         const int64_t x0 = (bin % g.ax[0].bins) * TX, y0 = (bin / g.ax[0].bins) * TY;
         if (rsub < RPW) {
@@ -565,22 +686,8 @@ __global__ __launch_bounds__(THREADS) void k_interp_tiled2(
                 support_start<T>(x[a], reach, g, a, &start, &off);
                 const int64_t ws = wrapped_start(start, g.ax[a].n);
                 l[a] = (int)(ws - (a == 0 ? x0 : y0));
-                if constexpr (sizeof(T) == 4) {
-                    constexpr float two_over_w = 2.0f / (float)W;
-                    const float u0 = (float)off * two_over_w;
-                    const float bl = (float)g.beta * 1.44269504088896341f;
-#pragma unroll
-                    for (int j = 0; j < W; ++j) {
-                        const float sv = u0 + (float)j * two_over_w;
-                        const float q = __builtin_fmaf(-sv, sv, 1.0f);
-                        const float e = __builtin_amdgcn_exp2f(
-                            __builtin_fmaf(__builtin_amdgcn_sqrtf(q), bl, -bl));
-                        wt[a][j] = q > 0.0f ? e : 0.0f;
-                    }
-                } else {
-#pragma unroll
-                    for (int j = 0; j < W; ++j) wt[a][j] = es_w<T>((T)j + (T)off, W, (T)g.beta);
-                }
+                es_axis_weights<T, W>((T)off, (T)g.beta, panels,
+                                      [&](int j, T wj) { wt[a][j] = wj; });
             }
             T sre = (T)0, sim = (T)0;
             if constexpr (kPairs) {
@@ -663,10 +770,23 @@ bool launch_tiled2_w(int w, int64_t M, int64_t vectors, const uint32_t *sorted,
         MNUFFT_TILED2(6)
         MNUFFT_TILED2(7)
         MNUFFT_TILED2(8)
-    default:
-        set_error("tiled interpolation needs a kernel width <= 8");
-        return false;
+    default: break;
     }
+    if constexpr (sizeof(T) == 8 && !MANY) {
+        switch (w) {
+            MNUFFT_TILED2(9)
+            MNUFFT_TILED2(10)
+            MNUFFT_TILED2(11)
+            MNUFFT_TILED2(12)
+            MNUFFT_TILED2(13)
+            MNUFFT_TILED2(14)
+            MNUFFT_TILED2(15)
+            MNUFFT_TILED2(16)
+        default: break;
+        }
+    }
+    set_error("tiled 2D interpolation needs a kernel width <= 8 (FP32) or <= 16 (FP64)");
+    return false;
 #undef MNUFFT_TILED2
 }
 
@@ -685,6 +805,26 @@ bool launch_tiled(int64_t M, int64_t vectors, const uint32_t *sorted, const uint
     k_interp_tiled3<T, W, TX, TY, TZ, THREADS, P><<<grid3, THREADS, 0, stream>>>(
         M, sorted, offsets, item_off, coords, g, grid, out);
     return hip_ok(hipGetLastError(), "tiled interpolation launch");
+}
+
+template <int W>
+bool launch_wide3(int64_t M, int64_t vectors, const uint32_t *sorted, const uint32_t *offsets,
+                  uint32_t *item_off, const double *coords, const GridParams &g,
+                  const double *grid, double *out, hipStream_t stream)
+{
+    for (int a = 0; a < 3; ++a)
+        if (1 << g.ax[a].shift != wide3_side(W, a)) {
+            set_error("wide tiled interpolation: unsupported tile geometry");
+            return false;
+        }
+    const int64_t n = g.nbins + 1;
+    k_item_counts<<<(unsigned)((n + 255) / 256), 256, 0, stream>>>(
+        g.nbins, (uint32_t)kWide3Points, offsets, item_off);
+    scan_u32(item_off, n, item_off + n, item_off, stream);
+    const int64_t items = std::min<int64_t>(g.nbins + M / kWide3Points + 64, 16384);
+    k_interp_wide3<W><<<dim3((unsigned)items, (unsigned)vectors), kWide3Threads, 0, stream>>>(
+        M, sorted, offsets, item_off, coords, g, grid, out);
+    return hip_ok(hipGetLastError(), "wide tiled interpolation launch");
 }
 
 template <typename T, int W>
@@ -798,6 +938,28 @@ template bool interpolate_tiled3<float>(int64_t, int64_t, const uint32_t *, cons
 template bool interpolate_tiled3<double>(int64_t, int64_t, const uint32_t *, const uint32_t *,
                                          uint32_t *, const double *, const GridParams &,
                                          const double *, double *, hipStream_t);
+
+bool interpolate_wide3(int64_t M, int64_t vectors, const uint32_t *sorted,
+                       const uint32_t *offsets, uint32_t *item_off, const double *coords,
+                       const GridParams &g, const double *grid, double *out, hipStream_t stream)
+{
+    if (M == 0) return true;
+#define MNUFFT_WIDE3(Wd)                                                                          \
+    case Wd:                                                                                      \
+        return launch_wide3<Wd>(M, vectors, sorted, offsets, item_off, coords, g, grid, out, stream)
+    switch (g.width) {
+        MNUFFT_WIDE3(9);
+        MNUFFT_WIDE3(10);
+        MNUFFT_WIDE3(11);
+        MNUFFT_WIDE3(12);
+        MNUFFT_WIDE3(13);
+        MNUFFT_WIDE3(14);
+        MNUFFT_WIDE3(15);
+        MNUFFT_WIDE3(16);
+    default: set_error("wide tiled interpolation needs a kernel width of 9..16"); return false;
+    }
+#undef MNUFFT_WIDE3
+}
 
 bool interpolate_tiled3_many(const uint32_t *sorted, const uint32_t *offsets, uint32_t *item_off,
                              int64_t nbins, const BatchProblem *probs, int nprob,

@@ -20,7 +20,19 @@ template <int D, typename T>
 bool interpolate_many(const uint32_t *sorted, const BatchProblem *probs, int nprob,
                       int64_t item_begin, int64_t items, int width, hipStream_t stream);
 
-// 2D, width <= 8, bins of 8 x 8 cells: tiles staged in LDS (like the 3D
+// Sides of the wide FP64 tiled interpolation's tiles (and of its plans' bins)
+// along axis a at kernel width w.
+constexpr int wide3_side(int w, int a)
+{
+    return w <= 10 ? 8 : w == 11 ? (a < 2 ? 8 : 4) : w == 12 ? (a < 1 ? 8 : 4) : 4;
+}
+
+// 3D FP64, width 9..16, bins of wide3_side cells: as interpolate_tiled3.
+bool interpolate_wide3(int64_t M, int64_t vectors, const uint32_t *sorted,
+                       const uint32_t *offsets, uint32_t *item_off, const double *coords,
+                       const GridParams &g, const double *grid, double *out, hipStream_t stream);
+
+// 2D, width <= 8 (FP64: 16), bins of 8 x 8 cells: tiles staged in LDS (like the 3D
 // tiled interpolation), one workgroup per bin.
 template <typename T>
 bool interpolate_tiled2(int64_t M, int64_t vectors, const uint32_t *sorted,

@@ -301,9 +301,19 @@ bool Plan::tiled_interp() const
     return true;
 }
 
+// Wide FP64 kernels: the grid qualifies for the wide tiled interpolation
+// (every axis at least a tile and its halo long).
+bool Plan::wide3_interp() const
+{
+    if (dim != 3 || precision == Precision::F32 || kernel.width <= 8) return false;
+    for (int a = 0; a < 3; ++a)
+        if (fine[a] < wide3_side(kernel.width, a) + kernel.width - 1) return false;
+    return true;
+}
+
 bool Plan::tiled2_interp() const
 {
-    if (dim != 2 || kernel.width > 8) return false;
+    if (dim != 2 || kernel.width > (precision == Precision::F32 ? 8 : 16)) return false;
     for (int a = 0; a < 2; ++a)
         if (fine[a] < 8 + kernel.width - 1 || fine[a] < 8) return false;
     return true;
@@ -312,8 +322,10 @@ bool Plan::tiled2_interp() const
 GridParams Plan::type2_geometry() const
 {
     int64_t side[kMaxDims] = {1, 1, 1, 1, 1, 1, 1, 1};
+    const bool wide = wide3_interp();
     for (int a = 0; a < dim; ++a) {
         int64_t s = dim >= 4 ? 4 : dim == 3 ? (tiled_interp() ? 8 : 4) : dim == 2 ? 8 : 32;
+        if (wide) s = wide3_side(kernel.width, a);
         side[a] = std::min<int64_t>(s, pow2_ceil(fine[a]));
     }
     return grid_params(side);
@@ -698,6 +710,15 @@ bool Plan::execute_t(int64_t active, const T *in, T *out, hipStream_t stream, bo
             if (!ensure_items(gp.nbins + 1 + scan_tiles(gp.nbins + 1) + 1)) return false;
             if (!interpolate_tiled3<T>(M, active, sorter.sorted(), sorter.offsets(), item_off,
                                        (const T *)points, gp, (const T *)grid, out, stream))
+                return false;
+        } else if (D == 3 && sizeof(T) == 8 && wide3_interp() && M >= 8 * gp.nbins) {
+            // a tile costs its halo's loads, as much as gathering two to
+            // five points (tile and halo over w^3 cells): from 8 points a
+            // tile on
+            if (!ensure_items(gp.nbins + 1 + scan_tiles(gp.nbins + 1) + 1)) return false;
+            if (!interpolate_wide3(M, active, sorter.sorted(), sorter.offsets(), item_off,
+                                   (const double *)points, gp, (const double *)grid,
+                                   (double *)out, stream))
                 return false;
         } else if (D == 2 && tiled2_interp()) {
             if (!interpolate_tiled2<T>(M, active, sorter.sorted(), sorter.offsets(),

@@ -33,25 +33,25 @@ __device__ inline UniformPtr<T> panel_coefficients(const GridParams &g)
 }
 
 // The weight of a support's first or last cell, at distance d: directly,
-// for W known (no division), FP32 as exp2 of -beta log2(e) s^2 / (1 + sqrt q)
-// on the hardware square root, reciprocal and exponential.  That form has no
-// cancellation near the centre, so its error (2e-7 of the exponent) stays
-// below the correctly rounded sqrt(q) - 1 form's.
+// for W known (no division), FP32 on the hardware square root and base-2
+// exponential (these cells' weights are small from width 4 on, so the
+// cancellation in sqrt(q) - 1 does not show).
 template <typename T, int W>
 __device__ inline T es_edge_weight(T d, T beta)
 {
     const T s = d * (T)(2.0 / W);
     const T q = (T)1 - s * s;
     if constexpr (sizeof(T) == 4) {
-        const float r = __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_sqrtf(fmaxf(q, 0.0f)));
-        const float e = __builtin_amdgcn_exp2f(-1.44269504f * beta * (s * s) * r);
+        const float bl = 1.44269504f * beta;
+        const float e = __builtin_amdgcn_exp2f(
+            __builtin_fmaf(__builtin_amdgcn_sqrtf(q), bl, -bl));
         return q > 0.0f ? e : 0.0f;
     } else {
         return q > 0.0 ? exp(beta * (sqrt(q) - 1.0)) : 0.0;
     }
 }
 
-// The W weights of one axis of a record, put(t, weight) for cell t of its
+// The W weights of one axis of a point, put(t, weight) for cell t of its
 // support, from its offset (start - position, in [-W/2, 1 - W/2)).  Inner
 // cells come in pairs from the panel polynomials (about 5 FMAs a weight in
 // FP32 and 8 in FP64, where sqrt and exp take 30 and 60 instructions),
