@@ -614,6 +614,7 @@ int mnufft_autotune(mnufft_plan plan, int64_t active_batch, int64_t M, const voi
             uint32_t light;
         };
         const Knob base{p.plain_rows, p.rows_side0, p.spreader.light_limit};
+        const bool base_auto = p.spreader.auto_split;
         std::vector<Knob> knobs;
         const bool rows = p.sweep || (p.rows2 && p.spread_method == mnufft::SpreadMethod::Plain);
         if (rows && p.spread_method == mnufft::SpreadMethod::Plain)
@@ -634,6 +635,7 @@ int mnufft_autotune(mnufft_plan plan, int64_t active_batch, int64_t M, const voi
             p.plain_rows = cand.plain_rows;
             p.rows_side0 = cand.side0;
             p.spreader.light_limit = cand.light;
+            p.spreader.auto_split = base_auto && cand.light == base.light;
             ok = p.set_points(M, d_points, st) && p.execute(active_batch, d_in, d_out, st);
             ok = ok && mnufft::hip_ok(hipEventRecord(e0, st), "autotune event");
             for (int r = 0; r < repeats && ok; ++r)
@@ -654,6 +656,7 @@ int mnufft_autotune(mnufft_plan plan, int64_t active_batch, int64_t M, const voi
         p.plain_rows = keep.plain_rows;
         p.rows_side0 = keep.side0;
         p.spreader.light_limit = keep.light;
+        p.spreader.auto_split = base_auto && keep.light == base.light;
         if (!ok) return MNUFFT_ERROR_GPU;
         // without dense bins their scratch is given back (it cannot be
         // needed before the threshold changes again)
@@ -701,6 +704,7 @@ int mnufft_set_spread_tuning(mnufft_plan plan, int64_t light_limit, int64_t min_
     Plan &q = p.type == 3 && p.outer ? *p.outer : p;
     if (light_limit) q.spreader.light_limit = (uint32_t)light_limit;
     if (min_part) q.spreader.min_part = (uint32_t)min_part;
+    if (light_limit || min_part) q.spreader.auto_split = false;
     if (part_budget_bytes) q.spreader.budget_bytes = part_budget_bytes;
     return MNUFFT_SUCCESS;
 }

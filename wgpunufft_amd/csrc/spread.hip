@@ -35,8 +35,11 @@ constexpr int kKw = 16;  // weights per axis staged per record
 template <int D>
 __global__ __launch_bounds__(256) void k_classify(GridParams g, SpreadParams sp,
                                                   const uint32_t *__restrict__ offsets,
-                                                  uint32_t *__restrict__ totals)
+                                                  uint32_t *__restrict__ totals,
+                                                  uint32_t *__restrict__ ctrl)
 {
+    // the plan that follows counts from zero
+    if (blockIdx.x == 0 && threadIdx.x < 8) ctrl[threadIdx.x] = 0;
     const int lane = threadIdx.x & 63;
     const int64_t b = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
     if (b >= sp.block_count) return;
@@ -52,141 +55,169 @@ __global__ __launch_bounds__(256) void k_classify(GridParams g, SpreadParams sp,
     if (lane == 0) totals[b] = (uint32_t)(total > 0xffffffffull ? 0xffffffffull : total);
 }
 
+// A plan whose split is left to the engine aims at this many waves of work
+// (256 CUs by 4 SIMDs, twice over) while its blocks hold few records: parts
+// of an even share of the records in reach, at least kAutoPart of them (below
+// that a part's fixed cost, its reach rows and its partial sums, outweighs
+// the shorter chain), and blocks of more than two such parts are split.
+// 1e5 points on 256^2 cells (256 tiles of 740 records in reach, one wave
+// each): spread 41 -> 12 us.
+constexpr uint32_t kAutoPart = 128;
+
 // One workgroup plans the work items: a light block is one item, a heavy
 // block as many parts as its records need.  ctrl[0] = items, ctrl[1] = heavy
-// parts, ctrl[2] = heavy blocks, ctrl[3] = records per part.  (One
-// instantiation per kernel: each keeps its LDS variables to itself.)
+// parts, ctrl[2] = heavy blocks, ctrl[3] = records per part.  A thread takes
+// kPlanRun consecutive blocks a round, so a round is one scan over 8192
+// blocks.  (One instantiation per kernel: each keeps its LDS variables to
+// itself.)
+constexpr int kPlanRun = 8;
+
 template <int Kernel>
 __device__ inline void plan_blocks(int64_t nblocks, const uint32_t *__restrict__ totals,
-                                   uint32_t light_limit, uint32_t min_part,
+                                   uint32_t light_limit, uint32_t min_part, bool auto_split,
                                    int64_t part_capacity, uint32_t *__restrict__ parts,
                                    uint32_t *__restrict__ item_off,
                                    uint32_t *__restrict__ heavy_base,
                                    uint32_t *__restrict__ heavy_list,
                                    uint32_t *__restrict__ ctrl)
 {
-    __shared__ uint64_t s_heavy_records;
+    __shared__ unsigned long long s_heavy_records, s_records;
     __shared__ uint32_t s_heavy_blocks;
-    __shared__ uint32_t s_part;
-    __shared__ uint32_t s_wsum[16];
-    __shared__ uint32_t s_carry[2];
+    __shared__ uint32_t s_wsum[2][16];
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
     if (threadIdx.x == 0) {
-        s_heavy_records = 0;
+        s_heavy_records = s_records = 0;
         s_heavy_blocks = 0;
-        s_carry[0] = s_carry[1] = 0;
     }
     __syncthreads();
+    if (auto_split) {
+        unsigned long long mine = 0;
+        for (int64_t b = threadIdx.x; b < nblocks; b += blockDim.x) mine += totals[b];
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) mine += __shfl_xor(mine, o, 64);
+        if (lane == 0) atomicAdd(&s_records, mine);
+        __syncthreads();
+        const unsigned long long share = (s_records + kAutoWaves - 1) / kAutoWaves;
+        const uint32_t part = share > kAutoPart ? (uint32_t)(share < 0x3fffffffull ? share : 0x3fffffffull)
+                                                : kAutoPart;
+        if (2 * part < light_limit) {
+            light_limit = 2 * part;
+            min_part = part < min_part ? part : min_part;
+        }
+    }
     // Raise the light limit until the heavy blocks fill at most half of the
     // partial-sum slots, so every heavy block keeps room for several parts.
-    __shared__ uint32_t s_limit;
-    if (threadIdx.x == 0) s_limit = light_limit;
-    __syncthreads();
     for (;;) {
-        const uint32_t limit = s_limit;
-        uint64_t mine = 0;
+        unsigned long long mine = 0;
         uint32_t mine_blocks = 0;
         for (int64_t b = threadIdx.x; b < nblocks; b += blockDim.x) {
-            uint32_t t = totals[b];
-            if (t > limit) {
+            const uint32_t t = totals[b];
+            if (t > light_limit) {
                 mine += t;
                 ++mine_blocks;
             }
         }
-        atomicAdd((unsigned long long *)&s_heavy_records, (unsigned long long)mine);
-        atomicAdd(&s_heavy_blocks, mine_blocks);
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) {
+            mine += __shfl_xor(mine, o, 64);
+            mine_blocks += __shfl_xor(mine_blocks, o, 64);
+        }
+        if (lane == 0 && mine_blocks) {
+            atomicAdd(&s_heavy_records, mine);
+            atomicAdd(&s_heavy_blocks, mine_blocks);
+        }
         __syncthreads();
-        const bool fits = (int64_t)s_heavy_blocks * 2 <= part_capacity || limit >= 0x7fffffffu;
-        __syncthreads();
+        const bool fits = (int64_t)s_heavy_blocks * 2 <= part_capacity || light_limit >= 0x7fffffffu;
         if (fits) break;
+        light_limit *= 2;
+        __syncthreads();
         if (threadIdx.x == 0) {
-            s_limit = limit * 2;
             s_heavy_records = 0;
             s_heavy_blocks = 0;
         }
         __syncthreads();
     }
-    light_limit = s_limit;
-    if (threadIdx.x == 0) {
-        uint64_t spare = part_capacity > (int64_t)s_heavy_blocks
-                             ? (uint64_t)(part_capacity - s_heavy_blocks)
-                             : 1ull;
-        uint64_t part = (s_heavy_records + spare - 1) / spare;
-        if (part < min_part) part = min_part;
-        s_part = (uint32_t)(part > 0xffffffffull ? 0xffffffffull : part);
+    uint32_t part;
+    {
+        const uint64_t spare = part_capacity > (int64_t)s_heavy_blocks
+                                   ? (uint64_t)(part_capacity - s_heavy_blocks)
+                                   : 1ull;
+        uint64_t len = (s_heavy_records + spare - 1) / spare;
+        if (len < min_part) len = min_part;
+        part = (uint32_t)(len > 0xffffffffull ? 0xffffffffull : len);
     }
-    __syncthreads();
-    uint32_t part = s_part;
-    // Ordered exclusive scans of items and heavy parts, 1024 blocks a round.
-    int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    for (int64_t base = 0; base < nblocks; base += blockDim.x) {
-        int64_t b = base + threadIdx.x;
-        uint32_t np = 0, hp = 0, hb = 0;
-        if (b < nblocks) {
-            uint32_t t = totals[b];
-            np = 1;
-            if (t > light_limit) {
-                np = (uint32_t)((t + (uint64_t)part - 1) / part);
+    // Ordered exclusive scans of items and heavy parts.
+    uint32_t carry_items = 0, carry_parts = 0;
+    for (int64_t base = 0; base < nblocks; base += (int64_t)blockDim.x * kPlanRun) {
+        const int64_t b0 = base + (int64_t)threadIdx.x * kPlanRun;
+        uint32_t np[kPlanRun], items = 0, heavy = 0;
+#pragma unroll
+        for (int j = 0; j < kPlanRun; ++j) {
+            np[j] = 0;
+            if (b0 + j < nblocks) {
+                const uint32_t t = totals[b0 + j];
                 // a block that fits one part is written directly (np == 1
                 // means light to the tile kernels and the reduction)
-                if (np > 1) {
-                    hp = np;
-                    hb = 1;
-                } else {
-                    np = 1;
-                }
+                np[j] = t > light_limit ? (uint32_t)((t + (uint64_t)part - 1) / part) : 1u;
             }
-            parts[b] = np;
+            items += np[j];
+            heavy += np[j] > 1 ? np[j] : 0u;
         }
-        // pack (items, heavy parts) into one 64-bit scan via two passes
-        for (int pass = 0; pass < 2; ++pass) {
-            uint32_t v = pass == 0 ? np : hp;
-            uint32_t x = v;
-            for (int o = 1; o < 64; o <<= 1) {
-                uint32_t y = __shfl_up(x, o, 64);
-                if (lane >= o) x += y;
+        uint32_t xi = items, xh = heavy;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const uint32_t yi = __shfl_up(xi, o, 64), yh = __shfl_up(xh, o, 64);
+            if (lane >= o) {
+                xi += yi;
+                xh += yh;
             }
-            if (lane == 63) s_wsum[wid] = x;
-            __syncthreads();
-            uint32_t pre = 0, all = 0;
-            for (int w = 0; w < (int)(blockDim.x >> 6); ++w) {
-                if (w < wid) pre += s_wsum[w];
-                all += s_wsum[w];
-            }
-            uint32_t ex = s_carry[pass] + pre + x - v;
-            if (b < nblocks) {
-                if (pass == 0)
-                    item_off[b] = ex;
-                else
-                    heavy_base[b] = ex;
-            }
-            __syncthreads();
-            if (threadIdx.x == 0) s_carry[pass] += all;
-            __syncthreads();
         }
-        if (hb) {
-            uint32_t slot = atomicAdd(&ctrl[2], 1u);  // ctrl[2] cleared by the host
-            heavy_list[slot] = (uint32_t)b;
+        __syncthreads();  // the previous round's sums have been read
+        if (lane == 63) {
+            s_wsum[0][wid] = xi;
+            s_wsum[1][wid] = xh;
+        }
+        __syncthreads();
+        uint32_t ei = carry_items + xi - items, eh = carry_parts + xh - heavy;
+        for (int w = 0; w < (int)(blockDim.x >> 6); ++w) {
+            if (w < wid) {
+                ei += s_wsum[0][w];
+                eh += s_wsum[1][w];
+            }
+            carry_items += s_wsum[0][w];
+            carry_parts += s_wsum[1][w];
+        }
+#pragma unroll
+        for (int j = 0; j < kPlanRun; ++j) {
+            if (b0 + j >= nblocks) break;
+            parts[b0 + j] = np[j];
+            item_off[b0 + j] = ei;
+            heavy_base[b0 + j] = eh;
+            ei += np[j];
+            if (np[j] > 1) {
+                eh += np[j];
+                heavy_list[atomicAdd(&ctrl[2], 1u)] = (uint32_t)(b0 + j);  // ctrl[2] cleared before
+            }
         }
     }
-    __syncthreads();
     if (threadIdx.x == 0) {
-        ctrl[0] = s_carry[0];
-        ctrl[1] = s_carry[1];
+        ctrl[0] = carry_items;
+        ctrl[1] = carry_parts;
         ctrl[3] = part;
     }
 }
 
 __global__ __launch_bounds__(1024) void k_plan(int64_t nblocks, const uint32_t *__restrict__ totals,
                                                uint32_t light_limit, uint32_t min_part,
-                                               int64_t part_capacity,
+                                               bool auto_split, int64_t part_capacity,
                                                uint32_t *__restrict__ parts,
                                                uint32_t *__restrict__ item_off,
                                                uint32_t *__restrict__ heavy_base,
                                                uint32_t *__restrict__ heavy_list,
                                                uint32_t *__restrict__ ctrl)
 {
-    plan_blocks<0>(nblocks, totals, light_limit, min_part, part_capacity, parts, item_off,
-                   heavy_base, heavy_list, ctrl);
+    plan_blocks<0>(nblocks, totals, light_limit, min_part, auto_split, part_capacity, parts,
+                   item_off, heavy_base, heavy_list, ctrl);
 }
 
 // Many problems: workgroup q plans problem q's blocks alone, with its own
@@ -202,8 +233,8 @@ __global__ __launch_bounds__(1024) void k_plan_many(const SpreadProblem *__restr
 {
     const SpreadProblem &q = sprobs[blockIdx.x];
     const int64_t bb = q.block_base;
-    plan_blocks<1>(q.sp.block_count, totals + bb, q.light_limit, q.min_part, q.part_capacity,
-                   parts + bb, item_off + bb, heavy_base + bb, heavy_list + bb,
+    plan_blocks<1>(q.sp.block_count, totals + bb, q.light_limit, q.min_part, q.auto_split,
+                   q.part_capacity, parts + bb, item_off + bb, heavy_base + bb, heavy_list + bb,
                    ctrl + 8 * (int64_t)blockIdx.x);
 }
 
@@ -442,6 +473,167 @@ __device__ __forceinline__ void spread_block(SpreadShared<D, T, R> &sh, const Gr
     __syncthreads();
 }
 
+// 1D: a record reaches w of the block's 64 R cells, so every lane walks only
+// the records that can reach its own cells: their slots follow from the bin
+// offsets (no search, no record that misses), and a record's weights are
+// staged once, by the lane that holds it, from the panel polynomials.  Bound
+// by the latency of the staged reads; the loop over every staged record
+// before it took 222 us for 3e5 FP64 points on 1e5 cells at width 10, with
+// 4 of 64 lanes adding at a time.
+template <typename T, int R>
+struct Staged1 {
+    T kx[2 * R + kKw];  // weights, R - 1 zeros before and R after the support
+    T cre, cim;
+    int s;
+};
+
+template <typename T, int R>
+struct Spread1Shared {
+    Staged1<T, R> st[kLanes];
+};
+
+// The weights of a support of w cells (w known at run time), as
+// es_axis_weights.
+template <typename T, typename Put>
+__device__ inline void es_axis_weights_any(int w, T off, T beta, UniformPtr<T> c, Put put)
+{
+    constexpr int NE = sizeof(T) == 4 ? kPanelEven32 : kPanelEven64;
+    constexpr int NO = sizeof(T) == 4 ? kPanelOdd32 : kPanelOdd64;
+    put(0, es_weight<T>(off, w, beta));
+    put(w - 1, es_weight<T>(off + (T)(w - 1), w, beta));
+    const T x = off + (T)0.5 * (T)(w - 1);
+    const T x2 = x * x;
+    for (int t = 1; t <= (w - 1) / 2; ++t) {
+        UniformPtr<T> e = c + (t - 1) * (NE + NO), o = e + NE;
+        T even = e[NE - 1], odd = o[NO - 1];
+#pragma unroll
+        for (int i = NE - 2; i >= 0; --i) even = __builtin_elementwise_fma(even, x2, e[i]);
+#pragma unroll
+        for (int i = NO - 2; i >= 0; --i) odd = __builtin_elementwise_fma(odd, x2, o[i]);
+        put(w - 1 - t, __builtin_elementwise_fma(-x, odd, even));
+        put(t, __builtin_elementwise_fma(x, odd, even));
+    }
+}
+
+// spread_block for one dimension.
+template <typename T, int R>
+__device__ __forceinline__ void spread_block(Spread1Shared<T, R> &sh, const GridParams &g,
+                                             const SpreadParams &sp, int64_t b, int64_t rlo,
+                                             int64_t rhi, uint32_t np,
+                                             const uint32_t *__restrict__ offsets,
+                                             const int4 *__restrict__ rec_start,
+                                             const T *__restrict__ rec_off,
+                                             const T *__restrict__ cv, T *__restrict__ grid_v,
+                                             T *__restrict__ part_v)
+{
+    Staged1<T, R> *st = sh.st;
+    const int lane = threadIdx.x;
+    const int w = g.width;
+    const T beta = (T)g.beta;
+    const UniformPtr<T> panels = panel_coefficients<T>(g);
+    const int64_t n = g.ax[0].n;
+    const int64_t b0 = b * sp.block[0], x0 = b0 + (int64_t)lane * R;
+    // the block's records: slots [f0, f0 + n0), then [f1, ...) past a wrap
+    const AxisReach br = axis_reach(b0, sp.block[0], w, g.ax[0]);
+    const int64_t f0 = offsets[br.lo0], n0 = (int64_t)offsets[br.lo0 + br.len0] - f0;
+    const int64_t f1 = br.len1 > 0 ? (int64_t)offsets[br.lo1] : 0;
+    // the lane's records, as ranges of the block's
+    int64_t ka[2] = {0, 0}, ke[2] = {0, 0};
+    if (x0 < n) {
+        const AxisReach lr = axis_reach(x0, R, w, g.ax[0]);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int64_t lo = i ? lr.lo1 : lr.lo0, len = i ? lr.len1 : lr.len0;
+            if (len > 0) {
+                const int64_t a = offsets[lo], e = offsets[lo + len];
+                const int64_t at = lo >= br.lo0 && lo < br.lo0 + br.len0 ? -f0 : n0 - f1;
+                ka[i] = a + at;
+                ke[i] = e + at;
+            }
+        }
+    }
+    T acc_re[R], acc_im[R];
+#pragma unroll
+    for (int i = 0; i < R; ++i) acc_re[i] = acc_im[i] = (T)0;
+    // the zeros around the weights
+#pragma unroll
+    for (int j = 0; j < 2 * R + kKw; ++j) st[lane].kx[j] = (T)0;
+    for (int64_t k0 = rlo; k0 < rhi; k0 += kLanes) {
+        const int m = (int)(rhi - k0 < kLanes ? rhi - k0 : kLanes);
+        if (lane < m) {
+            const int64_t k = k0 + lane;
+            const int64_t slot = k < n0 ? f0 + k : f1 + (k - n0);
+            Staged1<T, R> &S = st[lane];
+            S.s = rec_start[slot].x;
+            S.cre = cv[2 * slot];
+            S.cim = cv[2 * slot + 1];
+            es_axis_weights_any<T>(w, rec_off[4 * slot], beta, panels,
+                                   [&](int t, T v) { S.kx[R - 1 + t] = v; });
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int lo = (int)(ka[i] > k0 ? ka[i] - k0 : 0);
+            const int hi = (int)(ke[i] - k0 < m ? ke[i] - k0 : m);
+#pragma unroll 2
+            for (int q = lo; q < hi; ++q) {
+                const Staged1<T, R> &S = st[q];
+                int64_t e = x0 - S.s;
+                if (e < 0) e += n;
+                if (e > n - R) e -= n;
+                if (e < w) {
+                    const T *kx = S.kx + (int)e + R - 1;
+#pragma unroll
+                    for (int j = 0; j < R; ++j) {
+                        acc_re[j] += kx[j] * S.cre;
+                        acc_im[j] += kx[j] * S.cim;
+                    }
+                }
+            }
+        }
+        __syncthreads();
+    }
+    if (np == 1) {
+#pragma unroll
+        for (int i = 0; i < R; ++i) {
+            if (x0 + i < n) {
+                grid_v[2 * (x0 + i)] = acc_re[i];
+                grid_v[2 * (x0 + i) + 1] = acc_im[i];
+            }
+        }
+    } else {
+        T *out = part_v + 2 * ((int64_t)lane * R);
+#pragma unroll
+        for (int i = 0; i < R; ++i) {
+            out[2 * i] = acc_re[i];
+            out[2 * i + 1] = acc_im[i];
+        }
+    }
+    __syncthreads();
+}
+
+// LDS and body of a rank's blocks.
+template <int D, typename T, int R>
+struct BlockSpread {
+    using Shared = SpreadShared<D, T, R>;
+    template <typename... A>
+    __device__ static __forceinline__ void run(Shared &sh, const GridParams &g,
+                                               const SpreadParams &sp, A... a)
+    {
+        spread_block<D, T, R>(sh, g, sp, a...);
+    }
+};
+template <typename T, int R>
+struct BlockSpread<1, T, R> {
+    using Shared = Spread1Shared<T, R>;
+    template <typename... A>
+    __device__ static __forceinline__ void run(Shared &sh, const GridParams &g,
+                                               const SpreadParams &sp, A... a)
+    {
+        spread_block<T, R>(sh, g, sp, a...);
+    }
+};
+
 // Record range of work item `item` of the plan: block b, part p of np.
 __device__ inline void item_records(int64_t item, int64_t nblocks,
                                     const uint32_t *__restrict__ item_off,
@@ -489,7 +681,7 @@ __global__ __launch_bounds__(kLanes) void k_spread(GridParams g, SpreadParams sp
                                                    T *__restrict__ grid, T *__restrict__ partial,
                                                    int64_t block_cells)
 {
-    __shared__ SpreadShared<D, T, R> sh;
+    __shared__ typename BlockSpread<D, T, R>::Shared sh;
     const int64_t v = blockIdx.y;
     const int64_t n_items = ctrl[0];
     const uint32_t part_len_cap = ctrl[3];
@@ -500,9 +692,9 @@ __global__ __launch_bounds__(kLanes) void k_spread(GridParams g, SpreadParams sp
         item_records(item, sp.block_count, item_off, parts, totals, part_len_cap, &b, &p, &np,
                      &rlo, &rhi);
         const int64_t slot = (int64_t)heavy_base[b] + p;
-        spread_block<D, T, R>(sh, g, sp, b, rlo, rhi, np, offsets, rec_start, rec_off, cv,
-                              grid + 2 * v * g.fine_total,
-                              partial + 2 * (slot * gridDim.y + v) * block_cells);
+        BlockSpread<D, T, R>::run(sh, g, sp, b, rlo, rhi, np, offsets, rec_start, rec_off, cv,
+                                  grid + 2 * v * g.fine_total,
+                                  partial + 2 * (slot * gridDim.y + v) * block_cells);
     }
 }
 
@@ -682,7 +874,7 @@ __global__ __launch_bounds__(kLanes) void k_spread_many(
     const uint32_t *__restrict__ pctrl, const int64_t *__restrict__ pbase,
     T *__restrict__ partial, int64_t block_cells)
 {
-    __shared__ SpreadShared<D, T, R> sh;
+    __shared__ typename BlockSpread<D, T, R>::Shared sh;
     const int64_t n_items = pbase[4 * nprob];
     for (int64_t item = blockIdx.x; item < n_items; item += gridDim.x) {
         const int q = batch_problem_of(pbase, nprob, 0, item);
@@ -694,8 +886,9 @@ __global__ __launch_bounds__(kLanes) void k_spread_many(
         item_records(item - pbase[4 * q], spb.sp.block_count, item_off + bb, parts + bb,
                      totals + bb, pctrl[8 * q + 3], &b, &p, &np, &rlo, &rhi);
         const int64_t slot = pbase[4 * q + 1] + (int64_t)heavy_base[bb + b] + p;
-        spread_block<D, T, R>(sh, pb.g, spb.sp, b, rlo, rhi, np, offsets + pb.bin_base, rec_start,
-                              rec_off, c_sorted, (T *)pb.grid, partial + 2 * slot * block_cells);
+        BlockSpread<D, T, R>::run(sh, pb.g, spb.sp, b, rlo, rhi, np, offsets + pb.bin_base,
+                                  rec_start, rec_off, c_sorted, (T *)pb.grid,
+                                  partial + 2 * slot * block_cells);
     }
 }
 
@@ -837,11 +1030,6 @@ __global__ __launch_bounds__(256) void k_reduce_tiles(GridParams g, SpreadParams
 }
 
 inline unsigned grid_for(int64_t n, int threads) { return (unsigned)((n + threads - 1) / threads); }
-
-__global__ void k_fill_ctrl(uint32_t *ctrl)
-{
-    if (threadIdx.x < 8) ctrl[threadIdx.x] = 0;
-}
 
 // Tile kernels and heavy-part reductions for one chunk of vectors (gridDim.y
 // = chunk; c_sorted and grid point at the chunk's first vector).  The work
@@ -1024,18 +1212,20 @@ bool Spreader::spread(const GridParams &g, const SpreadParams &sp, const uint32_
     const int64_t nb = sp.block_count;
     const bool reuse = reuse_plan && planned_epoch == blocks_epoch && planned_blocks == nb &&
                        planned_capacity == part_capacity && planned_light == light_limit &&
-                       planned_min == min_part && planned_offsets == offsets;
+                       planned_min == min_part && planned_auto == auto_split &&
+                       planned_offsets == offsets;
     reuse_plan = false;
     if (!reuse) {
-        k_classify<D><<<grid_for(nb * 64, 256), 256, 0, stream>>>(g, sp, offsets, totals);
-        k_fill_ctrl<<<1, 64, 0, stream>>>(ctrl);
-        k_plan<<<1, 1024, 0, stream>>>(nb, totals, light_limit, min_part, part_capacity, parts,
-                                       item_off, heavy_base, heavy_list, ctrl);
+        k_classify<D><<<grid_for(nb * 64, 256), 256, 0, stream>>>(g, sp, offsets, totals, ctrl);
+        k_plan<<<1, 1024, 0, stream>>>(nb, totals, light_limit, min_part, auto_split,
+                                       part_capacity, parts, item_off, heavy_base, heavy_list,
+                                       ctrl);
         planned_epoch = blocks_epoch;
         planned_blocks = nb;
         planned_capacity = part_capacity;
         planned_light = light_limit;
         planned_min = min_part;
+        planned_auto = auto_split;
         planned_offsets = offsets;
     }
     if constexpr (sizeof(T) == 4) {

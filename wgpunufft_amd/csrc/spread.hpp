@@ -61,7 +61,12 @@ struct SpreadProblem {
     int64_t block_base;
     int64_t part_capacity;
     uint32_t light_limit, min_part;
+    uint32_t auto_split;
 };
+
+// Waves of work that a plan with few records in reach is split for (plan_blocks
+// in spread.hip): its heavy parts are then at most this many and one a block.
+constexpr uint32_t kAutoWaves = 2048;
 
 // A class of consecutive problems [p0, p1) of one run length (or of the row
 // tiles and one kernel width): its blocks
@@ -115,6 +120,7 @@ struct Spreader {
     uint64_t blocks_epoch = 0, planned_epoch = ~0ull;
     int64_t planned_blocks = -1, planned_capacity = -1;
     uint32_t planned_light = 0, planned_min = 0;
+    bool planned_auto = false;
     const uint32_t *planned_offsets = nullptr;
 
     uint32_t *totals = nullptr;      // records in reach per block
@@ -133,9 +139,12 @@ struct Spreader {
     int64_t vmax_cap = 0;
     int64_t part_capacity = 0;
     // Records in reach above which a block is split into parts, and the
-    // smallest part.
+    // smallest part; with auto_split both are lowered for point sets that
+    // would leave the chip idle (never by a caller's or the autotuner's own
+    // values).
     uint32_t light_limit = 4096;
     uint32_t min_part = 1024;
+    bool auto_split = true;
     // Partial-sum slots of one vector, and the scratch a chunk of vectors
     // may take (the chunk is at least one vector).
     int64_t budget_bytes = (int64_t)256 << 20;
