@@ -14,7 +14,9 @@
 // which leaves the transform in natural order after the last pass.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
+#include <cstring>
 #include <mutex>
 #include <vector>
 
@@ -37,12 +39,14 @@ template <>
 struct LdsElems<float> {
     static constexpr int value = 9728;  // 80 KB less the per-line arrays
     static constexpr int base = 7680;   // 64 KB less the per-line arrays
+    static constexpr int group = 18 * kThreads;  // elements of a workgroup's lines
     static constexpr int columns = 16;
 };
 template <>
 struct LdsElems<double> {
     static constexpr int value = 4864;
     static constexpr int base = 3840;
+    static constexpr int group = 9 * kThreads;
     static constexpr int columns = 8;
 };
 // static LDS: line bases, mode rows and two factors per line
@@ -91,19 +95,20 @@ __device__ inline void divmod_small(int a, int b, float inv_b, int &q, int &r)
     }
 }
 
-// Small DFTs, X_s = sum_t u_t exp(DIR 2 pi i s t / R).
-template <typename T, int DIR>
-__device__ inline void dft2(Cx<T> *u)
+// Small DFTs, X_s = sum_t u_t exp(2 pi i s t / R).  The other sign is the same
+// transform with real and imaginary parts exchanged on the way in and out.
+template <typename T>
+__device__ __forceinline__ void dft2(Cx<T> *u)
 {
     const Cx<T> a = u[0], b = u[1];
     u[0] = cadd(a, b);
     u[1] = csub(a, b);
 }
 
-template <typename T, int DIR>
-__device__ inline void dft3(Cx<T> *u)
+template <typename T>
+__device__ __forceinline__ void dft3(Cx<T> *u)
 {
-    const T s = (T)DIR * (T)0.86602540378443864676;  // sin(2 pi / 3)
+    const T s = (T)0.86602540378443864676;  // sin(2 pi / 3)
     const Cx<T> t1 = cadd(u[1], u[2]);
     const Cx<T> d = irot(csub(u[1], u[2]), s);
     const Cx<T> m = Cx<T>{u[0].re - (T)0.5 * t1.re, u[0].im - (T)0.5 * t1.im};
@@ -112,25 +117,25 @@ __device__ inline void dft3(Cx<T> *u)
     u[2] = csub(m, d);
 }
 
-template <typename T, int DIR>
-__device__ inline void dft4(Cx<T> *u)
+template <typename T>
+__device__ __forceinline__ void dft4(Cx<T> *u)
 {
     const Cx<T> a = cadd(u[0], u[2]), b = csub(u[0], u[2]);
     const Cx<T> c = cadd(u[1], u[3]);
-    const Cx<T> d = irot(csub(u[1], u[3]), (T)DIR);
+    const Cx<T> d = irot(csub(u[1], u[3]), (T)1);
     u[0] = cadd(a, c);
     u[2] = csub(a, c);
     u[1] = cadd(b, d);
     u[3] = csub(b, d);
 }
 
-template <typename T, int DIR>
-__device__ inline void dft5(Cx<T> *u)
+template <typename T>
+__device__ __forceinline__ void dft5(Cx<T> *u)
 {
     const T c1 = (T)0.30901699437494742410;           // cos(2 pi / 5)
     const T c2 = (T)-0.80901699437494742410;          // cos(4 pi / 5)
-    const T s1 = (T)DIR * (T)0.95105651629515357212;  // sin(2 pi / 5)
-    const T s2 = (T)DIR * (T)0.58778525229247312917;  // sin(4 pi / 5)
+    const T s1 = (T)0.95105651629515357212;  // sin(2 pi / 5)
+    const T s2 = (T)0.58778525229247312917;  // sin(4 pi / 5)
     const Cx<T> a1 = cadd(u[1], u[4]), b1 = csub(u[1], u[4]);
     const Cx<T> a2 = cadd(u[2], u[3]), b2 = csub(u[2], u[3]);
     const Cx<T> u0 = u[0];
@@ -146,16 +151,16 @@ __device__ inline void dft5(Cx<T> *u)
     u[3] = csub(m2, e2);
 }
 
-// Even and odd halves as two DFT4s, the odd half turned by w^s, w = exp(DIR 2 pi i / 8).
-template <typename T, int DIR>
-__device__ inline void dft8(Cx<T> *u)
+// Even and odd halves as two DFT4s, the odd half turned by w^s, w = exp(2 pi i / 8).
+template <typename T>
+__device__ __forceinline__ void dft8(Cx<T> *u)
 {
     const T h = (T)0.70710678118654752440;  // cos(pi / 4)
-    const T d = (T)DIR;
+    const T d = (T)1;
     Cx<T> e[4] = {u[0], u[2], u[4], u[6]};
     Cx<T> o[4] = {u[1], u[3], u[5], u[7]};
-    dft4<T, DIR>(e);
-    dft4<T, DIR>(o);
+    dft4<T>(e);
+    dft4<T>(o);
     const Cx<T> o1 = Cx<T>{h * (o[1].re - d * o[1].im), h * (o[1].im + d * o[1].re)};
     const Cx<T> o2 = irot(o[2], d);
     const Cx<T> o3 = Cx<T>{h * (-o[3].re - d * o[3].im), h * (-o[3].im + d * o[3].re)};
@@ -190,10 +195,10 @@ __host__ __device__ constexpr double prime_sin(int R, int k)
 }
 
 // Odd prime R from the pairs t, R - t:
-//   X_s = u_0 + sum_t (u_t + u_{R-t}) cos(2 pi s t / R) + i DIR (u_t - u_{R-t}) sin(2 pi s t / R),
+//   X_s = u_0 + sum_t (u_t + u_{R-t}) cos(2 pi s t / R) + i (u_t - u_{R-t}) sin(2 pi s t / R),
 // t = 1 .. (R - 1) / 2, and X_{R-s} with the sine terms negated.
-template <typename T, int DIR, int R>
-__device__ inline void dft_prime(Cx<T> *u)
+template <typename T, int R>
+__device__ __forceinline__ void dft_prime(Cx<T> *u)
 {
     constexpr int H = (R - 1) / 2;
     Cx<T> a[H], b[H];
@@ -217,7 +222,7 @@ __device__ inline void dft_prime(Cx<T> *u)
             m = Cx<T>{m.re + c * a[t - 1].re, m.im + c * a[t - 1].im};
             e = Cx<T>{e.re + sn * b[t - 1].re, e.im + sn * b[t - 1].im};
         }
-        const Cx<T> ie = Cx<T>{-(T)DIR * e.im, (T)DIR * e.re};
+        const Cx<T> ie = Cx<T>{-e.im, e.re};
         out[s] = cadd(m, ie);
         out[R - s] = csub(m, ie);
     }
@@ -225,24 +230,110 @@ __device__ inline void dft_prime(Cx<T> *u)
     for (int t = 0; t < R; ++t) u[t] = out[t];
 }
 
-template <typename T, int DIR, int R>
-__device__ inline void dft(Cx<T> *u)
+// cos(2 pi k / n) and sin(2 pi k / n) at compile time: the angle folded to
+// the first octant on the integers, then the Taylor series.
+constexpr double octant_series(double x, bool sine)
 {
-    if constexpr (R == 7 || R == 11 || R == 13) dft_prime<T, DIR, R>(u);
-    if constexpr (R == 2) dft2<T, DIR>(u);
-    if constexpr (R == 3) dft3<T, DIR>(u);
-    if constexpr (R == 4) dft4<T, DIR>(u);
-    if constexpr (R == 5) dft5<T, DIR>(u);
-    if constexpr (R == 8) dft8<T, DIR>(u);
+    double term = sine ? x : 1.0, sum = term;
+    for (int i = sine ? 2 : 1; i < 28; i += 2) {
+        term *= -x * x / (i * (i + 1.0));
+        sum += term;
+    }
+    return sum;
+}
+constexpr double unit_cos(int k, int n)
+{
+    k = ((k % n) + n) % n;
+    if (2 * k > n) k = n - k;                      // cos(-x) = cos x
+    if (4 * k > n) return -unit_cos(n - 2 * k, 2 * n);  // cos(pi - x) = -cos x
+    constexpr double tau = 6.28318530717958647692;
+    return 8 * k <= n ? octant_series(tau * k / n, false)
+                      : octant_series(tau * (n - 4.0 * k) / (4.0 * n), true);
+}
+template <int R>
+struct UnitRoots {
+    double c[R], s[R];
+    constexpr UnitRoots() : c(), s()
+    {
+        for (int k = 0; k < R; ++k) {
+            c[k] = unit_cos(k, R);
+            s[k] = unit_cos(4 * k - R, 4 * R);  // sin x = cos(x - pi / 2)
+        }
+    }
+};
+
+template <typename T, int R>
+__device__ __forceinline__ void dft(Cx<T> *u);
+
+// R = A B with A and B coprime (prime-factor mapping, no twiddles): element
+// (B a + A b) mod R, frequency k from (k mod A, k mod B).
+template <typename T, int A, int B>
+__device__ __forceinline__ void dft_coprime(Cx<T> *u)
+{
+    constexpr int R = A * B;
+    Cx<T> y[B][A];
+#pragma unroll
+    for (int b = 0; b < B; ++b) {
+#pragma unroll
+        for (int a = 0; a < A; ++a) y[b][a] = u[(B * a + A * b) % R];
+        dft<T, A>(y[b]);
+    }
+#pragma unroll
+    for (int a = 0; a < A; ++a) {
+        Cx<T> v[B];
+#pragma unroll
+        for (int b = 0; b < B; ++b) v[b] = y[b][a];
+        dft<T, B>(v);
+#pragma unroll
+        for (int k = 0; k < R; ++k)
+            if (k % A == a) u[k] = v[k % B];
+    }
 }
 
-// One Stockham pass over the workgroup's lines.  kFromGrid: the pass reads
-// its butterflies' inputs from the grid (the first pass: p = 1, no
-// twiddles; cells outside the read window are zeros); kToGrid: it writes its
-// outputs to the grid (the last pass: p R = n; cells outside the write
-// window are dropped).  Otherwise LDS in place: every thread reads its
-// butterflies into registers, the workgroup waits, every thread writes.
-constexpr int kFromGrid = 1, kToGrid = 2;
+// R = Q Q: elements Q a + b, DFT_Q over a, twiddles w_R^{b k}, DFT_Q over b.
+template <typename T, int Q>
+__device__ __forceinline__ void dft_square(Cx<T> *u)
+{
+    constexpr int R = Q * Q;
+    constexpr UnitRoots<R> w;
+    Cx<T> y[Q][Q];
+#pragma unroll
+    for (int b = 0; b < Q; ++b) {
+#pragma unroll
+        for (int a = 0; a < Q; ++a) y[b][a] = u[Q * a + b];
+        dft<T, Q>(y[b]);
+#pragma unroll
+        for (int k = 1; k < Q; ++k)
+            if (b > 0)
+                y[b][k] = cmul(y[b][k], Cx<T>{(T)w.c[b * k], (T)w.s[b * k]});
+    }
+#pragma unroll
+    for (int k = 0; k < Q; ++k) {
+        Cx<T> v[Q];
+#pragma unroll
+        for (int b = 0; b < Q; ++b) v[b] = y[b][k];
+        dft<T, Q>(v);
+#pragma unroll
+        for (int m = 0; m < Q; ++m) u[k + Q * m] = v[m];
+    }
+}
+
+template <typename T, int R>
+__device__ __forceinline__ void dft(Cx<T> *u)
+{
+    if constexpr (R == 7 || R == 11 || R == 13) dft_prime<T, R>(u);
+    if constexpr (R == 2) dft2<T>(u);
+    if constexpr (R == 3) dft3<T>(u);
+    if constexpr (R == 4) dft4<T>(u);
+    if constexpr (R == 5) dft5<T>(u);
+    if constexpr (R == 6) dft_coprime<T, 2, 3>(u);
+    if constexpr (R == 8) dft8<T>(u);
+    if constexpr (R == 9) dft_square<T, 3>(u);
+    if constexpr (R == 10) dft_coprime<T, 2, 5>(u);
+    if constexpr (R == 12) dft_coprime<T, 4, 3>(u);
+    if constexpr (R == 15) dft_coprime<T, 3, 5>(u);
+    if constexpr (R == 16) dft_square<T, 4>(u);
+}
 
 // Per-line data of a workgroup in LDS: grid base, mode row and the line's
 // deconvolution factors (type 2: the u and v axes' 1/phi_hat; type 1: their
@@ -259,157 +350,238 @@ __device__ inline int64_t mode_slot(int64_t m, int64_t N, int centered)
     return centered ? m + N / 2 : (m >= 0 ? m : m + N);
 }
 
+// A butterfly of the first pass reads, and one of the last pass writes, the
+// elements e = i + t nb, t = 0 .. R - 1.  visit(t, kept): whether the lane's
+// element lies in the kept window [0, hi) and [n - lo, n) (for most t the
+// same for every lane: scalar branches on the masks).
+template <int R, typename Visit>
+__device__ __forceinline__ void for_kept(const LineFftKept &m, int i, int nb, int n, int hi, int lo,
+                                         Visit visit)
+{
+#pragma unroll
+    for (int t = 0; t < R; ++t) {
+        if ((m.all >> t) & 1u) {
+            visit(t, true);
+        } else if ((m.some >> t) & 1u) {
+            const int e = i + t * nb;
+            visit(t, e < hi || e >= n - lo);
+        } else {
+            visit(t, false);
+        }
+    }
+}
+
 // IO (the launch's mode reads or writes): 0 grid only; 1 the first pass
 // reads the modes and predeconvolves them (type 2); 2 the last pass writes
 // the deconvolved modes (type 1).
-template <typename T, int DIR, int R, int LDS, int MODE, int IO>
-__device__ inline void line_pass(Cx<T> *X, const Cx<T> *tw, const LineFftAxis &P,
-                                 const LineFftPass &ps, Cx<T> *__restrict__ grid,
-                                 const LineData &ld)
+//
+// What bounds the passes: HBM for FP32 (512^3, 4 vectors: x 1.55 ms, y 0.75
+// ms, 4.1 and 4.3 TB/s where a copy reaches 4.6), HBM latency on the short
+// rows of long FP64 axes (900^3: x 1.6, y 2.3, z 6.4 ms, 2.7 to 3.7 TB/s).
+// The vector ALU bounded them before (x 2.1, y 1.0 ms; 900^3 1.8, 2.7, 7.1
+// ms): an address product, a window test and index divisions for every
+// element, divisions of the pass constants in every thread and five small
+// radices at 900 took 124 (FP32) and 156 (FP64) instructions an element; now
+// one 64-bit pointer a butterfly stepped by a uniform stride, windows as
+// masks over t, constants from the host and the largest radices: 56 and 77.
+// One butterfly index of the workgroup: line c, butterfly i of the line.
+template <typename T>
+__device__ inline void butterfly(const LineFftAxis &P, const LineFftPass &ps, int b, int *c, int *i)
 {
-    const int64_t *base = ld.base;
-    Cx<T> *modes = (Cx<T> *)ld.modes;
-    constexpr int MAXB = (LDS / R + kThreads - 1) / kThreads;
-    const int n = P.n, nb = n / R, total = P.lines * nb;
+    if (P.line_major) {
+        divmod_small(b, ps.nb, ps.inv_nb, *c, *i);
+    } else {
+        *i = b >> P.log_lines;
+        *c = b & (P.lines - 1);
+    }
+}
+
+template <typename T, int R>
+__device__ __forceinline__ void exchange(Cx<T> (&u)[R])
+{
+#pragma unroll
+    for (int t = 0; t < R; ++t) u[t] = Cx<T>{u[t].im, u[t].re};
+}
+
+// u_t times w^(t k), the pass's twiddles.
+template <typename T, int R>
+__device__ __forceinline__ void turn(Cx<T> (&u)[R], const Cx<T> *tw, int wstep)
+{
+#pragma unroll
+    for (int t = 1; t < R; ++t) {
+        tw += wstep;
+        u[t] = cmul(u[t], *tw);
+    }
+}
+
+// The first pass (p = 1, no twiddles): butterflies from the grid or the
+// modes into LDS.
+template <typename T, int R, int IO>
+__device__ __forceinline__ void pass_in(Cx<T> *X, const LineFftAxis &P, const LineFftPass &ps,
+                                        const Cx<T> *__restrict__ grid, const LineData &ld)
+{
+    const int n = P.n, nb = ps.nb, total = P.lines * nb;
     const int ks = P.line_major ? 1 : P.lines, cs = P.line_major ? n : 1;
-    const float inv_nb = 1.0f / (float)nb, inv_p = 1.0f / (float)ps.p;
+    const int64_t tstep = (int64_t)nb * P.estride;  // elements between a butterfly's
+    // mode slot of element e: e + half at the window's low end, e + back at
+    // its high end
+    const int half = P.centered ? (int)(P.eN / 2) : 0;
+    const int back = P.centered ? half - n : (int)P.eN - n;
+    for (int b = (int)threadIdx.x; b < total; b += kThreads) {
+        int c, i;
+        butterfly<T>(P, ps, b, &c, &i);
+        Cx<T> u[R];
+        const int64_t bc = ld.base[c];
+        if (bc < 0) {
+#pragma unroll
+            for (int t = 0; t < R; ++t) u[t] = Cx<T>{(T)0, (T)0};
+        } else if constexpr (IO == 1) {
+            // the predeconvolution: mode times (1/phi_hat) in axis order
+            const Cx<T> *row = (const Cx<T> *)ld.modes + ld.mrow[c];
+            const double g1 = ld.f1[c], g2 = ld.f2[c];
+            const double *phi = P.inv_phihat + P.eph;
+            for_kept<R>(P.in, i, nb, n, P.in_hi, P.in_lo, [&](int t, bool in) {
+                u[t] = Cx<T>{(T)0, (T)0};
+                if (in) {
+                    const int e = i + t * nb;
+                    const bool low = e < P.in_hi;
+                    double amp = 1.0;
+                    amp *= phi[low ? e : n - e];
+                    amp *= g1;
+                    amp *= g2;
+                    const Cx<T> src = row[(int64_t)(e + (low ? half : back)) * P.ems];
+                    const T ta = (T)amp;
+                    u[t] = Cx<T>{src.re * ta, src.im * ta};
+                }
+            });
+        } else {
+            const Cx<T> *src = grid + bc + (int64_t)i * P.estride;
+            for_kept<R>(P.in, i, nb, n, P.in_hi, P.in_lo, [&](int t, bool in) {
+                u[t] = Cx<T>{(T)0, (T)0};
+                if (in) u[t] = src[t * tstep];
+            });
+        }
+        if (P.exchange) exchange<T, R>(u);
+        dft<T, R>(u);
+        Cx<T> *out = X + i * R * ks + c * cs;
+#pragma unroll
+        for (int t = 0; t < R; ++t) out[t * ks] = u[t];
+    }
+    __syncthreads();
+}
+
+// A middle pass, in place in LDS: every thread reads its butterflies into
+// registers, the workgroup waits, every thread writes them.
+template <typename T, int R>
+__device__ __forceinline__ void pass_mid(Cx<T> *X, const Cx<T> *tw, const LineFftAxis &P,
+                                         const LineFftPass &ps)
+{
+    constexpr int MAXB = (LdsElems<T>::group / R + kThreads - 1) / kThreads;
+    const int n = P.n, nb = ps.nb, total = P.lines * nb;
+    const int ks = P.line_major ? 1 : P.lines, cs = P.line_major ? n : 1;
+    const int in_step = nb * ks, out_step = ps.p * ks;
     Cx<T> u[MAXB][R];
-    int dst[MAXB], line[MAXB];
+    int at[MAXB];
 #pragma unroll
     for (int s = 0; s < MAXB; ++s) {
         const int b = (int)threadIdx.x + s * kThreads;
-        dst[s] = -1;
+        at[s] = -1;
         if (b < total) {
-            int c, i;
-            if (P.line_major) {
-                divmod_small(b, nb, inv_nb, c, i);
-            } else {
-                i = b >> P.log_lines;
-                c = b & (P.lines - 1);
-            }
-            int q, k;
-            divmod_small(i, ps.p, inv_p, q, k);
-            line[s] = c;
-            if constexpr ((MODE & kFromGrid) != 0) {
-                const int64_t bc = base[c];
-                if constexpr (IO == 1) {
-                    // the predeconvolution: mode times (1/phi_hat) in axis order
-                    const int64_t mr = ld.mrow[c];
-                    const double g1 = ld.f1[c], g2 = ld.f2[c];
+            int c, i, q, k;
+            butterfly<T>(P, ps, b, &c, &i);
+            divmod_small(i, ps.p, ps.inv_p, q, k);
+            const Cx<T> *src = X + i * ks + c * cs;
 #pragma unroll
-                    for (int t = 0; t < R; ++t) {
-                        const int e = i + t * nb;
-                        u[s][t] = Cx<T>{(T)0, (T)0};
-                        if (bc >= 0 && (e < P.in_hi || e >= n - P.in_lo)) {
-                            const int64_t m = e < P.in_hi ? e : (int64_t)e - n;
-                            double amp = 1.0;
-                            amp *= P.inv_phihat[P.eph + (m < 0 ? -m : m)];
-                            amp *= g1;
-                            amp *= g2;
-                            const Cx<T> src = modes[mr + mode_slot(m, P.eN, P.centered) * P.ems];
-                            const T ta = (T)amp;
-                            u[s][t] = Cx<T>{src.re * ta, src.im * ta};
-                        }
-                    }
-                } else {
-#pragma unroll
-                    for (int t = 0; t < R; ++t) {
-                        const int e = i + t * nb;
-                        u[s][t] = Cx<T>{(T)0, (T)0};
-                        if (bc >= 0 && (e < P.in_hi || e >= n - P.in_lo))
-                            u[s][t] = grid[bc + (int64_t)e * P.estride];
-                    }
-                }
-            } else {
-#pragma unroll
-                for (int t = 0; t < R; ++t) u[s][t] = X[(i + t * nb) * ks + c * cs];
-#pragma unroll
-                for (int t = 1; t < R; ++t) u[s][t] = cmul(u[s][t], tw[t * k * ps.tw_step]);
-            }
-            dft<T, DIR, R>(u[s]);
-            dst[s] = q * ps.p * R + k;
+            for (int t = 0; t < R; ++t) u[s][t] = src[t * in_step];
+            turn<T, R>(u[s], tw, k * ps.tw_step);
+            dft<T, R>(u[s]);
+            at[s] = (q * ps.p * R + k) * ks + c * cs;
         }
     }
-    if constexpr ((MODE & kToGrid) != 0) {
+    __syncthreads();
 #pragma unroll
-        for (int s = 0; s < MAXB; ++s) {
-            if (dst[s] >= 0) {
-                const int64_t bc = base[line[s]];
-                if constexpr (IO == 2) {
-                    // the deconvolution: cell times (1/phi_hat) in axis order
-                    const int64_t mr = ld.mrow[line[s]];
-                    const double g = ld.f1[line[s]];
+    for (int s = 0; s < MAXB; ++s) {
+        if (at[s] < 0) continue;
+        Cx<T> *out = X + at[s];
 #pragma unroll
-                    for (int t = 0; t < R; ++t) {
-                        const int e = dst[s] + t * ps.p;
-                        if (bc >= 0 && (e < P.out_hi || e >= n - P.out_lo)) {
-                            const int64_t m = e < P.out_hi ? e : (int64_t)e - n;
-                            double amp = g;
-                            amp *= P.inv_phihat[P.eph + (m < 0 ? -m : m)];
-                            const T ta = (T)amp;
-                            modes[mr + mode_slot(m, P.eN, P.centered) * P.ems] =
-                                Cx<T>{u[s][t].re * ta, u[s][t].im * ta};
-                        }
-                    }
-                } else {
+        for (int t = 0; t < R; ++t) out[t * out_step] = u[s][t];
+    }
+    __syncthreads();
+}
+
+// The last pass (p R = n): butterflies from LDS to the grid or the modes.
+// Radix 1 only writes (an axis of one pass).
+template <typename T, int R, int IO>
+__device__ __forceinline__ void pass_out(const Cx<T> *X, const Cx<T> *tw, const LineFftAxis &P,
+                                         const LineFftPass &ps, Cx<T> *__restrict__ grid,
+                                         const LineData &ld)
+{
+    const int n = P.n, nb = ps.nb, total = P.lines * nb;
+    const int ks = P.line_major ? 1 : P.lines, cs = P.line_major ? n : 1;
+    const int in_step = nb * ks;
+    const int64_t tstep = (int64_t)nb * P.estride;
+    const int half = P.centered ? (int)(P.eN / 2) : 0;
+    const int back = P.centered ? half - n : (int)P.eN - n;
+    for (int b = (int)threadIdx.x; b < total; b += kThreads) {
+        int c, i;
+        butterfly<T>(P, ps, b, &c, &i);
+        const int64_t bc = ld.base[c];
+        if (bc < 0) continue;
+        Cx<T> u[R];
+        const Cx<T> *src = X + i * ks + c * cs;
 #pragma unroll
-                    for (int t = 0; t < R; ++t) {
-                        const int e = dst[s] + t * ps.p;
-                        if (bc >= 0 && (e < P.out_hi || e >= n - P.out_lo))
-                            grid[bc + (int64_t)e * P.estride] = u[s][t];
-                    }
+        for (int t = 0; t < R; ++t) u[t] = src[t * in_step];
+        if constexpr (R > 1) {
+            turn<T, R>(u, tw, i * ps.tw_step);
+            dft<T, R>(u);
+        }
+        if (P.exchange) exchange<T, R>(u);
+        if constexpr (IO == 2) {
+            // the deconvolution: cell times (1/phi_hat) in axis order
+            Cx<T> *row = (Cx<T> *)ld.modes + ld.mrow[c];
+            const double g = ld.f1[c];
+            const double *phi = P.inv_phihat + P.eph;
+            for_kept<R>(P.out, i, nb, n, P.out_hi, P.out_lo, [&](int t, bool in) {
+                if (in) {
+                    const int e = i + t * nb;
+                    const bool low = e < P.out_hi;
+                    double amp = g;
+                    amp *= phi[low ? e : n - e];
+                    const T ta = (T)amp;
+                    row[(int64_t)(e + (low ? half : back)) * P.ems] =
+                        Cx<T>{u[t].re * ta, u[t].im * ta};
                 }
-            }
+            });
+        } else {
+            Cx<T> *out = grid + bc + (int64_t)i * P.estride;
+            for_kept<R>(P.out, i, nb, n, P.out_hi, P.out_lo, [&](int t, bool in) {
+                if (in) out[t * tstep] = u[t];
+            });
         }
-    } else {
-        if constexpr ((MODE & kFromGrid) == 0) __syncthreads();
-#pragma unroll
-        for (int s = 0; s < MAXB; ++s) {
-            if (dst[s] >= 0) {
-#pragma unroll
-                for (int t = 0; t < R; ++t)
-                    X[(dst[s] + t * ps.p) * ks + line[s] * cs] = u[s][t];
-            }
-        }
-        __syncthreads();
     }
 }
 
-template <typename T, int DIR, int LDS, int MODE, int IO>
-__device__ inline void line_pass_any(Cx<T> *X, const Cx<T> *tw, const LineFftAxis &P,
-                                     const LineFftPass &ps, Cx<T> *grid, const LineData &base)
-{
-    switch (ps.radix) {
-    case 2: line_pass<T, DIR, 2, LDS, MODE, IO>(X, tw, P, ps, grid, base); break;
-    case 3: line_pass<T, DIR, 3, LDS, MODE, IO>(X, tw, P, ps, grid, base); break;
-    case 4: line_pass<T, DIR, 4, LDS, MODE, IO>(X, tw, P, ps, grid, base); break;
-    case 5: line_pass<T, DIR, 5, LDS, MODE, IO>(X, tw, P, ps, grid, base); break;
-    case 7: line_pass<T, DIR, 7, LDS, MODE, IO>(X, tw, P, ps, grid, base); break;
-    case 8: line_pass<T, DIR, 8, LDS, MODE, IO>(X, tw, P, ps, grid, base); break;
-    case 11: line_pass<T, DIR, 11, LDS, MODE, IO>(X, tw, P, ps, grid, base); break;
-    default: line_pass<T, DIR, 13, LDS, MODE, IO>(X, tw, P, ps, grid, base); break;
-    }
-}
+#define MNUFFT_RADICES(X) X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10) X(11) X(12) X(13) X(15) X(16)
 
 // The transform of workgroup `group`'s lines of one axis pass (P) of the
 // grid `grid` (one vector), X: (lines + 1) n elements of LDS.
-template <typename T, int DIR, int IO>
+template <typename T, int IO>
 __device__ __forceinline__ void fft_lines_body(const LineFftAxis &P, Cx<T> *__restrict__ grid,
                                                const Cx<T> *__restrict__ tw_global,
                                                int64_t group, Cx<T> *X, const LineData &ld)
 {
     int64_t *base = ld.base;
-    constexpr int LDS = LdsElems<T>::value;
     Cx<T> *tw = X + P.lines * P.n;
     const int n = P.n;
     for (int m = threadIdx.x; m < n; m += kThreads) tw[m] = tw_global[m];
-    const int64_t nlines = P.nu * P.nv;
-    const int64_t line0 = group * P.lines;
+    // (line numbers are below 2^32: at most 65536 per axis)
+    const uint32_t nu = (uint32_t)P.nu, nlines = (uint32_t)(P.nu * P.nv);
+    const uint32_t line0 = (uint32_t)group * (uint32_t)P.lines;
     for (int c = threadIdx.x; c < P.lines; c += kThreads) {
-        const int64_t L = line0 + c;
+        const uint32_t L = line0 + (uint32_t)c;
         int64_t b = -1;
         if (L < nlines) {
-            const int64_t u = L % P.nu, w = L / P.nu;
+            const int64_t w = L / nu, u = L - (uint32_t)w * nu;
             const int64_t uu = u < P.u_hi ? u : u + P.u_gap;
             const int64_t vv = w < P.v_hi ? w : w + P.v_gap;
             b = uu * P.su + vv * P.sv;
@@ -443,64 +615,62 @@ __device__ __forceinline__ void fft_lines_body(const LineFftAxis &P, Cx<T> *__re
         base[c] = b;
     }
     __syncthreads();
-    const int np = P.npass;
-    if (np == 1) {
-        line_pass_any<T, DIR, LDS, kFromGrid | kToGrid, IO>(X, tw, P, P.pass[0], grid, ld);
-        return;
+    if (P.npass < 2) return;  // one cell
+#define MNUFFT_IN(R)                                              \
+    case R: pass_in<T, R, IO == 1 ? 1 : 0>(X, P, P.pass[0], grid, ld); break;
+    switch (P.pass[0].radix) { MNUFFT_RADICES(MNUFFT_IN) }
+#undef MNUFFT_IN
+    const int last = P.npass - 1;
+    for (int s = 1; s < last; ++s) {
+#define MNUFFT_MID(R) \
+    case R: pass_mid<T, R>(X, tw, P, P.pass[s]); break;
+        switch (P.pass[s].radix) { MNUFFT_RADICES(MNUFFT_MID) }
+#undef MNUFFT_MID
     }
-    if (np == 0) return;
-    // first pass from the grid, the middle ones in LDS grouped by radix (5s,
-    // 3s, 7s, 11s, 13s, 8s, then a 4 or a 2; separate loops keep each
-    // radix's registers to itself), the last one to the grid
-    line_pass_any<T, DIR, LDS, kFromGrid, IO == 1 ? 1 : 0>(X, tw, P, P.pass[0], grid, ld);
-    const int last = np - 1;
-    int s = 1;
-    for (; s < last && P.pass[s].radix == 5; ++s)
-        line_pass<T, DIR, 5, LDS, 0, 0>(X, tw, P, P.pass[s], grid, ld);
-    for (; s < last && P.pass[s].radix == 3; ++s)
-        line_pass<T, DIR, 3, LDS, 0, 0>(X, tw, P, P.pass[s], grid, ld);
-    for (; s < last && P.pass[s].radix == 7; ++s)
-        line_pass<T, DIR, 7, LDS, 0, 0>(X, tw, P, P.pass[s], grid, ld);
-    for (; s < last && P.pass[s].radix == 11; ++s)
-        line_pass<T, DIR, 11, LDS, 0, 0>(X, tw, P, P.pass[s], grid, ld);
-    for (; s < last && P.pass[s].radix == 13; ++s)
-        line_pass<T, DIR, 13, LDS, 0, 0>(X, tw, P, P.pass[s], grid, ld);
-    for (; s < last && P.pass[s].radix == 8; ++s)
-        line_pass<T, DIR, 8, LDS, 0, 0>(X, tw, P, P.pass[s], grid, ld);
-    for (; s < last && P.pass[s].radix == 4; ++s)
-        line_pass<T, DIR, 4, LDS, 0, 0>(X, tw, P, P.pass[s], grid, ld);
-    for (; s < last && P.pass[s].radix == 2; ++s)
-        line_pass<T, DIR, 2, LDS, 0, 0>(X, tw, P, P.pass[s], grid, ld);
-    line_pass_any<T, DIR, LDS, kToGrid, IO == 2 ? 2 : 0>(X, tw, P, P.pass[last], grid, ld);
+#define MNUFFT_OUT(R)                                             \
+    case R: pass_out<T, R, IO == 2 ? 2 : 0>(X, tw, P, P.pass[last], grid, ld); break;
+    switch (P.pass[last].radix) { MNUFFT_RADICES(MNUFFT_OUT) MNUFFT_OUT(1) }
+#undef MNUFFT_OUT
+}
+
+// Workgroups go round the eight XCDs in turn; neighbouring groups of a
+// strided pass share cache lines, DRAM pages and page translations, so each
+// XCD takes a contiguous run of groups.
+__device__ inline int64_t xcd_group(uint32_t block, uint32_t blocks)
+{
+    const uint32_t x = block & 7u, per = blocks >> 3, rest = blocks & 7u;
+    return (int64_t)x * per + (x < rest ? x : rest) + (block >> 3);
 }
 
 // One plan's axis pass: workgroup (group, vector); IO / modes_all: this
 // launch's mode reads or writes (all vectors' modes).
-template <typename T, int DIR, int IO>
-__global__ __launch_bounds__(kThreads) void k_fft_lines(LineFftAxis P,
-                                                        void *modes_all, T *__restrict__ data,
-                                                        const Cx<T> *__restrict__ tw_global)
+template <typename T, int IO>
+__global__ __launch_bounds__(kThreads, 4) void k_fft_lines(const LineFftAxis *__restrict__ ax,
+                                                           void *modes_all, T *__restrict__ data,
+                                                           const Cx<T> *__restrict__ tw_global)
 {
+    const LineFftAxis &P = *ax;
     extern __shared__ __align__(16) unsigned char lds_raw[];
     Cx<T> *grid = (Cx<T> *)data + (int64_t)blockIdx.y * P.vec_stride;
+    const int64_t group = P.line_major ? (int64_t)blockIdx.x : xcd_group(blockIdx.x, gridDim.x);
     if constexpr (IO == 0) {
         __shared__ int64_t base[kMaxGroupLines];
-        fft_lines_body<T, DIR, 0>(P, grid, tw_global, blockIdx.x, (Cx<T> *)lds_raw,
-                                  LineData{base, nullptr, nullptr, nullptr, nullptr});
+        fft_lines_body<T, 0>(P, grid, tw_global, group, (Cx<T> *)lds_raw,
+                             LineData{base, nullptr, nullptr, nullptr, nullptr});
     } else {
         __shared__ int64_t base[kMaxGroupLines], mrow[kMaxGroupLines];
         __shared__ double f1[kMaxGroupLines], f2[kMaxGroupLines];
         Cx<T> *modes = (Cx<T> *)modes_all + (int64_t)blockIdx.y * P.mode_total;
-        fft_lines_body<T, DIR, IO>(P, grid, tw_global, blockIdx.x, (Cx<T> *)lds_raw,
-                                   LineData{base, mrow, f1, f2, modes});
+        fft_lines_body<T, IO>(P, grid, tw_global, group, (Cx<T> *)lds_raw,
+                              LineData{base, mrow, f1, f2, modes});
     }
 }
 
 // The same axis pass of many plans (one vector each) in one launch: job q
 // takes workgroups [group0[q], group0[q + 1]).
-template <typename T, int DIR>
-__global__ __launch_bounds__(kThreads) void k_fft_lines_many(const LineFftJob *__restrict__ jobs,
-                                                             int njobs)
+template <typename T>
+__global__ __launch_bounds__(kThreads, 4) void k_fft_lines_many(const LineFftJob *__restrict__ jobs,
+                                                                int njobs)
 {
     extern __shared__ __align__(16) unsigned char lds_raw[];
     __shared__ int64_t base[kMaxGroupLines];
@@ -513,52 +683,66 @@ __global__ __launch_bounds__(kThreads) void k_fft_lines_many(const LineFftJob *_
         else
             hi = mid - 1;
     }
-    const LineFftJob &J = jobs[lo];
-    fft_lines_body<T, DIR, 0>(J.ax, (Cx<T> *)J.grid, (const Cx<T> *)J.tw, b - J.group0,
-                              (Cx<T> *)lds_raw, LineData{base, nullptr, nullptr, nullptr, nullptr});
+    // the job is the workgroup's: its fields in scalar registers
+    const LineFftJob &J = jobs[__builtin_amdgcn_readfirstlane(lo)];
+    fft_lines_body<T, 0>(*J.ax, (Cx<T> *)J.grid, (const Cx<T> *)J.tw, b - J.group0,
+                         (Cx<T> *)lds_raw, LineData{base, nullptr, nullptr, nullptr, nullptr});
 }
 
-// Radix plan: 5s, 3s, 7s, 11s, 13s, 8s, then a 4 or a 2; false for other
-// prime factors.
+// Radix plan: the fewest passes of radix 2 .. 16 (each costs an LDS round
+// trip of every element, two barriers and the twiddles), of those the one
+// with the smallest largest radix (its registers, its idle lanes), larger
+// radices first (the first pass's reads are in flight together); false for
+// prime factors beyond 13.  At 900 cells 10 x 10 x 9 instead of 5 x 5 x 3 x 3
+// x 4, at 256 16 x 16 instead of 8 x 8 x 4.
 bool radix_plan(int n, LineFftAxis *ax)
 {
-    std::vector<int> r;
-    int m = n;
-    while (m % 5 == 0) {
-        r.push_back(5);
-        m /= 5;
-    }
-    while (m % 3 == 0) {
-        r.push_back(3);
-        m /= 3;
-    }
-    for (int q : {7, 11, 13})
-        while (m % q == 0) {
-            r.push_back(q);
-            m /= q;
+    int best[kLineFftMaxPasses], cur[kLineFftMaxPasses], best_count = 0;
+    const auto search = [&](const auto &self, int m, int most, int depth) -> void {
+        if (m == 1) {
+            if (best_count == 0 || depth < best_count ||
+                (depth == best_count && cur[0] < best[0])) {
+                best_count = depth;
+                for (int i = 0; i < depth; ++i) best[i] = cur[i];
+            }
+            return;
         }
-    while (m % 8 == 0) {
-        r.push_back(8);
-        m /= 8;
-    }
-    while (m % 4 == 0) {
-        r.push_back(4);
-        m /= 4;
-    }
-    while (m % 2 == 0) {
-        r.push_back(2);
-        m /= 2;
-    }
-    if (m != 1 || (int)r.size() > kLineFftMaxPasses) return false;
+        if (depth == kLineFftMaxPasses || (best_count && depth >= best_count)) return;
+        for (int r = std::min(most, m); r >= 2; --r)
+            if (m % r == 0 && r != 14) {
+                cur[depth] = r;
+                self(self, m / r, r, depth + 1);
+            }
+    };
+    if (n < 1) return false;
+    search(search, n, 16, 0);
+    if (best_count == 0 && n != 1) return false;
     ax->n = n;
-    ax->npass = (int)r.size();
+    ax->npass = best_count;
     int p = 1;
-    for (size_t i = 0; i < r.size(); ++i) {
-        ax->pass[i] = LineFftPass{r[i], p, n / (p * r[i])};
-        p *= r[i];
+    for (int i = 0; i < best_count; ++i) {
+        const int r = best[i];
+        ax->pass[i] = LineFftPass{r, p, n / (p * r), n / r, (float)r / (float)n, 1.0f / (float)p};
+        p *= r;
     }
-    ax->inv_n = 1.0f / (float)n;
+    if (ax->npass == 1)  // the write as a pass of its own
+        ax->pass[ax->npass++] = LineFftPass{1, n, 1, n, 1.0f / (float)n, 1.0f / (float)n};
     return true;
+}
+
+// Masks of a pass of radix r for the kept window [0, hi) and [n - lo, n).
+LineFftKept kept_masks(int r, int n, int hi, int lo)
+{
+    LineFftKept m{0u, 0u};
+    const int nb = n / r;
+    for (int t = 0; t < r; ++t) {
+        const int e0 = t * nb, e1 = e0 + nb;
+        if (e1 <= hi || e0 >= n - lo)
+            m.all |= 1u << t;
+        else if (e0 < hi || e1 > n - lo)
+            m.some |= 1u << t;
+    }
+    return m;
 }
 
 // Lines per workgroup: the lines and the twiddle table fit the LDS array;
@@ -572,14 +756,10 @@ bool wide_lds()
     static bool ok = false;
     std::call_once(once, [] {
         const void *kernels[] = {
-            (const void *)k_fft_lines<float, 1, 0>,      (const void *)k_fft_lines<float, 1, 1>,
-            (const void *)k_fft_lines<float, 1, 2>,      (const void *)k_fft_lines<float, -1, 0>,
-            (const void *)k_fft_lines<float, -1, 1>,     (const void *)k_fft_lines<float, -1, 2>,
-            (const void *)k_fft_lines<double, 1, 0>,     (const void *)k_fft_lines<double, 1, 1>,
-            (const void *)k_fft_lines<double, 1, 2>,     (const void *)k_fft_lines<double, -1, 0>,
-            (const void *)k_fft_lines<double, -1, 1>,    (const void *)k_fft_lines<double, -1, 2>,
-            (const void *)k_fft_lines_many<float, 1>,    (const void *)k_fft_lines_many<float, -1>,
-            (const void *)k_fft_lines_many<double, 1>,   (const void *)k_fft_lines_many<double, -1>};
+            (const void *)k_fft_lines<float, 0>,  (const void *)k_fft_lines<float, 1>,
+            (const void *)k_fft_lines<float, 2>,  (const void *)k_fft_lines<double, 0>,
+            (const void *)k_fft_lines<double, 1>, (const void *)k_fft_lines<double, 2>,
+            (const void *)k_fft_lines_many<float>, (const void *)k_fft_lines_many<double>};
         ok = true;
         for (const void *k : kernels)
             ok = ok && hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -594,17 +774,18 @@ bool group_lines(int n, bool line_major, bool f64, int64_t count, bool wide, Lin
 {
     const int lds = f64 ? (wide ? LdsElems<double>::value : LdsElems<double>::base)
                         : (wide ? LdsElems<float>::value : LdsElems<float>::base);
+    const int most = f64 ? LdsElems<double>::group : LdsElems<float>::group;
     if (2 * n > lds) return false;
     ax->line_major = line_major ? 1 : 0;
     if (line_major) {
         const int64_t fill = std::max<int64_t>((kThreads + n - 1) / n, count / 2048);
         int c = (int)std::min<int64_t>(kMaxGroupLines, fill);
-        while (c > 1 && (c + 1) * n > lds) --c;
+        while (c > 1 && ((c + 1) * n > lds || c * n > most)) --c;
         ax->lines = c;
         ax->log_lines = 0;
     } else {
         int c = f64 ? LdsElems<double>::columns : LdsElems<float>::columns;
-        while (c > 1 && (c + 1) * n > lds) c /= 2;
+        while (c > 1 && ((c + 1) * n > lds || c * n > most)) c /= 2;
         ax->lines = c;
         ax->log_lines = 0;
         while ((1 << ax->log_lines) < c) ++ax->log_lines;
@@ -647,8 +828,7 @@ int64_t LineFft::row_length_limit(bool f64)
 
 LineFft::~LineFft()
 {
-    for (void *&p : tw_)
-        if (p) (void)hipFree(p);
+    if (tables_) (void)hipFree(tables_);
 }
 
 bool LineFft::init(int dim, const int64_t *fine, const int64_t *n_modes, int type, bool f64,
@@ -749,16 +929,31 @@ bool LineFft::init(int dim, const int64_t *fine, const int64_t *n_modes, int typ
     mx.eN = n_modes[ea];
     mx.ems = mstride[ea];
     mx.eph = phihat_off[ea];
-    // twiddles w_n^m = exp(dir 2 pi i m / n), from long double
+    for (int a = 0; a < dim; ++a) {
+        LineFftAxis &x = ax_[a];
+        if (x.npass == 0) continue;
+        x.exchange = dir_ < 0 ? 1 : 0;
+        x.in = kept_masks(x.pass[0].radix, x.n, x.in_hi, x.in_lo);
+        x.out = kept_masks(x.pass[x.npass - 1].radix, x.n, x.out_hi, x.out_lo);
+    }
+    // one device allocation: the axes (for batches), then per axis the
+    // twiddles w_n^m = exp(2 pi i m / n), from long double
+    const size_t eb = f64 ? 2 * sizeof(double) : 2 * sizeof(float);
+    size_t at[3], bytes = (sizeof(ax_) + 255) / 256 * 256;
+    for (int a = 0; a < dim; ++a) {
+        at[a] = bytes;
+        bytes += (eb * (size_t)fine[a] + 255) / 256 * 256;
+    }
+    std::vector<unsigned char> host(bytes, 0);
+    std::memcpy(host.data(), ax_, sizeof(ax_));
     for (int a = 0; a < dim; ++a) {
         const int n = (int)fine[a];
-        const size_t eb = f64 ? 2 * sizeof(double) : 2 * sizeof(float);
-        std::vector<double> hd(f64 ? 2 * (size_t)n : 0);
-        std::vector<float> hf(f64 ? 0 : 2 * (size_t)n);
+        float *hf = (float *)(host.data() + at[a]);
+        double *hd = (double *)(host.data() + at[a]);
         for (int m = 0; m < n; ++m) {
             const long double ang =
                 2.0L * 3.14159265358979323846264338327950288L * (long double)m / (long double)n;
-            const long double c = cosl(ang), s = (long double)dir_ * sinl(ang);
+            const long double c = cosl(ang), s = sinl(ang);
             if (f64) {
                 hd[2 * m] = (double)c;
                 hd[2 * m + 1] = (double)s;
@@ -767,14 +962,15 @@ bool LineFft::init(int dim, const int64_t *fine, const int64_t *n_modes, int typ
                 hf[2 * m + 1] = (float)s;
             }
         }
-        if (tw_[a]) (void)hipFree(tw_[a]);
-        tw_[a] = nullptr;
-        if (!hip_ok(hipMalloc(&tw_[a], eb * (size_t)n), "line FFT twiddles") ||
-            !hip_ok(hipMemcpy(tw_[a], f64 ? (const void *)hd.data() : (const void *)hf.data(),
-                              eb * (size_t)n, hipMemcpyHostToDevice),
-                    "line FFT twiddle upload"))
-            return false;
     }
+    if (tables_) (void)hipFree(tables_);
+    tables_ = nullptr;
+    if (!hip_ok(hipMalloc(&tables_, bytes), "line FFT tables") ||
+        !hip_ok(hipMemcpy(tables_, host.data(), bytes, hipMemcpyHostToDevice),
+                "line FFT table upload"))
+        return false;
+    dev_ax_ = (LineFftAxis *)tables_;
+    for (int a = 0; a < dim; ++a) tw_[a] = (char *)tables_ + at[a];
     return true;
 }
 
@@ -788,7 +984,7 @@ struct JobChunk {
 
 __global__ void k_line_jobs(JobChunk chunk, LineFftJob *dst)
 {
-    if ((int)threadIdx.x < chunk.n) dst[threadIdx.x] = chunk.j[threadIdx.x];
+    for (int i = threadIdx.x; i < chunk.n; i += blockDim.x) dst[i] = chunk.j[i];
 }
 
 }  // namespace
@@ -805,31 +1001,28 @@ bool LineFft::run_many(const std::vector<const LineFft *> &ffts, const std::vect
             set_error("batched line FFT: plans of one rank and precision");
             return false;
         }
-    // jobs grouped by (axis, sign), each group's workgroups numbered from 0
+    // jobs grouped by axis, each group's workgroups numbered from 0
     struct Launch {
-        int dir;
         size_t first, count;
         int64_t groups;
         size_t lds;
     };
     std::vector<LineFftJob> all;
     std::vector<Launch> launches;
-    for (int a = 0; a < naxes; ++a)
-        for (int dir : {1, -1}) {
-            Launch L{dir, all.size(), 0, 0, 0};
-            for (size_t i = 0; i < ffts.size(); ++i) {
-                const LineFft &f = *ffts[i];
-                if (f.dir_ != dir) continue;
-                const LineFftAxis &x = f.ax_[a];
-                const int64_t g = (x.nu * x.nv + x.lines - 1) / x.lines;
-                if (g == 0) continue;
-                all.push_back(LineFftJob{x, grids[i], f.tw_[a], L.groups});
-                L.groups += g;
-                L.lds = std::max(L.lds, (size_t)(x.lines + 1) * (size_t)x.n * (f64 ? 16 : 8));
-            }
-            L.count = all.size() - L.first;
-            if (L.count) launches.push_back(L);
+    for (int a = 0; a < naxes; ++a) {
+        Launch L{all.size(), 0, 0, 0};
+        for (size_t i = 0; i < ffts.size(); ++i) {
+            const LineFft &f = *ffts[i];
+            const LineFftAxis &x = f.ax_[a];
+            const int64_t g = (x.nu * x.nv + x.lines - 1) / x.lines;
+            if (g == 0) continue;
+            all.push_back(LineFftJob{f.dev_ax_ + a, grids[i], f.tw_[a], L.groups});
+            L.groups += g;
+            L.lds = std::max(L.lds, (size_t)(x.lines + 1) * (size_t)x.n * (f64 ? 16 : 8));
         }
+        L.count = all.size() - L.first;
+        if (L.count) launches.push_back(L);
+    }
     const int64_t n = (int64_t)all.size();
     if (n > *cap) {
         if (*jobs) (void)hipFree(*jobs);
@@ -851,17 +1044,10 @@ bool LineFft::run_many(const std::vector<const LineFft *> &ffts, const std::vect
         }
         const dim3 g((unsigned)L.groups);
         const LineFftJob *J = *jobs + L.first;
-        if (f64) {
-            if (L.dir > 0)
-                k_fft_lines_many<double, 1><<<g, kThreads, L.lds, stream>>>(J, (int)L.count);
-            else
-                k_fft_lines_many<double, -1><<<g, kThreads, L.lds, stream>>>(J, (int)L.count);
-        } else {
-            if (L.dir > 0)
-                k_fft_lines_many<float, 1><<<g, kThreads, L.lds, stream>>>(J, (int)L.count);
-            else
-                k_fft_lines_many<float, -1><<<g, kThreads, L.lds, stream>>>(J, (int)L.count);
-        }
+        if (f64)
+            k_fft_lines_many<double><<<g, kThreads, L.lds, stream>>>(J, (int)L.count);
+        else
+            k_fft_lines_many<float><<<g, kThreads, L.lds, stream>>>(J, (int)L.count);
     }
     return hip_ok(hipGetLastError(), "batched line FFT launch");
 }
@@ -869,24 +1055,15 @@ bool LineFft::run_many(const std::vector<const LineFft *> &ffts, const std::vect
 namespace {
 
 template <typename T>
-void launch_axis(int dir, int io, dim3 g, size_t lds, hipStream_t stream, const LineFftAxis *hx,
-                 void *mv, T *d, const Cx<T> *t)
+void launch_axis(int io, dim3 g, size_t lds, hipStream_t stream, const LineFftAxis *ax, void *mv,
+                 T *d, const Cx<T> *t)
 {
-    if (dir > 0) {
-        if (io == 1)
-            k_fft_lines<T, 1, 1><<<g, kThreads, lds, stream>>>(*hx, mv, d, t);
-        else if (io == 2)
-            k_fft_lines<T, 1, 2><<<g, kThreads, lds, stream>>>(*hx, mv, d, t);
-        else
-            k_fft_lines<T, 1, 0><<<g, kThreads, lds, stream>>>(*hx, mv, d, t);
-    } else {
-        if (io == 1)
-            k_fft_lines<T, -1, 1><<<g, kThreads, lds, stream>>>(*hx, mv, d, t);
-        else if (io == 2)
-            k_fft_lines<T, -1, 2><<<g, kThreads, lds, stream>>>(*hx, mv, d, t);
-        else
-            k_fft_lines<T, -1, 0><<<g, kThreads, lds, stream>>>(*hx, mv, d, t);
-    }
+    if (io == 1)
+        k_fft_lines<T, 1><<<g, kThreads, lds, stream>>>(ax, mv, d, t);
+    else if (io == 2)
+        k_fft_lines<T, 2><<<g, kThreads, lds, stream>>>(ax, mv, d, t);
+    else
+        k_fft_lines<T, 0><<<g, kThreads, lds, stream>>>(ax, mv, d, t);
 }
 
 }  // namespace
@@ -907,14 +1084,14 @@ bool LineFft::run(void *data, int64_t vectors, hipStream_t stream, void *modes) 
             if (groups == 0) continue;
             const dim3 g((unsigned)groups, vc);
             const size_t lds = (size_t)(x.lines + 1) * (size_t)x.n * eb;
-            const LineFftAxis *hx = &ax_[a];
+            const LineFftAxis *hx = dev_ax_ + a;
             if (f64_) {
                 double *d = (double *)data + 2 * v0 * fine_total_;
-                launch_axis<double>(dir_, mode_io, g, lds, stream, hx, mv, d,
+                launch_axis<double>(mode_io, g, lds, stream, hx, mv, d,
                                     (const Cx<double> *)tw_[a]);
             } else {
                 float *d = (float *)data + 2 * v0 * fine_total_;
-                launch_axis<float>(dir_, mode_io, g, lds, stream, hx, mv, d,
+                launch_axis<float>(mode_io, g, lds, stream, hx, mv, d,
                                    (const Cx<float> *)tw_[a]);
             }
         }

@@ -1,7 +1,7 @@
 // Fine-grid FFT of 2D and 3D plans as passes of batched line transforms
 // (one per axis), each line staged in LDS and transformed there by
-// Stockham passes of radix 2, 3, 4, 5, 7, 8, 11 and 13 (the fine lengths'
-// prime factors), with the passes pruned to the
+// Stockham passes of radix 2 to 16 (products of the fine lengths' prime
+// factors 2, 3, 5, 7, 11 and 13), with the passes pruned to the
 // lines that carry data: a type-2 grid holds modes only in the kept window
 // of every axis (the other cells are never read), and a type-1 grid is
 // needed only at the kept window, so
@@ -31,10 +31,18 @@
 
 namespace mnufft {
 
-constexpr int kLineFftMaxPasses = 24;
+constexpr int kLineFftMaxPasses = 6;
 
 struct LineFftPass {
     int radix, p, tw_step;  // radix, product of the earlier radices, n / (p radix)
+    int nb;                 // butterflies of a line, n / radix
+    float inv_nb, inv_p;
+};
+
+// Bit t of a butterfly's elements i + t nb: all of them are in the kept
+// window, or some are.
+struct LineFftKept {
+    uint32_t all, some;
 };
 
 // One axis pass: lines enumerated as (u, v), u fastest, each mapped through
@@ -46,11 +54,12 @@ struct LineFftAxis {
     LineFftPass pass[kLineFftMaxPasses] = {};
     int lines = 1, log_lines = 0;
     int line_major = 0;  // the axis is the contiguous one
+    int exchange = 0;    // real and imaginary parts exchanged in and out (isign < 0)
     int64_t estride = 1;
     int64_t nu = 1, nv = 1, u_hi = 1, u_gap = 0, v_hi = 1, v_gap = 0, su = 0, sv = 0;
     int in_hi = 1, in_lo = 0, out_hi = 1, out_lo = 0;  // elements read / written
+    LineFftKept in = {}, out = {};  // of the first pass's reads, the last one's writes
     int64_t vec_stride = 0;
-    float inv_n = 1.0f;
     // Modes in place of the grid (chosen per launch): the first pass reads
     // each cell from the modes, scaled by the deconvolution factors (type 2),
     // or the last pass writes each kept cell to the modes, scaled (type 1).
@@ -67,7 +76,7 @@ struct LineFftAxis {
 // One plan's axis pass inside a batched launch: its workgroups start at
 // group0 of the launch.
 struct LineFftJob {
-    LineFftAxis ax;
+    const LineFftAxis *ax;  // in device memory
     void *grid;
     const void *tw;
     int64_t group0;
@@ -91,7 +100,7 @@ public:
     // the results equal predeconvolution + FFT (+ deconvolution) bit for bit.
     bool run(void *data, int64_t vectors, hipStream_t stream, void *modes = nullptr) const;
     // One vector of each of many plans (one rank and precision): every axis
-    // pass of all of them in one launch per transform sign.  The job table
+    // pass of all of them in one launch.  The job table
     // (*jobs, *cap entries) grows as needed and is filled by kernel launches
     // (no host copies), so the call can be captured in a graph.
     static bool run_many(const std::vector<const LineFft *> &ffts,
@@ -104,7 +113,9 @@ private:
     int dir_ = 1;
     int64_t fine_total_ = 1;
     LineFftAxis ax_[3];
-    void *tw_[3] = {nullptr, nullptr, nullptr};
+    void *tw_[3] = {nullptr, nullptr, nullptr};  // views of tables_
+    LineFftAxis *dev_ax_ = nullptr;  // ax_ on the device, first in tables_
+    void *tables_ = nullptr;
 };
 
 }  // namespace mnufft
