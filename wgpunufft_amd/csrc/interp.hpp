@@ -6,7 +6,8 @@
 namespace mnufft {
 
 // out[v * M + j] = sum over the support of point j of grid[v] * weights, for
-// the `vectors` grids; points are visited in the order of `sorted`.
+// the `vectors` grids; points are visited in the order of `sorted` (null:
+// their own order).
 template <int D, typename T>
 bool interpolate(int64_t M, int64_t vectors, const uint32_t *sorted, const T *coords,
                  const GridParams &g, const T *grid, T *out, hipStream_t stream);
@@ -38,6 +39,12 @@ template <typename T>
 bool interpolate_tiled2(int64_t M, int64_t vectors, const uint32_t *sorted,
                         const uint32_t *offsets, const T *coords, const GridParams &g,
                         const T *grid, T *out, hipStream_t stream);
+
+// The same sums (bit for bit) for points in their own order, read from the
+// grid without tiles: few points.
+template <typename T>
+bool interpolate_direct2(int64_t M, int64_t vectors, const T *coords, const GridParams &g,
+                         const T *grid, T *out, hipStream_t stream);
 
 // The same for the problems of a batch (F32): offsets over the combined bin
 // list, one launch per kernel width c over bins [bin_lo[c], bin_hi[c]) (the

@@ -319,6 +319,36 @@ bool Plan::tiled2_interp() const
     return true;
 }
 
+Plan::Interp Plan::interp_kind(int64_t M) const
+{
+    // Unsorted while the gather's cache-line traffic (w^(d-1) rows of w cells
+    // and a line of slack) stays below 128 MB, in 1D on any grid of at most
+    // 64 MB: the bin sort costs 45 to 65 us and earns the gather less.  Whole
+    // encodes / executes, sorted against unsorted: 2D w7 on 1024^2 cells, 1e5
+    // points 127 / 58 against 62 / 52 us, 4e5 160 / 60 against 88 / 78; 3D w7
+    // on 256^3, 2e4 points 237 / 170 against 181 / 171, 16e4 347 / 264 against
+    // 339 / 330; 1D w7 on 1e5 cells, 3e6 points 278 / 142 against 128 / 119.
+    if (dim <= 3) {
+        double rows = 1.0;
+        for (int a = 1; a < dim; ++a) rows *= kernel.width;
+        const double bytes = (double)M * rows * (2.0 * real_bytes() * kernel.width + 64.0);
+        if (bytes <= 128e6 || (dim == 1 && 2.0 * real_bytes() * (double)fine_total <= 64e6))
+            return tiled2_interp() ? Interp::Direct2 : Interp::Unsorted;
+    }
+    // A 3D tile costs the loads of its halo, as much as gathering 20 points:
+    // executes gathered against tiled, w7 on 256^3 (32768 tiles) 3.2e5 points
+    // 309 against 431, 6.4e5 397 / 434, 1.3e6 599 / 450; FP64 w10 on 128^3
+    // (4096 tiles) 4e4 points 153 against 211, 8e4 230 / 216.  (A 2D tile
+    // 12 points; the sets below that are unsorted already.)
+    const double tiles = (double)type2_geometry().nbins;
+    if ((double)M >= 20.0 * tiles) {
+        if (tiled_interp()) return Interp::Tiled3;
+        if (wide3_interp()) return Interp::Wide3;
+    }
+    if (tiled2_interp()) return Interp::Tiled2;
+    return Interp::Gather;
+}
+
 GridParams Plan::type2_geometry() const
 {
     int64_t side[kMaxDims] = {1, 1, 1, 1, 1, 1, 1, 1};
@@ -587,10 +617,23 @@ bool Plan::begin_call()
     while ((int64_t)slots.size() <= slot) {
         slots.emplace_back();
         for (auto &e : slots.back().ev)
-            if (!hip_ok(hipEventCreate(&e), "timing event")) return false;
+            // (timing only: nothing reads memory after these events, so no
+            // system-scope fence)
+            if (!hip_ok(hipEventCreateWithFlags(&e, hipEventDisableSystemFence), "timing event"))
+                return false;
     }
     for (auto &u : slots[slot].used) u = false;
     return true;
+}
+
+// The end of one stage and the beginning of the next, as one event (an event
+// costs a call 2 to 3 us).
+void Plan::mark_between(int done, int next, hipStream_t stream)
+{
+    if (!timing || slot >= (int64_t)slots.size()) return;
+    mark(done, true, stream);
+    slots[slot].used[next] = true;
+    slots[slot].begin[next] = 2 * done + 1;
 }
 
 void Plan::mark(int stage, bool end, hipStream_t stream)
@@ -598,6 +641,7 @@ void Plan::mark(int stage, bool end, hipStream_t stream)
     if (!timing || slot >= (int64_t)slots.size()) return;
     (void)hipEventRecord(slots[slot].ev[2 * stage + (end ? 1 : 0)], stream);
     slots[slot].used[stage] = true;
+    if (!end) slots[slot].begin[stage] = 2 * stage;
 }
 
 void Plan::reset_marks() { (void)begin_call(); }
@@ -620,10 +664,9 @@ bool Plan::set_points_t(int64_t M, const T *pts, hipStream_t stream)
         binned_order = point_order;
         binned_dense = sizeof(T) == 4 ? dense_threshold(gp) : 0u;
         mark(kStageSort, false, stream);
-        if (!sorter.sort<D, T>(M, pts, gp, point_order, stream)) return false;
-        mark(kStageSort, true, stream);
         if (!ensure_records(M)) return false;
-        mark(kStagePrepare, false, stream);
+        if (!sorter.sort<D, T>(M, pts, gp, point_order, stream)) return false;
+        mark_between(kStageSort, kStagePrepare, stream);
         if (binned_dense && !dense.classify(gp, spread_params(), sorter.offsets(), stream))
             return false;
         if (!sorter.prepare<D, T>(M, pts, gp, point_order, rec_start, (T *)rec_off, rec_perm,
@@ -632,9 +675,12 @@ bool Plan::set_points_t(int64_t M, const T *pts, hipStream_t stream)
         mark(kStagePrepare, true, stream);
     } else {
         gp = type2_geometry();
-        mark(kStageSort, false, stream);
-        if (!sorter.sort<D, T>(M, pts, gp, BinOrder::Grouped, stream)) return false;
-        mark(kStageSort, true, stream);
+        binned_interp = interp_kind(M);
+        if (!unsorted(binned_interp)) {
+            mark(kStageSort, false, stream);
+            if (!sorter.sort<D, T>(M, pts, gp, BinOrder::Grouped, stream)) return false;
+            mark(kStageSort, true, stream);
+        }
     }
     points_set = true;
     return true;
@@ -661,7 +707,10 @@ bool Plan::execute_t(int64_t active, const T *in, T *out, hipStream_t stream, bo
         bool timed = timing && slot < (int64_t)slots.size();
         spreader.kernel_start = timed ? slots[slot].ev[2 * kStageSpreadKernel] : nullptr;
         spreader.kernel_end = timed ? slots[slot].ev[2 * kStageSpreadKernel + 1] : nullptr;
-        if (timed) slots[slot].used[kStageSpreadKernel] = true;
+        if (timed) {
+            slots[slot].used[kStageSpreadKernel] = true;
+            slots[slot].begin[kStageSpreadKernel] = 2 * kStageSpreadKernel;
+        }
         // dense-bin records read their strengths in point order
         if (!gather_strengths<T>(M, active, rec_perm, in, (T *)c_sorted, stream,
                                  binned_dense ? dense.before + gp.nbins : nullptr))
@@ -672,9 +721,11 @@ bool Plan::execute_t(int64_t active, const T *in, T *out, hipStream_t stream, bo
                                    (const T *)rec_off, (const T *)c_sorted, M, active, (T *)grid,
                                    stream, spread_method, binned_dense ? &dense : nullptr))
             return false;
-        mark(kStageSpread, true, stream);
-        if (spread_only) return true;
-        mark(kStageFft, false, stream);
+        if (spread_only) {
+            mark(kStageSpread, true, stream);
+            return true;
+        }
+        mark_between(kStageSpread, kStageFft, stream);
         if (use_line_fft()) {
             // the last line pass writes the deconvolved modes
             if (!ensure_fft(active) || !line_fft->run(grid, active, stream, out)) return false;
@@ -682,8 +733,7 @@ bool Plan::execute_t(int64_t active, const T *in, T *out, hipStream_t stream, bo
             return true;
         }
         if (!fft(active, grid, stream)) return false;
-        mark(kStageFft, true, stream);
-        mark(kStageDeconv, false, stream);
+        mark_between(kStageFft, kStageDeconv, stream);
         if (!deconvolve<D, T>(mp, d_inv_phihat, (const T *)grid, out, active, stream))
             return false;
         mark(kStageDeconv, true, stream);
@@ -694,37 +744,38 @@ bool Plan::execute_t(int64_t active, const T *in, T *out, hipStream_t stream, bo
             mark(kStageFft, false, stream);
             if (!ensure_fft(active) || !line_fft->run(grid, active, stream, (void *)in))
                 return false;
-            mark(kStageFft, true, stream);
         } else {
             mark(kStageDeconv, false, stream);
             if (!predeconvolve<D, T>(mp, d_inv_phihat, in, (T *)grid, active, stream))
                 return false;
-            mark(kStageDeconv, true, stream);
-            mark(kStageFft, false, stream);
+            mark_between(kStageDeconv, kStageFft, stream);
             if (!fft(active, grid, stream)) return false;
-            mark(kStageFft, true, stream);
         }
-        mark(kStageInterp, false, stream);
-        if (D == 3 && tiled_interp()) {
+        mark_between(kStageFft, kStageInterp, stream);
+        if (D == 3 && binned_interp == Interp::Tiled3) {
             // bin item offsets and the scratch of their scan
             if (!ensure_items(gp.nbins + 1 + scan_tiles(gp.nbins + 1) + 1)) return false;
             if (!interpolate_tiled3<T>(M, active, sorter.sorted(), sorter.offsets(), item_off,
                                        (const T *)points, gp, (const T *)grid, out, stream))
                 return false;
-        } else if (D == 3 && sizeof(T) == 8 && wide3_interp() && M >= 8 * gp.nbins) {
-            // a tile costs its halo's loads, as much as gathering two to
-            // five points (tile and halo over w^3 cells): from 8 points a
-            // tile on
+        } else if (D == 3 && sizeof(T) == 8 && binned_interp == Interp::Wide3) {
             if (!ensure_items(gp.nbins + 1 + scan_tiles(gp.nbins + 1) + 1)) return false;
             if (!interpolate_wide3(M, active, sorter.sorted(), sorter.offsets(), item_off,
                                    (const double *)points, gp, (const double *)grid,
                                    (double *)out, stream))
                 return false;
-        } else if (D == 2 && tiled2_interp()) {
+        } else if (D == 2 && binned_interp == Interp::Direct2) {
+            if (!interpolate_direct2<T>(M, active, (const T *)points, gp, (const T *)grid, out,
+                                        stream))
+                return false;
+        } else if (D == 2 && binned_interp == Interp::Tiled2) {
             if (!interpolate_tiled2<T>(M, active, sorter.sorted(), sorter.offsets(),
                                        (const T *)points, gp, (const T *)grid, out, stream))
                 return false;
-        } else if (!interpolate<D, T>(M, active, sorter.sorted(), (const T *)points, gp,
+        } else if (!interpolate<D, T>(M, active,
+                                      binned_interp == Interp::Unsorted ? nullptr
+                                                                        : sorter.sorted(),
+                                      (const T *)points, gp,
                                       (const T *)grid, out, stream)) {
             return false;
         }
@@ -1134,7 +1185,8 @@ bool Plan::stage_times(double *ms, int n, int64_t *calls)
             if (!slots[sl].used[st]) continue;
             if (!hip_ok(hipEventSynchronize(slots[sl].ev[2 * st + 1]), "stage event")) return false;
             float t = 0.0f;
-            if (hipEventElapsedTime(&t, slots[sl].ev[2 * st], slots[sl].ev[2 * st + 1]) ==
+            if (hipEventElapsedTime(&t, slots[sl].ev[slots[sl].begin[st]],
+                                    slots[sl].ev[2 * st + 1]) ==
                 hipSuccess)
                 ms[st] = (ms[st] < 0 ? 0.0 : ms[st]) + t;
         }
@@ -1221,7 +1273,9 @@ bool execute_type2_many_t(int64_t count, Plan *const *plans, const int64_t *M,
     std::vector<int64_t> order((size_t)count);
     for (int64_t i = 0; i < count; ++i) order[(size_t)i] = i;
     auto tiled_w = [&](int64_t i) {
-        const bool tiled = (D == 2 && plans[i]->tiled2_interp()) || (D == 3 && plans[i]->tiled_interp());
+        const Plan::Interp kind = plans[i]->interp_kind(M[i]);
+        const bool tiled = kind == Plan::Interp::Tiled2 || kind == Plan::Interp::Direct2 ||
+                           kind == Plan::Interp::Tiled3;
         return tiled ? plans[i]->kernel.width : 1000;
     };
     std::stable_sort(order.begin(), order.end(),

@@ -94,9 +94,17 @@ struct Plan {
     }
 
     // points
+    // The type-2 interpolation of M points: from LDS tiles (3D, 2D, wide
+    // FP64 3D), else gathered from the grid, in bin order or (few points) in
+    // the points' own; Direct2 gathers unsorted points with the 2D tiles'
+    // sums, so a batch takes its 2D plans' small sets through the tiles.
+    enum class Interp { Unsorted, Direct2, Gather, Tiled3, Wide3, Tiled2 };
+    static bool unsorted(Interp k) { return k == Interp::Unsorted || k == Interp::Direct2; }
+    Interp interp_kind(int64_t M) const;
     const void *points = nullptr;
     int64_t point_count = 0;
     bool points_set = false;
+    Interp binned_interp = Interp::Gather;  // type 2: of the points set
     GridParams gp{};
     int geometry_index = 0;
 
@@ -156,6 +164,7 @@ struct Plan {
     // timed region without synchronizing inside it
     struct TimingSlot {
         hipEvent_t ev[2 * kStageCount] = {};
+        int begin[kStageCount] = {};  // event that begins each stage used
         bool used[kStageCount] = {};
     };
     std::vector<TimingSlot> slots;
@@ -188,6 +197,7 @@ struct Plan {
     // run = false: create the plans and the scratch only
     bool fft_nd(int64_t vectors, void *data, hipStream_t stream, bool run);
     void mark(int stage, bool end, hipStream_t stream);
+    void mark_between(int done, int next, hipStream_t stream);
     void reset_marks();
 
     bool set_points(int64_t M, const void *pts, hipStream_t stream);
