@@ -28,6 +28,7 @@ namespace {
 
 constexpr int kThreads = 512;
 constexpr int kMaxGroupLines = 128;
+constexpr int kMaxRowWords = 4864 / 32;  // bits of the longest axis
 
 // Dynamic LDS per workgroup: lines + twiddles, at most 80 KB (two
 // workgroups per CU) where the device allows it, else 64 KB; the static
@@ -339,9 +340,10 @@ __device__ __forceinline__ void dft(Cx<T> *u)
 // deconvolution factors (type 2: the u and v axes' 1/phi_hat; type 1: their
 // product in axis order).
 struct LineData {
-    int64_t *base, *mrow;
-    double *f1, *f2;
-    void *modes;  // this vector's modes (IO != 0)
+    int64_t *base, *mrow = nullptr;
+    double *f1 = nullptr, *f2 = nullptr;
+    void *modes = nullptr;  // this vector's modes (IO 1, 2)
+    uint32_t *rows = nullptr;  // the elements to write, as bits (IO 3)
 };
 
 // Mode storage index of signed frequency m on an axis of N modes.
@@ -373,7 +375,8 @@ __device__ __forceinline__ void for_kept(const LineFftKept &m, int i, int nb, in
 
 // IO (the launch's mode reads or writes): 0 grid only; 1 the first pass
 // reads the modes and predeconvolves them (type 2); 2 the last pass writes
-// the deconvolved modes (type 1).
+// the deconvolved modes (type 1); 3 the last pass writes the elements whose
+// bit is set (a sparse type 2, whose points reach few cells).
 //
 // What bounds the passes: HBM for FP32 (512^3, 4 vectors: x 1.55 ms, y 0.75
 // ms, 4.1 and 4.3 TB/s where a copy reaches 4.6), HBM latency on the short
@@ -555,6 +558,10 @@ __device__ __forceinline__ void pass_out(const Cx<T> *X, const Cx<T> *tw, const 
         } else {
             Cx<T> *out = grid + bc + (int64_t)i * P.estride;
             for_kept<R>(P.out, i, nb, n, P.out_hi, P.out_lo, [&](int t, bool in) {
+                if constexpr (IO == 3) {
+                    const int e = i + t * nb;
+                    in = in && ((ld.rows[e >> 5] >> (e & 31)) & 1u);
+                }
                 if (in) out[t * tstep] = u[t];
             });
         }
@@ -585,7 +592,7 @@ __device__ __forceinline__ void fft_lines_body(const LineFftAxis &P, Cx<T> *__re
             const int64_t uu = u < P.u_hi ? u : u + P.u_gap;
             const int64_t vv = w < P.v_hi ? w : w + P.v_gap;
             b = uu * P.su + vv * P.sv;
-            if constexpr (IO != 0) {
+            if constexpr (IO == 1 || IO == 2) {
                 // the line's mode row and factors (u, v: fine indices of the
                 // kept windows of their axes)
                 int64_t mr = 0;
@@ -628,7 +635,7 @@ __device__ __forceinline__ void fft_lines_body(const LineFftAxis &P, Cx<T> *__re
 #undef MNUFFT_MID
     }
 #define MNUFFT_OUT(R)                                             \
-    case R: pass_out<T, R, IO == 2 ? 2 : 0>(X, tw, P, P.pass[last], grid, ld); break;
+    case R: pass_out<T, R, IO == 1 ? 0 : IO>(X, tw, P, P.pass[last], grid, ld); break;
     switch (P.pass[last].radix) { MNUFFT_RADICES(MNUFFT_OUT) MNUFFT_OUT(1) }
 #undef MNUFFT_OUT
 }
@@ -647,18 +654,24 @@ __device__ inline int64_t xcd_group(uint32_t block, uint32_t blocks)
 template <typename T, int IO>
 __global__ __launch_bounds__(kThreads, 4) void k_fft_lines(const LineFftAxis *__restrict__ ax,
                                                            void *modes_all, T *__restrict__ data,
-                                                           const Cx<T> *__restrict__ tw_global)
+                                                           const Cx<T> *__restrict__ tw_global,
+                                                           const uint32_t *__restrict__ rows_all)
 {
     const LineFftAxis &P = *ax;
     extern __shared__ __align__(16) unsigned char lds_raw[];
     Cx<T> *grid = (Cx<T> *)data + (int64_t)blockIdx.y * P.vec_stride;
     const int64_t group = P.line_major ? (int64_t)blockIdx.x : xcd_group(blockIdx.x, gridDim.x);
+    __shared__ int64_t base[kMaxGroupLines];
     if constexpr (IO == 0) {
-        __shared__ int64_t base[kMaxGroupLines];
-        fft_lines_body<T, 0>(P, grid, tw_global, group, (Cx<T> *)lds_raw,
-                             LineData{base, nullptr, nullptr, nullptr, nullptr});
+        fft_lines_body<T, 0>(P, grid, tw_global, group, (Cx<T> *)lds_raw, LineData{base});
+    } else if constexpr (IO == 3) {
+        __shared__ uint32_t rows[kMaxRowWords];
+        const int words = (P.n + 31) / 32;
+        for (int w = threadIdx.x; w < words; w += kThreads) rows[w] = rows_all[group * words + w];
+        fft_lines_body<T, 3>(P, grid, tw_global, group, (Cx<T> *)lds_raw,
+                             LineData{base, nullptr, nullptr, nullptr, nullptr, rows});
     } else {
-        __shared__ int64_t base[kMaxGroupLines], mrow[kMaxGroupLines];
+        __shared__ int64_t mrow[kMaxGroupLines];
         __shared__ double f1[kMaxGroupLines], f2[kMaxGroupLines];
         Cx<T> *modes = (Cx<T> *)modes_all + (int64_t)blockIdx.y * P.mode_total;
         fft_lines_body<T, IO>(P, grid, tw_global, group, (Cx<T> *)lds_raw,
@@ -686,7 +699,7 @@ __global__ __launch_bounds__(kThreads, 4) void k_fft_lines_many(const LineFftJob
     // the job is the workgroup's: its fields in scalar registers
     const LineFftJob &J = jobs[__builtin_amdgcn_readfirstlane(lo)];
     fft_lines_body<T, 0>(*J.ax, (Cx<T> *)J.grid, (const Cx<T> *)J.tw, b - J.group0,
-                         (Cx<T> *)lds_raw, LineData{base, nullptr, nullptr, nullptr, nullptr});
+                         (Cx<T> *)lds_raw, LineData{base});
 }
 
 // Radix plan: the fewest passes of radix 2 .. 16 (each costs an LDS round
@@ -757,8 +770,9 @@ bool wide_lds()
     std::call_once(once, [] {
         const void *kernels[] = {
             (const void *)k_fft_lines<float, 0>,  (const void *)k_fft_lines<float, 1>,
-            (const void *)k_fft_lines<float, 2>,  (const void *)k_fft_lines<double, 0>,
-            (const void *)k_fft_lines<double, 1>, (const void *)k_fft_lines<double, 2>,
+            (const void *)k_fft_lines<float, 2>,  (const void *)k_fft_lines<float, 3>,
+            (const void *)k_fft_lines<double, 0>, (const void *)k_fft_lines<double, 1>,
+            (const void *)k_fft_lines<double, 2>, (const void *)k_fft_lines<double, 3>,
             (const void *)k_fft_lines_many<float>, (const void *)k_fft_lines_many<double>};
         ok = true;
         for (const void *k : kernels)
@@ -1056,19 +1070,22 @@ namespace {
 
 template <typename T>
 void launch_axis(int io, dim3 g, size_t lds, hipStream_t stream, const LineFftAxis *ax, void *mv,
-                 T *d, const Cx<T> *t)
+                 T *d, const Cx<T> *t, const uint32_t *rows)
 {
     if (io == 1)
-        k_fft_lines<T, 1><<<g, kThreads, lds, stream>>>(ax, mv, d, t);
+        k_fft_lines<T, 1><<<g, kThreads, lds, stream>>>(ax, mv, d, t, rows);
     else if (io == 2)
-        k_fft_lines<T, 2><<<g, kThreads, lds, stream>>>(ax, mv, d, t);
+        k_fft_lines<T, 2><<<g, kThreads, lds, stream>>>(ax, mv, d, t, rows);
+    else if (io == 3)
+        k_fft_lines<T, 3><<<g, kThreads, lds, stream>>>(ax, mv, d, t, rows);
     else
-        k_fft_lines<T, 0><<<g, kThreads, lds, stream>>>(ax, mv, d, t);
+        k_fft_lines<T, 0><<<g, kThreads, lds, stream>>>(ax, mv, d, t, rows);
 }
 
 }  // namespace
 
-bool LineFft::run(void *data, int64_t vectors, hipStream_t stream, void *modes) const
+bool LineFft::run(void *data, int64_t vectors, hipStream_t stream, void *modes,
+                  const uint32_t *rows) const
 {
     if (vectors <= 0) return true;
     const size_t eb = f64_ ? 16 : 8;
@@ -1077,7 +1094,7 @@ bool LineFft::run(void *data, int64_t vectors, hipStream_t stream, void *modes) 
         for (int a = 0; a < naxes_; ++a) {
             const LineFftAxis &x = ax_[a];
             const bool io = modes && a == (type_ == 2 ? 0 : naxes_ - 1);
-            const int mode_io = io ? (type_ == 2 ? 1 : 2) : 0;
+            const int mode_io = io ? (type_ == 2 ? 1 : 2) : (rows && a == 2 ? 3 : 0);
             void *mv = io ? (void *)((char *)modes + (size_t)v0 * (size_t)x.mode_total * eb)
                           : nullptr;
             const int64_t groups = (x.nu * x.nv + x.lines - 1) / x.lines;
@@ -1088,11 +1105,11 @@ bool LineFft::run(void *data, int64_t vectors, hipStream_t stream, void *modes) 
             if (f64_) {
                 double *d = (double *)data + 2 * v0 * fine_total_;
                 launch_axis<double>(mode_io, g, lds, stream, hx, mv, d,
-                                    (const Cx<double> *)tw_[a]);
+                                    (const Cx<double> *)tw_[a], rows);
             } else {
                 float *d = (float *)data + 2 * v0 * fine_total_;
                 launch_axis<float>(mode_io, g, lds, stream, hx, mv, d,
-                                   (const Cx<float> *)tw_[a]);
+                                   (const Cx<float> *)tw_[a], rows);
             }
         }
     }

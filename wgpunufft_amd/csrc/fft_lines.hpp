@@ -98,7 +98,18 @@ public:
     // With `modes`: type 2 reads the modes (vectors x mode_total) and scales
     // them as the predeconvolution does, type 1 writes the deconvolved modes;
     // the results equal predeconvolution + FFT (+ deconvolution) bit for bit.
-    bool run(void *data, int64_t vectors, hipStream_t stream, void *modes = nullptr) const;
+    // With `rows` (3D type 2; rows_words() 32-bit words for each of
+    // rows_groups() groups of adjacent columns): the last pass writes only the
+    // cells whose bit (column group, z) is set, and leaves the others as they
+    // were.
+    bool run(void *data, int64_t vectors, hipStream_t stream, void *modes = nullptr,
+             const uint32_t *rows = nullptr) const;
+    int rows_lines() const { return ax_[2].lines; }
+    int rows_words() const { return (ax_[2].n + 31) / 32; }
+    int64_t rows_groups() const
+    {
+        return (ax_[2].nu * ax_[2].nv + ax_[2].lines - 1) / ax_[2].lines;
+    }
     // One vector of each of many plans (one rank and precision): every axis
     // pass of all of them in one launch.  The job table
     // (*jobs, *cap entries) grows as needed and is filled by kernel launches

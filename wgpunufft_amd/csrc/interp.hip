@@ -895,6 +895,61 @@ bool launch_tiled_w(int64_t M, int64_t vectors, const uint32_t *sorted, const ui
     return false;
 }
 
+__global__ __launch_bounds__(256) void k_clear_bits(uint32_t *__restrict__ bits, int64_t n)
+{
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256)
+        bits[i] = 0u;
+}
+
+// The rows that the points' supports read (mark_rows): 16 lanes a point, lane
+// j the support's row y + j.  Integer ORs, so the marks do not depend on
+// their order.
+template <typename T>
+__global__ __launch_bounds__(256) void k_mark_rows(int64_t M, const T *__restrict__ coords,
+                                                   GridParams g, int lines, int words,
+                                                   uint32_t *__restrict__ bits)
+{
+    const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int64_t p = t >> 4;
+    const int j = (int)(t & 15);
+    if (p >= M || j >= g.width) return;
+    T x[3];
+#pragma unroll
+    for (int a = 0; a < 3; ++a) x[a] = coords[p * 3 + a];
+    const bool reach = FoldTraits<T>::in_reach(x[0]) && FoldTraits<T>::in_reach(x[1]) &&
+                       FoldTraits<T>::in_reach(x[2]);
+    int64_t st[3];
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        int64_t start;
+        double off;
+        support_start<T>(x[a], reach, g, a, &start, &off);
+        st[a] = wrapped_start(start, g.ax[a].n);
+    }
+    const int64_t n0 = g.ax[0].n, n2 = g.ax[2].n;
+    const int w = g.width;
+    const int64_t row = n0 * wrap_idx(st[1] + j, g.ax[1].n);
+    // the row's columns: [x, x + w), cut where it wraps
+    const int64_t x1 = st[0] + w - 1;
+    for (int part = 0; part < 2; ++part) {
+        if (part && x1 < n0) break;
+        const int64_t c0 = row + (part ? 0 : st[0]), c1 = row + (part ? x1 - n0 : (x1 < n0 ? x1 : n0 - 1));
+        for (int64_t gr = c0 / lines; gr <= c1 / lines; ++gr) {
+            uint32_t *b = bits + gr * words;
+            for (int64_t z = st[2], left = w; left > 0;) {
+                const int64_t zz = z >= n2 ? z - n2 : z;
+                const int at = (int)(zz & 31);
+                int64_t run = 32 - at < left ? 32 - at : left;
+                if (zz + run > n2) run = n2 - zz;
+                const uint32_t m = run == 32 ? 0xffffffffu : ((1u << run) - 1u) << at;
+                atomicOr(b + (zz >> 5), m);
+                z += run;
+                left -= run;
+            }
+        }
+    }
+}
+
 template <int D, typename T, int G>
 bool launch(int64_t M, int64_t vectors, const uint32_t *sorted, const T *coords,
             const GridParams &g, const T *grid, T *out, hipStream_t stream)
@@ -906,6 +961,22 @@ bool launch(int64_t M, int64_t vectors, const uint32_t *sorted, const T *coords,
 }
 
 }  // namespace
+
+template <typename T>
+bool mark_rows(int64_t M, const T *coords, const GridParams &g, int lines, int words,
+               int64_t groups, uint32_t *bits, hipStream_t stream)
+{
+    const int64_t n = groups * words;
+    k_clear_bits<<<(unsigned)std::min<int64_t>((n + 255) / 256, 8192), 256, 0, stream>>>(bits, n);
+    if (M > 0)
+        k_mark_rows<T><<<(unsigned)((M * 16 + 255) / 256), 256, 0, stream>>>(M, coords, g, lines,
+                                                                             words, bits);
+    return hip_ok(hipGetLastError(), "interpolation row marks launch");
+}
+template bool mark_rows<float>(int64_t, const float *, const GridParams &, int, int, int64_t,
+                               uint32_t *, hipStream_t);
+template bool mark_rows<double>(int64_t, const double *, const GridParams &, int, int, int64_t,
+                                uint32_t *, hipStream_t);
 
 template <int D, typename T>
 bool interpolate(int64_t M, int64_t vectors, const uint32_t *sorted, const T *coords,

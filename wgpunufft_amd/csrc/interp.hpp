@@ -12,6 +12,13 @@ template <int D, typename T>
 bool interpolate(int64_t M, int64_t vectors, const uint32_t *sorted, const T *coords,
                  const GridParams &g, const T *grid, T *out, hipStream_t stream);
 
+// Clears `bits` (groups x words) and sets, for every point, the bits of the
+// rows its support reads in 3D: bit z % 32 of word z / 32 of the group of
+// `lines` adjacent columns (x + n0 y) / lines.
+template <typename T>
+bool mark_rows(int64_t M, const T *coords, const GridParams &g, int lines, int words,
+               int64_t groups, uint32_t *bits, hipStream_t stream);
+
 // One launch for many problems (1D/2D): problem p's points, at slots
 // [m_off, m_off + M) of `sorted` (indices of the concatenated point set),
 // are interpolated from its grid into its output, in work items of
