@@ -423,6 +423,7 @@ template <typename T, int R, int IO>
 __device__ __forceinline__ void pass_in(Cx<T> *X, const LineFftAxis &P, const LineFftPass &ps,
                                         const Cx<T> *__restrict__ grid, const LineData &ld)
 {
+    const int threads = (int)blockDim.x;
     const int n = P.n, nb = ps.nb, total = P.lines * nb;
     const int ks = P.line_major ? 1 : P.lines, cs = P.line_major ? n : 1;
     const int64_t tstep = (int64_t)nb * P.estride;  // elements between a butterfly's
@@ -430,7 +431,7 @@ __device__ __forceinline__ void pass_in(Cx<T> *X, const LineFftAxis &P, const Li
     // its high end
     const int half = P.centered ? (int)(P.eN / 2) : 0;
     const int back = P.centered ? half - n : (int)P.eN - n;
-    for (int b = (int)threadIdx.x; b < total; b += kThreads) {
+    for (int b = (int)threadIdx.x; b < total; b += threads) {
         int c, i;
         butterfly<T>(P, ps, b, &c, &i);
         Cx<T> u[R];
@@ -473,6 +474,9 @@ __device__ __forceinline__ void pass_in(Cx<T> *X, const LineFftAxis &P, const Li
     __syncthreads();
 }
 
+// (MAXB butterflies a thread cover the largest group at kThreads threads; a
+// smaller workgroup has a thread for every butterfly of every pass.)
+//
 // A middle pass, in place in LDS: every thread reads its butterflies into
 // registers, the workgroup waits, every thread writes them.
 template <typename T, int R>
@@ -480,6 +484,7 @@ __device__ __forceinline__ void pass_mid(Cx<T> *X, const Cx<T> *tw, const LineFf
                                          const LineFftPass &ps)
 {
     constexpr int MAXB = (LdsElems<T>::group / R + kThreads - 1) / kThreads;
+    const int threads = (int)blockDim.x;
     const int n = P.n, nb = ps.nb, total = P.lines * nb;
     const int ks = P.line_major ? 1 : P.lines, cs = P.line_major ? n : 1;
     const int in_step = nb * ks, out_step = ps.p * ks;
@@ -487,7 +492,7 @@ __device__ __forceinline__ void pass_mid(Cx<T> *X, const Cx<T> *tw, const LineFf
     int at[MAXB];
 #pragma unroll
     for (int s = 0; s < MAXB; ++s) {
-        const int b = (int)threadIdx.x + s * kThreads;
+        const int b = (int)threadIdx.x + s * threads;
         at[s] = -1;
         if (b < total) {
             int c, i, q, k;
@@ -519,13 +524,14 @@ __device__ __forceinline__ void pass_out(const Cx<T> *X, const Cx<T> *tw, const 
                                          const LineFftPass &ps, Cx<T> *__restrict__ grid,
                                          const LineData &ld)
 {
+    const int threads = (int)blockDim.x;
     const int n = P.n, nb = ps.nb, total = P.lines * nb;
     const int ks = P.line_major ? 1 : P.lines, cs = P.line_major ? n : 1;
     const int in_step = nb * ks;
     const int64_t tstep = (int64_t)nb * P.estride;
     const int half = P.centered ? (int)(P.eN / 2) : 0;
     const int back = P.centered ? half - n : (int)P.eN - n;
-    for (int b = (int)threadIdx.x; b < total; b += kThreads) {
+    for (int b = (int)threadIdx.x; b < total; b += threads) {
         int c, i;
         butterfly<T>(P, ps, b, &c, &i);
         const int64_t bc = ld.base[c];
@@ -580,11 +586,11 @@ __device__ __forceinline__ void fft_lines_body(const LineFftAxis &P, Cx<T> *__re
     int64_t *base = ld.base;
     Cx<T> *tw = X + P.lines * P.n;
     const int n = P.n;
-    for (int m = threadIdx.x; m < n; m += kThreads) tw[m] = tw_global[m];
+    for (int m = threadIdx.x; m < n; m += (int)blockDim.x) tw[m] = tw_global[m];
     // (line numbers are below 2^32: at most 65536 per axis)
     const uint32_t nu = (uint32_t)P.nu, nlines = (uint32_t)(P.nu * P.nv);
     const uint32_t line0 = (uint32_t)group * (uint32_t)P.lines;
-    for (int c = threadIdx.x; c < P.lines; c += kThreads) {
+    for (int c = threadIdx.x; c < P.lines; c += (int)blockDim.x) {
         const uint32_t L = line0 + (uint32_t)c;
         int64_t b = -1;
         if (L < nlines) {
@@ -667,7 +673,7 @@ __global__ __launch_bounds__(kThreads, 4) void k_fft_lines(const LineFftAxis *__
     } else if constexpr (IO == 3) {
         __shared__ uint32_t rows[kMaxRowWords];
         const int words = (P.n + 31) / 32;
-        for (int w = threadIdx.x; w < words; w += kThreads) rows[w] = rows_all[group * words + w];
+        for (int w = threadIdx.x; w < words; w += (int)blockDim.x) rows[w] = rows_all[group * words + w];
         fft_lines_body<T, 3>(P, grid, tw_global, group, (Cx<T> *)lds_raw,
                              LineData{base, nullptr, nullptr, nullptr, nullptr, rows});
     } else {
@@ -804,6 +810,17 @@ bool group_lines(int n, bool line_major, bool f64, int64_t count, bool wide, Lin
         ax->log_lines = 0;
         while ((1 << ax->log_lines) < c) ++ax->log_lines;
     }
+    // a thread for every butterfly of the pass with most of them, at most
+    // kThreads, rounded up to whole waves for every SIMD of the CU (7 waves
+    // ran 900-cell passes 9% slower than 8).  512 threads for every axis left
+    // most waves of short ones idle and fewer workgroups on a CU: 256^3 FP32
+    // type 2 x / y / z 44 / 28 / 50 -> 27 / 22 / 37 us, 162 x 128 x 100 FP64
+    // 18 / 15 / 28 -> 18 / 11 / 15 us.
+    int most_butterflies = 1;
+    for (int i = 0; i < ax->npass; ++i)
+        most_butterflies = std::max(most_butterflies, ax->lines * ax->pass[i].nb);
+    ax->threads = 64;
+    while (ax->threads < kThreads && ax->threads < most_butterflies) ax->threads *= 2;
     return ax->lines >= 1;
 }
 
@@ -1020,11 +1037,12 @@ bool LineFft::run_many(const std::vector<const LineFft *> &ffts, const std::vect
         size_t first, count;
         int64_t groups;
         size_t lds;
+        int threads;
     };
     std::vector<LineFftJob> all;
     std::vector<Launch> launches;
     for (int a = 0; a < naxes; ++a) {
-        Launch L{all.size(), 0, 0, 0};
+        Launch L{all.size(), 0, 0, 0, 64};
         for (size_t i = 0; i < ffts.size(); ++i) {
             const LineFft &f = *ffts[i];
             const LineFftAxis &x = f.ax_[a];
@@ -1032,6 +1050,7 @@ bool LineFft::run_many(const std::vector<const LineFft *> &ffts, const std::vect
             if (g == 0) continue;
             all.push_back(LineFftJob{f.dev_ax_ + a, grids[i], f.tw_[a], L.groups});
             L.groups += g;
+            L.threads = std::max(L.threads, x.threads);
             L.lds = std::max(L.lds, (size_t)(x.lines + 1) * (size_t)x.n * (f64 ? 16 : 8));
         }
         L.count = all.size() - L.first;
@@ -1059,9 +1078,9 @@ bool LineFft::run_many(const std::vector<const LineFft *> &ffts, const std::vect
         const dim3 g((unsigned)L.groups);
         const LineFftJob *J = *jobs + L.first;
         if (f64)
-            k_fft_lines_many<double><<<g, kThreads, L.lds, stream>>>(J, (int)L.count);
+            k_fft_lines_many<double><<<g, L.threads, L.lds, stream>>>(J, (int)L.count);
         else
-            k_fft_lines_many<float><<<g, kThreads, L.lds, stream>>>(J, (int)L.count);
+            k_fft_lines_many<float><<<g, L.threads, L.lds, stream>>>(J, (int)L.count);
     }
     return hip_ok(hipGetLastError(), "batched line FFT launch");
 }
@@ -1069,17 +1088,17 @@ bool LineFft::run_many(const std::vector<const LineFft *> &ffts, const std::vect
 namespace {
 
 template <typename T>
-void launch_axis(int io, dim3 g, size_t lds, hipStream_t stream, const LineFftAxis *ax, void *mv,
+void launch_axis(int io, dim3 g, int threads, size_t lds, hipStream_t stream, const LineFftAxis *ax, void *mv,
                  T *d, const Cx<T> *t, const uint32_t *rows)
 {
     if (io == 1)
-        k_fft_lines<T, 1><<<g, kThreads, lds, stream>>>(ax, mv, d, t, rows);
+        k_fft_lines<T, 1><<<g, threads, lds, stream>>>(ax, mv, d, t, rows);
     else if (io == 2)
-        k_fft_lines<T, 2><<<g, kThreads, lds, stream>>>(ax, mv, d, t, rows);
+        k_fft_lines<T, 2><<<g, threads, lds, stream>>>(ax, mv, d, t, rows);
     else if (io == 3)
-        k_fft_lines<T, 3><<<g, kThreads, lds, stream>>>(ax, mv, d, t, rows);
+        k_fft_lines<T, 3><<<g, threads, lds, stream>>>(ax, mv, d, t, rows);
     else
-        k_fft_lines<T, 0><<<g, kThreads, lds, stream>>>(ax, mv, d, t, rows);
+        k_fft_lines<T, 0><<<g, threads, lds, stream>>>(ax, mv, d, t, rows);
 }
 
 }  // namespace
@@ -1104,11 +1123,11 @@ bool LineFft::run(void *data, int64_t vectors, hipStream_t stream, void *modes,
             const LineFftAxis *hx = dev_ax_ + a;
             if (f64_) {
                 double *d = (double *)data + 2 * v0 * fine_total_;
-                launch_axis<double>(mode_io, g, lds, stream, hx, mv, d,
+                launch_axis<double>(mode_io, g, x.threads, lds, stream, hx, mv, d,
                                     (const Cx<double> *)tw_[a], rows);
             } else {
                 float *d = (float *)data + 2 * v0 * fine_total_;
-                launch_axis<float>(mode_io, g, lds, stream, hx, mv, d,
+                launch_axis<float>(mode_io, g, x.threads, lds, stream, hx, mv, d,
                                    (const Cx<float> *)tw_[a], rows);
             }
         }

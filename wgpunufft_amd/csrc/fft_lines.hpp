@@ -53,6 +53,7 @@ struct LineFftAxis {
     int n = 1, npass = 0;
     LineFftPass pass[kLineFftMaxPasses] = {};
     int lines = 1, log_lines = 0;
+    int threads = 64;  // of a workgroup
     int line_major = 0;  // the axis is the contiguous one
     int exchange = 0;    // real and imaginary parts exchanged in and out (isign < 0)
     int64_t estride = 1;
