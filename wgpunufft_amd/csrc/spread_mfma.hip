@@ -132,15 +132,15 @@ k_spread_mfma3(
     strength_scale(cmax + blockIdx.y, &scale, &unscale);
 
     const int64_t v = blockIdx.y;
-    const float two_over_w = 2.0f / (float)W;
-    const float beta_l2e = (float)(g.beta * 1.4426950408889634);
+    const UniformPtr<float> panels = panel_coefficients<float>(g);
     const int64_t n_items = ctrl[0];
     const uint32_t part_len_cap = ctrl[3];
     const float *cv = c_sorted + 2 * v * M;
     const int64_t n0 = g.ax[0].n, n1 = g.ax[1].n, n2 = g.ax[2].n;
 
     for (int64_t item = blockIdx.x; item < n_items; item += gridDim.x) {
-        const TileItem ti = tile_item(item, sp.block_count, item_off, parts, totals, part_len_cap);
+        const TileItem ti = tile_item(item, sp.block_count, item_off, parts, totals, part_len_cap,
+                                      n_items);
         const int64_t b = ti.b, p = ti.p, rlo = ti.rlo, rhi = ti.rhi;
         const uint32_t np = ti.np;
         const int64_t tbx = b % sp.nblocks[0];
@@ -201,12 +201,11 @@ k_spread_mfma3(
                         const float o = axis == 0 ? S.ox : (axis == 1 ? S.oy : S.oz);
                         float *tb = axis == 0 ? KX : (axis == 1 ? KY : KZ);
                         const unsigned lim = axis == 2 ? TZ : kTile;
-#pragma unroll
-                        for (int t = 0; t < W; ++t) {
+es_axis_weights<float, W>(o, (float)g.beta, panels, [&](int t, float wt) {
                             const unsigned c = (unsigned)(s + t);
                             const unsigned row = c < lim ? c : (unsigned)kTile;
-                            tb[row * kPitch + j] = es_weight_fast((float)t + o, two_over_w, beta_l2e);
-                        }
+                            tb[row * kPitch + j] = wt;
+                        });
                     }
                 } else {
                     const int j = lane - 48;
@@ -312,7 +311,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_
     const int64_t n0 = g.ax[0].n, n1 = g.ax[1].n;
 
     for (int64_t item = blockIdx.x; item < n_items; item += gridDim.x) {
-        const TileItem ti = tile_item(item, sp.block_count, item_off, parts, totals, part_len_cap);
+        const TileItem ti = tile_item(item, sp.block_count, item_off, parts, totals, part_len_cap,
+                                      n_items);
         const int64_t b = ti.b;
         const int64_t x0 = (b % sp.nblocks[0]) * kTile2, y0 = (b / sp.nblocks[0]) * kTile2;
         const AxisReach rx = axis_reach(x0, kTile2, W, g.ax[0]);

@@ -238,7 +238,8 @@ __global__ __launch_bounds__(64, sizeof(T) == 4 ? 4 : 2) void k_spread_rows(
     const T *cv = c_sorted + 2 * v * M;
 
     for (int64_t item = blockIdx.x; item < n_items; item += gridDim.x) {
-        const TileItem ti = tile_item(item, sp.block_count, item_off, parts, totals, part_len_cap);
+        const TileItem ti = tile_item(item, sp.block_count, item_off, parts, totals, part_len_cap,
+                                      n_items);
         const int64_t b = ti.b;
         const int64_t x0 = (b % sp.nblocks[0]) * TX;
         const int64_t y0 = ((b / sp.nblocks[0]) % sp.nblocks[1]) * TY;
@@ -281,7 +282,7 @@ __global__ __launch_bounds__(64, sizeof(T) == 4 ? 4 : 2) void k_spread_rows3_man
         const SpreadProblem &spb = sprobs[q];
         const int64_t bb = spb.block_base;
         const TileItem ti = tile_item(item - pbase[4 * q], spb.sp.block_count, item_off + bb,
-                                      parts + bb, totals + bb, pctrl[8 * q + 3]);
+                                      parts + bb, totals + bb, pctrl[8 * q + 3], pctrl[8 * q]);
         const int64_t b = ti.b;
         const int64_t nb0 = spb.sp.nblocks[0], nb1 = spb.sp.nblocks[1];
         const int64_t x0 = (b % nb0) * TX, y0 = ((b / nb0) % nb1) * TY, z0 = (b / (nb0 * nb1)) * TZ;
@@ -443,7 +444,8 @@ __global__ __launch_bounds__(64, sizeof(T) == 4 ? 4 : 2) void k_spread_rows2(
     const T *cv = c_sorted + 2 * v * M;
 
     for (int64_t item = blockIdx.x; item < n_items; item += gridDim.x) {
-        const TileItem ti = tile_item(item, sp.block_count, item_off, parts, totals, part_len_cap);
+        const TileItem ti = tile_item(item, sp.block_count, item_off, parts, totals, part_len_cap,
+                                      n_items);
         const int64_t b = ti.b;
         const int64_t x0 = (b % sp.nblocks[0]) * kRows2T, y0 = (b / sp.nblocks[0]) * kRows2T;
         typename mfma::ExactMma<T>::Acc acc[2];
@@ -484,7 +486,7 @@ __global__ __launch_bounds__(64, sizeof(T) == 4 ? 4 : 2) void k_spread_rows2_man
         const SpreadProblem &spb = sprobs[q];
         const int64_t bb = spb.block_base;
         const TileItem ti = tile_item(item - pbase[4 * q], spb.sp.block_count, item_off + bb,
-                                      parts + bb, totals + bb, pctrl[8 * q + 3]);
+                                      parts + bb, totals + bb, pctrl[8 * q + 3], pctrl[8 * q]);
         const int64_t b = ti.b;
         const int64_t x0 = (b % spb.sp.nblocks[0]) * kRows2T;
         const int64_t y0 = (b / spb.sp.nblocks[0]) * kRows2T;
