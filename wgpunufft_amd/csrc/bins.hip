@@ -889,18 +889,22 @@ __device__ inline int64_t bin_of_starts(const int *st, const GridParams &g)
 }
 
 // Record s of rank D (layout of rec_quads<D>): starts and offsets of every
-// axis; ranks 1-3 keep the point index in the fourth start word.
+// axis; ranks 1-3 keep the point index in the fourth start word, and the x
+// start again in the fourth offset word (record_start_x): the row tiles know
+// a record's other starts from its reach row, so they read only the offsets
+// and, where nothing else reads the starts, rec_start is null.
 template <int D, typename T>
 __device__ inline void store_record(int4 *__restrict__ rec_start, T *__restrict__ rec_off,
                                     int64_t s, const int *st, const T *off, uint32_t idx)
 {
     if constexpr (D <= 3) {
-        rec_start[s] = make_int4(st[0], st[1], st[2], (int)idx);
+        if (rec_start) rec_start[s] = make_int4(st[0], st[1], st[2], (int)idx);
         if constexpr (sizeof(T) == 4) {
-            *(float4 *)(rec_off + s * 4) = make_float4(off[0], off[1], off[2], off[3]);
+            *(float4 *)(rec_off + s * 4) =
+                make_float4(off[0], off[1], off[2], __int_as_float(st[0]));
         } else {
             *(double2 *)(rec_off + s * 4) = make_double2(off[0], off[1]);
-            *(double2 *)(rec_off + s * 4 + 2) = make_double2(off[2], off[3]);
+            *(double2 *)(rec_off + s * 4 + 2) = make_double2(off[2], (double)st[0]);
         }
     } else {
         rec_start[2 * s] = make_int4(st[0], st[1], st[2], st[3]);

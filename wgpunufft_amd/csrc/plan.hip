@@ -695,7 +695,9 @@ bool Plan::set_points_t(int64_t M, const T *pts, hipStream_t stream)
         mark_between(kStageSort, kStagePrepare, stream);
         if (binned_dense && !dense.classify(gp, spread_params(), sorter.offsets(), stream))
             return false;
-        if (!sorter.prepare<D, T>(M, pts, gp, point_order, rec_start, (T *)rec_off, rec_perm,
+        // the row tiles read no starts; the blocks and the dense windows do
+        int4 *starts = gp_rows && !binned_dense ? nullptr : rec_start;
+        if (!sorter.prepare<D, T>(M, pts, gp, point_order, starts, (T *)rec_off, rec_perm,
                                   stream, binned_dense ? dense.before : nullptr))
             return false;
         mark(kStagePrepare, true, stream);
@@ -1547,10 +1549,13 @@ bool execute_type1_many_t(int64_t count, Plan *const *plans, const int64_t *M,
     if (m_off > 0) {
         if (!head.batch_sorter) head.batch_sorter = std::make_unique<BinSorter>();
         BinSorter &bs = *head.batch_sorter;
+        bool blocks = false;  // a class on the output-stationary blocks reads the starts
+        for (const SpreadClass &k : classes) blocks = blocks || k.run != 0;
         if (!bs.sort_many<D, T>(m_off, head.batch_table, (int)count, bins, stream) ||
             !head.ensure_records(m_off) || !head.ensure_strengths(m_off, 1) ||
             !prepare_many<D, T>(m_off, bs.sorted(), head.batch_table, (int)count,
-                                head.rec_start, (T *)head.rec_off, head.rec_perm, stream) ||
+                                blocks ? head.rec_start : nullptr, (T *)head.rec_off,
+                                head.rec_perm, stream) ||
             !gather_strengths_many<T>(m_off, head.rec_perm, head.batch_table, (int)count,
                                       (T *)head.c_sorted, stream) ||
             !head.spreader.spread_many<D, T>(head.batch_table, head.batch_spread, classes,

@@ -1058,12 +1058,12 @@ bool chunk_spread(Spreader &s, const GridParams &g, const SpreadParams &sp,
 
 template <typename T>
 bool chunk_rows(Spreader &s, const GridParams &g, const SpreadParams &sp, const uint32_t *offsets,
-                const int4 *rec_start, const T *rec_off, const T *c_sorted, int64_t M,
+                const T *rec_off, const T *c_sorted, int64_t M,
                 int64_t vectors, T *grid, hipStream_t stream)
 {
     const dim3 ig = items_grid(sp.block_count, vectors);
     TileWork w{s.totals, s.parts, s.item_off, s.heavy_base, s.ctrl, nullptr, ig.x};
-    if (!launch_rows_tiles<T>(g, sp, offsets, rec_start, rec_off, c_sorted, M, vectors, w, grid,
+    if (!launch_rows_tiles<T>(g, sp, offsets, rec_off, c_sorted, M, vectors, w, grid,
                               (T *)s.partial, stream))
         return false;
     if (s.kernel_end) (void)hipEventRecord(s.kernel_end, stream);
@@ -1081,14 +1081,14 @@ bool chunk_rows(Spreader &s, const GridParams &g, const SpreadParams &sp, const 
 
 template <int D>
 bool chunk_mfma(Spreader &s, SpreadMethod method, const GridParams &g, const SpreadParams &sp,
-                const uint32_t *offsets, const int4 *rec_start, const float *rec_off,
+                const uint32_t *offsets, const float *rec_off,
                 const float *c_sorted, int64_t M, int64_t vectors, const uint32_t *vmax,
                 float *grid, bool mark_end, hipStream_t stream)
 {
     constexpr int TE = D == 3 ? 16 : 32;  // tile edge along x and y
     const dim3 ig = items_grid(sp.block_count, vectors);
     TileWork w{s.totals, s.parts, s.item_off, s.heavy_base, s.ctrl, vmax, ig.x};
-    if (!launch_mfma_tiles(method, D, g, sp, offsets, rec_start, rec_off, c_sorted, M, vectors, w,
+    if (!launch_mfma_tiles(method, D, g, sp, offsets, rec_off, c_sorted, M, vectors, w,
                            grid, (float *)s.partial, stream))
         return false;
     if (mark_end && s.kernel_end) (void)hipEventRecord(s.kernel_end, stream);
@@ -1251,7 +1251,7 @@ bool Spreader::spread(const GridParams &g, const SpreadParams &sp, const uint32_
                 ok = !dense || dense->spread(method, g, sp, M, rec_start, rec_off,
                                              dense->strengths + 2 * v0 * M, vmax + v0, vc, gr,
                                              false, stream);
-                ok = ok && chunk_mfma<D>(*this, method, g, sp, offsets, rec_start, rec_off, cs,
+                ok = ok && chunk_mfma<D>(*this, method, g, sp, offsets, rec_off, cs,
                                          M, vc, vmax + v0, gr, dense == nullptr, stream);
                 if (ok && dense)
                     ok = dense->spread(method, g, sp, M, rec_start, rec_off,
@@ -1261,7 +1261,7 @@ bool Spreader::spread(const GridParams &g, const SpreadParams &sp, const uint32_
             }
         } else if (tiles) {
             if constexpr (D == 2 || D == 3)
-                ok = chunk_rows<T>(*this, g, sp, offsets, rec_start, rec_off, cs, M, vc, gr,
+                ok = chunk_rows<T>(*this, g, sp, offsets, rec_off, cs, M, vc, gr,
                                    stream);
         } else {
             switch (sp.run) {
@@ -1351,14 +1351,14 @@ bool Spreader::spread_many(const BatchProblem *probs, const SpreadProblem *sprob
         switch (R) {
         case 0:
             if constexpr (D == 2) {
-                if (!launch_rows2_many<T>(k.width, pb, sb, n, ig.x, offsets, rec_start, rec_off,
+                if (!launch_rows2_many<T>(k.width, pb, sb, n, ig.x, offsets, rec_off,
                                           c_sorted, totals, parts, item_off, heavy_base, pctrl,
                                           pbase, (T *)partial, stream))
                     return false;
                 k_reduce_tiles_many<T, 16, 16, 1><<<rg, 256, 0, stream>>>(
                     pb, sb, n, parts, heavy_base, heavy_list, pbase, (const T *)partial);
             } else if constexpr (D == 3) {
-                if (!launch_rows3_many<T>(k.width, pb, sb, n, ig.x, offsets, rec_start, rec_off,
+                if (!launch_rows3_many<T>(k.width, pb, sb, n, ig.x, offsets, rec_off,
                                           c_sorted, totals, parts, item_off, heavy_base, pctrl,
                                           pbase, (T *)partial, stream))
                     return false;

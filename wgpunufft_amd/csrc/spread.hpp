@@ -161,7 +161,7 @@ struct TileWork {
 // Tile kernel of the matrix-core spread (spread_mfma.hip); partial sums of
 // heavy parts go to `partial` in the layout k_reduce_tiles reads.
 bool launch_mfma_tiles(SpreadMethod method, int dim, const GridParams &g, const SpreadParams &sp,
-                       const uint32_t *offsets, const int4 *rec_start, const float *rec_off,
+                       const uint32_t *offsets, const float *rec_off,
                        const float *c_sorted, int64_t M, int64_t vectors, const TileWork &w,
                        float *grid, float *partial, hipStream_t stream);
 
@@ -221,7 +221,7 @@ bool make_sweep_params(int d, const int64_t *fine, int width, int64_t tx, int ma
 template <typename T>
 bool launch_rows2_many(int width, const BatchProblem *probs, const SpreadProblem *sprobs,
                        int nprob, unsigned items_grid, const uint32_t *offsets,
-                       const int4 *rec_start, const T *rec_off, const T *c_sorted,
+                       const T *rec_off, const T *c_sorted,
                        const uint32_t *totals, const uint32_t *parts, const uint32_t *item_off,
                        const uint32_t *heavy_base, const uint32_t *pctrl, const int64_t *pbase,
                        T *partial, hipStream_t stream);
@@ -230,14 +230,14 @@ bool launch_rows2_many(int width, const BatchProblem *probs, const SpreadProblem
 template <typename T>
 bool launch_rows3_many(int width, const BatchProblem *probs, const SpreadProblem *sprobs,
                        int nprob, unsigned items_grid, const uint32_t *offsets,
-                       const int4 *rec_start, const T *rec_off, const T *c_sorted,
+                       const T *rec_off, const T *c_sorted,
                        const uint32_t *totals, const uint32_t *parts, const uint32_t *item_off,
                        const uint32_t *heavy_base, const uint32_t *pctrl, const int64_t *pbase,
                        T *partial, hipStream_t stream);
 
 template <typename T>
 bool launch_rows_tiles(const GridParams &g, const SpreadParams &sp, const uint32_t *offsets,
-                       const int4 *rec_start, const T *rec_off, const T *c_sorted, int64_t M,
+                       const T *rec_off, const T *c_sorted, int64_t M,
                        int64_t vectors, const TileWork &w, T *grid, T *partial,
                        hipStream_t stream);
 

@@ -99,7 +99,7 @@ template <int W, int MODE, int TZ>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void
 k_spread_mfma3(
     GridParams g, SpreadParams sp, const uint32_t *__restrict__ offsets,
-    const int4 *__restrict__ rec_start, const float *__restrict__ rec_off,
+    const float *__restrict__ rec_off,
     const float *__restrict__ c_sorted, int64_t M, const uint32_t *__restrict__ totals,
     const uint32_t *__restrict__ parts, const uint32_t *__restrict__ item_off,
     const uint32_t *__restrict__ heavy_base, const uint32_t *__restrict__ ctrl,
@@ -158,10 +158,10 @@ k_spread_mfma3(
         // records in chunks of 64, the next chunk's loads in flight while
         // the current one is contracted
         const int64_t klo = rlo, khi = rhi;
-        Fetched<float> nx = fetch_record<float, NROWS>(rows, klo + lane, khi, rec_start, rec_off, cv);
+        Fetched<float> nx = fetch_record<float, NROWS>(rows, klo + lane, khi, rec_off, cv);
         for (int64_t k0 = klo; k0 < khi; k0 += 64) {
             const Fetched<float> cur = nx;
-            nx = fetch_record<float, NROWS>(rows, k0 + 64 + lane, khi, rec_start, rec_off, cv);
+            nx = fetch_record<float, NROWS>(rows, k0 + 64 + lane, khi, rec_off, cv);
             bool take = false;
             MfmaRec R{};
             if (cur.valid) {
@@ -276,7 +276,7 @@ constexpr int kTile2 = 32;
 template <int W, int MODE>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_spread_mfma2(
     GridParams g, SpreadParams sp, const uint32_t *__restrict__ offsets,
-    const int4 *__restrict__ rec_start, const float *__restrict__ rec_off,
+    const float *__restrict__ rec_off,
     const float *__restrict__ c_sorted, int64_t M, const uint32_t *__restrict__ totals,
     const uint32_t *__restrict__ parts, const uint32_t *__restrict__ item_off,
     const uint32_t *__restrict__ heavy_base, const uint32_t *__restrict__ ctrl,
@@ -324,10 +324,10 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_
         // records in chunks of 64, the next chunk's loads in flight while
         // the current one is contracted
         const int64_t klo = ti.rlo, khi = ti.rhi;
-        Fetched<float> nx = fetch_record<float, NROWS>(rows, klo + lane, khi, rec_start, rec_off, cv);
+        Fetched<float> nx = fetch_record<float, NROWS>(rows, klo + lane, khi, rec_off, cv);
         for (int64_t k0 = klo; k0 < khi; k0 += 64) {
             const Fetched<float> cur = nx;
-            nx = fetch_record<float, NROWS>(rows, k0 + 64 + lane, khi, rec_start, rec_off, cv);
+            nx = fetch_record<float, NROWS>(rows, k0 + 64 + lane, khi, rec_off, cv);
             bool take = false;
             MfmaRec R{};
             if (cur.valid) {
@@ -419,39 +419,37 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_
 
 template <int D, int W, int MODE>
 void launch_kernel(dim3 grid3, const GridParams &g, const SpreadParams &sp,
-                   const uint32_t *offsets, const int4 *rec_start, const float *rec_off,
+                   const uint32_t *offsets, const float *rec_off,
                    const float *c_sorted, int64_t M, const TileWork &w, float *grid,
                    float *partial, hipStream_t stream)
 {
     if constexpr (D == 3)
         k_spread_mfma3<W, MODE, 8><<<grid3, 64, 0, stream>>>(
-            g, sp, offsets, rec_start, rec_off, c_sorted, M, w.totals, w.parts, w.item_off,
+            g, sp, offsets, rec_off, c_sorted, M, w.totals, w.parts, w.item_off,
             w.heavy_base, w.ctrl, w.cmax, grid, partial);
     else
         k_spread_mfma2<W, MODE><<<grid3, 64, 0, stream>>>(
-            g, sp, offsets, rec_start, rec_off, c_sorted, M, w.totals, w.parts, w.item_off,
+            g, sp, offsets, rec_off, c_sorted, M, w.totals, w.parts, w.item_off,
             w.heavy_base, w.ctrl, w.cmax, grid, partial);
 }
 
 template <int D, int W>
 bool launch_width(SpreadMethod method, dim3 grid3, const GridParams &g, const SpreadParams &sp,
-                  const uint32_t *offsets, const int4 *rec_start, const float *rec_off,
+                  const uint32_t *offsets, const float *rec_off,
                   const float *c_sorted, int64_t M, const TileWork &w, float *grid,
                   float *partial, hipStream_t stream)
 {
     switch (method) {
     case SpreadMethod::MfmaF16:
-        launch_kernel<D, W, (int)SpreadMethod::MfmaF16>(grid3, g, sp, offsets, rec_start, rec_off,
+        launch_kernel<D, W, (int)SpreadMethod::MfmaF16>(grid3, g, sp, offsets, rec_off,
                                                         c_sorted, M, w, grid, partial, stream);
         return true;
     case SpreadMethod::MfmaF16x3:
-        launch_kernel<D, W, (int)SpreadMethod::MfmaF16x3>(grid3, g, sp, offsets, rec_start,
-                                                          rec_off, c_sorted, M, w, grid, partial,
+        launch_kernel<D, W, (int)SpreadMethod::MfmaF16x3>(grid3, g, sp, offsets,                                                           rec_off, c_sorted, M, w, grid, partial,
                                                           stream);
         return true;
     case SpreadMethod::MfmaBf16x3:
-        launch_kernel<D, W, (int)SpreadMethod::MfmaBf16x3>(grid3, g, sp, offsets, rec_start,
-                                                           rec_off, c_sorted, M, w, grid, partial,
+        launch_kernel<D, W, (int)SpreadMethod::MfmaBf16x3>(grid3, g, sp, offsets,                                                            rec_off, c_sorted, M, w, grid, partial,
                                                            stream);
         return true;
     default:
@@ -461,13 +459,13 @@ bool launch_width(SpreadMethod method, dim3 grid3, const GridParams &g, const Sp
 
 template <int D>
 bool launch_dim(SpreadMethod method, dim3 grid3, const GridParams &g, const SpreadParams &sp,
-                const uint32_t *offsets, const int4 *rec_start, const float *rec_off,
+                const uint32_t *offsets, const float *rec_off,
                 const float *c_sorted, int64_t M, const TileWork &w, float *grid, float *partial,
                 hipStream_t stream)
 {
 #define MNUFFT_MFMA_WIDTH(Wd)                                                                     \
     case Wd:                                                                                      \
-        return launch_width<D, Wd>(method, grid3, g, sp, offsets, rec_start, rec_off, c_sorted,  \
+        return launch_width<D, Wd>(method, grid3, g, sp, offsets, rec_off, c_sorted,  \
                                    M, w, grid, partial, stream);
     switch (g.width) {
         MNUFFT_MFMA_WIDTH(2)
@@ -496,17 +494,17 @@ bool launch_absmax(const float *c, int64_t n, int64_t vectors, uint32_t *out,
 }
 
 bool launch_mfma_tiles(SpreadMethod method, int dim, const GridParams &g, const SpreadParams &sp,
-                       const uint32_t *offsets, const int4 *rec_start, const float *rec_off,
+                       const uint32_t *offsets, const float *rec_off,
                        const float *c_sorted, int64_t M, int64_t vectors, const TileWork &w,
                        float *grid, float *partial, hipStream_t stream)
 {
     dim3 grid3(w.items_grid, (unsigned)vectors);
     bool ok = false;
     if (dim == 3)
-        ok = launch_dim<3>(method, grid3, g, sp, offsets, rec_start, rec_off, c_sorted, M, w, grid,
+        ok = launch_dim<3>(method, grid3, g, sp, offsets, rec_off, c_sorted, M, w, grid,
                            partial, stream);
     else if (dim == 2)
-        ok = launch_dim<2>(method, grid3, g, sp, offsets, rec_start, rec_off, c_sorted, M, w, grid,
+        ok = launch_dim<2>(method, grid3, g, sp, offsets, rec_off, c_sorted, M, w, grid,
                            partial, stream);
     if (!ok) {
         set_error("matrix-core spread needs a 2D or 3D plan, a width <= 8 and an MFMA method");

@@ -107,7 +107,6 @@ __device__ __forceinline__ void rows3_accumulate(Rows3Stage<T> &st, TileRows<NRO
                                                  const GridParams &g, int64_t x0, int64_t y0,
                                                  int64_t z0, int64_t klo, int64_t khi,
                                                  const uint32_t *__restrict__ offsets,
-                                                 const int4 *__restrict__ rec_start,
                                                  const T *__restrict__ rec_off,
                                                  const T *__restrict__ cv,
                                                  typename mfma::ExactMma<T>::Acc (&acc)[4])
@@ -130,10 +129,10 @@ __device__ __forceinline__ void rows3_accumulate(Rows3Stage<T> &st, TileRows<NRO
     const int lx = (lane & 15) >> 1, lc = lane & 1;
     // records in chunks of 64, the next chunk's loads in flight while the
     // current one is added
-    Fetched<T> nx = fetch_record<T, NROWS>(rows, klo + lane, khi, rec_start, rec_off, cv);
+    Fetched<T> nx = fetch_record<T, NROWS>(rows, klo + lane, khi, rec_off, cv);
     for (int64_t k0 = klo; k0 < khi; k0 += 64) {
         const Fetched<T> cur = nx;
-        nx = fetch_record<T, NROWS>(rows, k0 + 64 + lane, khi, rec_start, rec_off, cv);
+        nx = fetch_record<T, NROWS>(rows, k0 + 64 + lane, khi, rec_off, cv);
         bool take = false;
         int ee = 0;
         if (cur.valid) {
@@ -218,7 +217,7 @@ __device__ __forceinline__ void rows3_store(int lane, const GridParams &g, int64
 template <typename T, int W>
 __global__ __launch_bounds__(64, sizeof(T) == 4 ? 4 : 2) void k_spread_rows(
     GridParams g, SpreadParams sp, const uint32_t *__restrict__ offsets,
-    const int4 *__restrict__ rec_start, const T *__restrict__ rec_off,
+    const T *__restrict__ rec_off,
     const T *__restrict__ c_sorted, int64_t M, const uint32_t *__restrict__ totals,
     const uint32_t *__restrict__ parts, const uint32_t *__restrict__ item_off,
     const uint32_t *__restrict__ heavy_base, const uint32_t *__restrict__ ctrl,
@@ -246,7 +245,7 @@ __global__ __launch_bounds__(64, sizeof(T) == 4 ? 4 : 2) void k_spread_rows(
         const int64_t z0 = (b / (sp.nblocks[0] * sp.nblocks[1])) * TZ;
         typename mfma::ExactMma<T>::Acc acc[4];
         rows3_accumulate<T, W, NROWS>(st, rows, lane, g, x0, y0, z0, ti.rlo, ti.rhi, offsets,
-                                      rec_start, rec_off, cv, acc);
+                                      rec_off, cv, acc);
         const bool whole = ti.np == 1;
         T *slot = whole ? nullptr
                         : partial + partial_index<TX, TY, TZ>((int64_t)heavy_base[b] + ti.p,
@@ -260,8 +259,7 @@ __global__ __launch_bounds__(64, sizeof(T) == 4 ? 4 : 2) void k_spread_rows(
 template <typename T, int W>
 __global__ __launch_bounds__(64, sizeof(T) == 4 ? 4 : 2) void k_spread_rows3_many(
     const BatchProblem *__restrict__ probs, const SpreadProblem *__restrict__ sprobs, int nprob,
-    const uint32_t *__restrict__ offsets, const int4 *__restrict__ rec_start,
-    const T *__restrict__ rec_off, const T *__restrict__ c_sorted,
+    const uint32_t *__restrict__ offsets, const T *__restrict__ rec_off, const T *__restrict__ c_sorted,
     const uint32_t *__restrict__ totals, const uint32_t *__restrict__ parts,
     const uint32_t *__restrict__ item_off, const uint32_t *__restrict__ heavy_base,
     const uint32_t *__restrict__ pctrl, const int64_t *__restrict__ pbase,
@@ -288,7 +286,7 @@ __global__ __launch_bounds__(64, sizeof(T) == 4 ? 4 : 2) void k_spread_rows3_man
         const int64_t x0 = (b % nb0) * TX, y0 = ((b / nb0) % nb1) * TY, z0 = (b / (nb0 * nb1)) * TZ;
         typename mfma::ExactMma<T>::Acc acc[4];
         rows3_accumulate<T, W, NROWS>(st, rows, lane, pb.g, x0, y0, z0, ti.rlo, ti.rhi,
-                                      offsets + pb.bin_base, rec_start, rec_off, c_sorted, acc);
+                                      offsets + pb.bin_base, rec_off, c_sorted, acc);
         const bool whole = ti.np == 1;
         T *slot = whole ? nullptr
                         : partial + partial_index<TX, TY, TZ>(
@@ -329,7 +327,6 @@ __device__ __forceinline__ void rows2_accumulate(Rows2Stage<T> &st, TileRows<NRO
                                                  const GridParams &g, int64_t x0, int64_t y0,
                                                  int64_t klo, int64_t khi,
                                                  const uint32_t *__restrict__ offsets,
-                                                 const int4 *__restrict__ rec_start,
                                                  const T *__restrict__ rec_off,
                                                  const T *__restrict__ cv,
                                                  typename mfma::ExactMma<T>::Acc (&acc)[2])
@@ -347,10 +344,10 @@ __device__ __forceinline__ void rows2_accumulate(Rows2Stage<T> &st, TileRows<NRO
 #pragma unroll
     for (int b = 0; b < 2; ++b) acc[b] = typename Mma::Acc{(T)0, (T)0, (T)0, (T)0};
     const int lk = lane >> 4, ly = lane & 15, lx = (lane & 15) >> 1, lc = lane & 1;
-    Fetched<T> nx = fetch_record<T, NROWS>(rows, klo + lane, khi, rec_start, rec_off, cv);
+    Fetched<T> nx = fetch_record<T, NROWS>(rows, klo + lane, khi, rec_off, cv);
     for (int64_t k0 = klo; k0 < khi; k0 += 64) {
         const Fetched<T> cur = nx;
-        nx = fetch_record<T, NROWS>(rows, k0 + 64 + lane, khi, rec_start, rec_off, cv);
+        nx = fetch_record<T, NROWS>(rows, k0 + 64 + lane, khi, rec_off, cv);
         bool take = false;
         int ee = 0;
         if (cur.valid) {
@@ -425,7 +422,7 @@ __device__ __forceinline__ void rows2_store(int lane, const GridParams &g, int64
 template <typename T, int W>
 __global__ __launch_bounds__(64, sizeof(T) == 4 ? 4 : 2) void k_spread_rows2(
     GridParams g, SpreadParams sp, const uint32_t *__restrict__ offsets,
-    const int4 *__restrict__ rec_start, const T *__restrict__ rec_off,
+    const T *__restrict__ rec_off,
     const T *__restrict__ c_sorted, int64_t M, const uint32_t *__restrict__ totals,
     const uint32_t *__restrict__ parts, const uint32_t *__restrict__ item_off,
     const uint32_t *__restrict__ heavy_base, const uint32_t *__restrict__ ctrl,
@@ -450,7 +447,7 @@ __global__ __launch_bounds__(64, sizeof(T) == 4 ? 4 : 2) void k_spread_rows2(
         const int64_t x0 = (b % sp.nblocks[0]) * kRows2T, y0 = (b / sp.nblocks[0]) * kRows2T;
         typename mfma::ExactMma<T>::Acc acc[2];
         rows2_accumulate<T, W, NROWS>(st, rows, lane, g, x0, y0, ti.rlo, ti.rhi, offsets,
-                                      rec_start, rec_off, cv, acc);
+                                      rec_off, cv, acc);
         const bool whole = ti.np == 1;
         T *slot = whole ? nullptr
                         : partial + partial_index<kRows2T, kRows2T, 1>(
@@ -465,8 +462,7 @@ __global__ __launch_bounds__(64, sizeof(T) == 4 ? 4 : 2) void k_spread_rows2(
 template <typename T, int W>
 __global__ __launch_bounds__(64, sizeof(T) == 4 ? 4 : 2) void k_spread_rows2_many(
     const BatchProblem *__restrict__ probs, const SpreadProblem *__restrict__ sprobs, int nprob,
-    const uint32_t *__restrict__ offsets, const int4 *__restrict__ rec_start,
-    const T *__restrict__ rec_off, const T *__restrict__ c_sorted,
+    const uint32_t *__restrict__ offsets, const T *__restrict__ rec_off, const T *__restrict__ c_sorted,
     const uint32_t *__restrict__ totals, const uint32_t *__restrict__ parts,
     const uint32_t *__restrict__ item_off, const uint32_t *__restrict__ heavy_base,
     const uint32_t *__restrict__ pctrl, const int64_t *__restrict__ pbase,
@@ -492,7 +488,7 @@ __global__ __launch_bounds__(64, sizeof(T) == 4 ? 4 : 2) void k_spread_rows2_man
         const int64_t y0 = (b / spb.sp.nblocks[0]) * kRows2T;
         typename mfma::ExactMma<T>::Acc acc[2];
         rows2_accumulate<T, W, NROWS>(st, rows, lane, pb.g, x0, y0, ti.rlo, ti.rhi,
-                                      offsets + pb.bin_base, rec_start, rec_off, c_sorted, acc);
+                                      offsets + pb.bin_base, rec_off, c_sorted, acc);
         const bool whole = ti.np == 1;
         T *slot = whole ? nullptr
                         : partial + partial_index<kRows2T, kRows2T, 1>(
@@ -504,13 +500,13 @@ __global__ __launch_bounds__(64, sizeof(T) == 4 ? 4 : 2) void k_spread_rows2_man
 
 template <typename T, int W>
 bool launch_rows_width(int tx, dim3 grid3, const GridParams &g, const SpreadParams &sp,
-                       const uint32_t *offsets, const int4 *rec_start, const T *rec_off,
+                       const uint32_t *offsets, const T *rec_off,
                        const T *c_sorted, int64_t M, const TileWork &w, T *grid, T *partial,
                        hipStream_t stream)
 {
     if (tx != kRowsTX) return false;
     k_spread_rows<T, W><<<grid3, 64, 0, stream>>>(
-        g, sp, offsets, rec_start, rec_off, c_sorted, M, w.totals, w.parts, w.item_off,
+        g, sp, offsets, rec_off, c_sorted, M, w.totals, w.parts, w.item_off,
         w.heavy_base, w.ctrl, grid, partial);
     return true;
 }
@@ -519,7 +515,7 @@ bool launch_rows_width(int tx, dim3 grid3, const GridParams &g, const SpreadPara
 
 template <typename T>
 bool launch_rows2_tiles(const GridParams &g, const SpreadParams &sp, const uint32_t *offsets,
-                        const int4 *rec_start, const T *rec_off, const T *c_sorted, int64_t M,
+                        const T *rec_off, const T *c_sorted, int64_t M,
                         int64_t vectors, const TileWork &w, T *grid, T *partial,
                         hipStream_t stream)
 {
@@ -530,7 +526,7 @@ bool launch_rows2_tiles(const GridParams &g, const SpreadParams &sp, const uint3
     }
 #define MNUFFT_ROWS2(W)                                                                             \
     case W:                                                                                         \
-        k_spread_rows2<T, W><<<grid3, 64, 0, stream>>>(g, sp, offsets, rec_start, rec_off,          \
+        k_spread_rows2<T, W><<<grid3, 64, 0, stream>>>(g, sp, offsets, rec_off,          \
                                                        c_sorted, M, w.totals, w.parts, w.item_off,  \
                                                        w.heavy_base, w.ctrl, grid, partial);        \
         break;
@@ -553,7 +549,7 @@ bool launch_rows2_tiles(const GridParams &g, const SpreadParams &sp, const uint3
 template <typename T>
 bool launch_rows2_many(int width, const BatchProblem *probs, const SpreadProblem *sprobs,
                        int nprob, unsigned items_grid, const uint32_t *offsets,
-                       const int4 *rec_start, const T *rec_off, const T *c_sorted,
+                       const T *rec_off, const T *c_sorted,
                        const uint32_t *totals, const uint32_t *parts, const uint32_t *item_off,
                        const uint32_t *heavy_base, const uint32_t *pctrl, const int64_t *pbase,
                        T *partial, hipStream_t stream)
@@ -561,7 +557,7 @@ bool launch_rows2_many(int width, const BatchProblem *probs, const SpreadProblem
 #define MNUFFT_ROWS2_MANY(W)                                                                        \
     case W:                                                                                         \
         k_spread_rows2_many<T, W><<<items_grid, 64, 0, stream>>>(                                   \
-            probs, sprobs, nprob, offsets, rec_start, rec_off, c_sorted, totals, parts, item_off,   \
+            probs, sprobs, nprob, offsets, rec_off, c_sorted, totals, parts, item_off,   \
             heavy_base, pctrl, pbase, partial);                                                     \
         break;
     switch (width) {
@@ -581,12 +577,12 @@ bool launch_rows2_many(int width, const BatchProblem *probs, const SpreadProblem
 }
 
 template bool launch_rows2_many<float>(int, const BatchProblem *, const SpreadProblem *, int,
-                                       unsigned, const uint32_t *, const int4 *, const float *,
+                                       unsigned, const uint32_t *, const float *,
                                        const float *, const uint32_t *, const uint32_t *,
                                        const uint32_t *, const uint32_t *, const uint32_t *,
                                        const int64_t *, float *, hipStream_t);
 template bool launch_rows2_many<double>(int, const BatchProblem *, const SpreadProblem *, int,
-                                        unsigned, const uint32_t *, const int4 *, const double *,
+                                        unsigned, const uint32_t *, const double *,
                                         const double *, const uint32_t *, const uint32_t *,
                                         const uint32_t *, const uint32_t *, const uint32_t *,
                                         const int64_t *, double *, hipStream_t);
@@ -594,7 +590,7 @@ template bool launch_rows2_many<double>(int, const BatchProblem *, const SpreadP
 template <typename T>
 bool launch_rows3_many(int width, const BatchProblem *probs, const SpreadProblem *sprobs,
                        int nprob, unsigned items_grid, const uint32_t *offsets,
-                       const int4 *rec_start, const T *rec_off, const T *c_sorted,
+                       const T *rec_off, const T *c_sorted,
                        const uint32_t *totals, const uint32_t *parts, const uint32_t *item_off,
                        const uint32_t *heavy_base, const uint32_t *pctrl, const int64_t *pbase,
                        T *partial, hipStream_t stream)
@@ -603,7 +599,7 @@ bool launch_rows3_many(int width, const BatchProblem *probs, const SpreadProblem
 #define MNUFFT_ROWS3_MANY(W)                                                                        \
     case W:                                                                                         \
         k_spread_rows3_many<T, W><<<items_grid, 64, 0, stream>>>(                                   \
-            probs, sprobs, nprob, offsets, rec_start, rec_off, c_sorted, totals, parts, item_off,   \
+            probs, sprobs, nprob, offsets, rec_off, c_sorted, totals, parts, item_off,   \
             heavy_base, pctrl, pbase, partial);                                                     \
         break;
     switch (width) {
@@ -641,23 +637,23 @@ bool launch_rows3_many(int width, const BatchProblem *probs, const SpreadProblem
 }
 
 template bool launch_rows3_many<float>(int, const BatchProblem *, const SpreadProblem *, int,
-                                       unsigned, const uint32_t *, const int4 *, const float *,
+                                       unsigned, const uint32_t *, const float *,
                                        const float *, const uint32_t *, const uint32_t *,
                                        const uint32_t *, const uint32_t *, const uint32_t *,
                                        const int64_t *, float *, hipStream_t);
 template bool launch_rows3_many<double>(int, const BatchProblem *, const SpreadProblem *, int,
-                                        unsigned, const uint32_t *, const int4 *, const double *,
+                                        unsigned, const uint32_t *, const double *,
                                         const double *, const uint32_t *, const uint32_t *,
                                         const uint32_t *, const uint32_t *, const uint32_t *,
                                         const int64_t *, double *, hipStream_t);
 
 template <typename T>
 bool launch_rows_tiles(const GridParams &g, const SpreadParams &sp, const uint32_t *offsets,
-                       const int4 *rec_start, const T *rec_off, const T *c_sorted, int64_t M,
+                       const T *rec_off, const T *c_sorted, int64_t M,
                        int64_t vectors, const TileWork &w, T *grid, T *partial, hipStream_t stream)
 {
     if (g.dims == 2)
-        return launch_rows2_tiles<T>(g, sp, offsets, rec_start, rec_off, c_sorted, M, vectors, w,
+        return launch_rows2_tiles<T>(g, sp, offsets, rec_off, c_sorted, M, vectors, w,
                                      grid, partial, stream);
     const dim3 grid3(w.items_grid, (unsigned)vectors);
     const int tx = (int)sp.block[0];
@@ -667,24 +663,24 @@ bool launch_rows_tiles(const GridParams &g, const SpreadParams &sp, const uint32
     }
     bool ok = false;
     switch (g.width) {
-    case 2: ok = launch_rows_width<T, 2>(tx, grid3, g, sp, offsets, rec_start, rec_off, c_sorted, M, w, grid, partial, stream); break;
-    case 3: ok = launch_rows_width<T, 3>(tx, grid3, g, sp, offsets, rec_start, rec_off, c_sorted, M, w, grid, partial, stream); break;
-    case 4: ok = launch_rows_width<T, 4>(tx, grid3, g, sp, offsets, rec_start, rec_off, c_sorted, M, w, grid, partial, stream); break;
-    case 5: ok = launch_rows_width<T, 5>(tx, grid3, g, sp, offsets, rec_start, rec_off, c_sorted, M, w, grid, partial, stream); break;
-    case 6: ok = launch_rows_width<T, 6>(tx, grid3, g, sp, offsets, rec_start, rec_off, c_sorted, M, w, grid, partial, stream); break;
-    case 7: ok = launch_rows_width<T, 7>(tx, grid3, g, sp, offsets, rec_start, rec_off, c_sorted, M, w, grid, partial, stream); break;
-    case 8: ok = launch_rows_width<T, 8>(tx, grid3, g, sp, offsets, rec_start, rec_off, c_sorted, M, w, grid, partial, stream); break;
+    case 2: ok = launch_rows_width<T, 2>(tx, grid3, g, sp, offsets, rec_off, c_sorted, M, w, grid, partial, stream); break;
+    case 3: ok = launch_rows_width<T, 3>(tx, grid3, g, sp, offsets, rec_off, c_sorted, M, w, grid, partial, stream); break;
+    case 4: ok = launch_rows_width<T, 4>(tx, grid3, g, sp, offsets, rec_off, c_sorted, M, w, grid, partial, stream); break;
+    case 5: ok = launch_rows_width<T, 5>(tx, grid3, g, sp, offsets, rec_off, c_sorted, M, w, grid, partial, stream); break;
+    case 6: ok = launch_rows_width<T, 6>(tx, grid3, g, sp, offsets, rec_off, c_sorted, M, w, grid, partial, stream); break;
+    case 7: ok = launch_rows_width<T, 7>(tx, grid3, g, sp, offsets, rec_off, c_sorted, M, w, grid, partial, stream); break;
+    case 8: ok = launch_rows_width<T, 8>(tx, grid3, g, sp, offsets, rec_off, c_sorted, M, w, grid, partial, stream); break;
     default:
         if constexpr (sizeof(T) == 8) {
             switch (g.width) {
-            case 9: ok = launch_rows_width<T, 9>(tx, grid3, g, sp, offsets, rec_start, rec_off, c_sorted, M, w, grid, partial, stream); break;
-            case 10: ok = launch_rows_width<T, 10>(tx, grid3, g, sp, offsets, rec_start, rec_off, c_sorted, M, w, grid, partial, stream); break;
-            case 11: ok = launch_rows_width<T, 11>(tx, grid3, g, sp, offsets, rec_start, rec_off, c_sorted, M, w, grid, partial, stream); break;
-            case 12: ok = launch_rows_width<T, 12>(tx, grid3, g, sp, offsets, rec_start, rec_off, c_sorted, M, w, grid, partial, stream); break;
-            case 13: ok = launch_rows_width<T, 13>(tx, grid3, g, sp, offsets, rec_start, rec_off, c_sorted, M, w, grid, partial, stream); break;
-            case 14: ok = launch_rows_width<T, 14>(tx, grid3, g, sp, offsets, rec_start, rec_off, c_sorted, M, w, grid, partial, stream); break;
-            case 15: ok = launch_rows_width<T, 15>(tx, grid3, g, sp, offsets, rec_start, rec_off, c_sorted, M, w, grid, partial, stream); break;
-            case 16: ok = launch_rows_width<T, 16>(tx, grid3, g, sp, offsets, rec_start, rec_off, c_sorted, M, w, grid, partial, stream); break;
+            case 9: ok = launch_rows_width<T, 9>(tx, grid3, g, sp, offsets, rec_off, c_sorted, M, w, grid, partial, stream); break;
+            case 10: ok = launch_rows_width<T, 10>(tx, grid3, g, sp, offsets, rec_off, c_sorted, M, w, grid, partial, stream); break;
+            case 11: ok = launch_rows_width<T, 11>(tx, grid3, g, sp, offsets, rec_off, c_sorted, M, w, grid, partial, stream); break;
+            case 12: ok = launch_rows_width<T, 12>(tx, grid3, g, sp, offsets, rec_off, c_sorted, M, w, grid, partial, stream); break;
+            case 13: ok = launch_rows_width<T, 13>(tx, grid3, g, sp, offsets, rec_off, c_sorted, M, w, grid, partial, stream); break;
+            case 14: ok = launch_rows_width<T, 14>(tx, grid3, g, sp, offsets, rec_off, c_sorted, M, w, grid, partial, stream); break;
+            case 15: ok = launch_rows_width<T, 15>(tx, grid3, g, sp, offsets, rec_off, c_sorted, M, w, grid, partial, stream); break;
+            case 16: ok = launch_rows_width<T, 16>(tx, grid3, g, sp, offsets, rec_off, c_sorted, M, w, grid, partial, stream); break;
             default: break;
             }
         }
@@ -699,10 +695,10 @@ bool launch_rows_tiles(const GridParams &g, const SpreadParams &sp, const uint32
 }
 
 template bool launch_rows_tiles<float>(const GridParams &, const SpreadParams &, const uint32_t *,
-                                       const int4 *, const float *, const float *, int64_t,
+                                       const float *, const float *, int64_t,
                                        int64_t, const TileWork &, float *, float *, hipStream_t);
 template bool launch_rows_tiles<double>(const GridParams &, const SpreadParams &,
-                                        const uint32_t *, const int4 *, const double *,
+                                        const uint32_t *, const double *,
                                         const double *, int64_t, int64_t, const TileWork &,
                                         double *, double *, hipStream_t);
 

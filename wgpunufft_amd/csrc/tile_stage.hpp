@@ -89,6 +89,10 @@ struct Vec4Of<double> {
     using V2 = double2;
 };
 
+// The x start kept in a record's fourth offset word (store_record).
+__device__ inline int record_start_x(float w) { return __float_as_int(w); }
+__device__ inline int record_start_x(double w) { return (int)w; }
+
 // One lane's record of a chunk (the tile's k-th record), with its global
 // loads in flight until used.
 template <typename T>
@@ -101,7 +105,6 @@ struct Fetched {
 
 template <typename T, int NROWS>
 __device__ inline Fetched<T> fetch_record(const TileRows<NROWS> &rows, int64_t k, int64_t khi,
-                                          const int4 *__restrict__ rec_start,
                                           const T *__restrict__ rec_off,
                                           const T *__restrict__ cv)
 {
@@ -115,8 +118,8 @@ __device__ inline Fetched<T> fetch_record(const TileRows<NROWS> &rows, int64_t k
     f.c = V2{(T)0, (T)0};
     if (f.valid) {
         const uint32_t slot = tile_slot<NROWS>(rows, (uint32_t)k, &f.q);
-        f.sx0 = rec_start[slot].x;
         f.off = *(const V4 *)(rec_off + 4 * (int64_t)slot);
+        f.sx0 = record_start_x(f.off.w);
         f.c = *(const V2 *)(cv + 2 * (int64_t)slot);
     }
     return f;
