@@ -45,10 +45,11 @@ using namespace mfma;
 constexpr int kTile = 16;
 constexpr int kPitch = 20;  // LDS pitch of the weight tables, in floats
 
+template <int NV>
 struct MfmaRec {
     int sx, sy, sz;  // support start relative to the tile origin
     float ox, oy, oz;
-    float cre, cim;  // scaled strength
+    float2 c[NV];  // scaled strengths
 };
 
 // Largest |re|, |im| of each vector's strengths (blockIdx.y), as float bits
@@ -95,12 +96,21 @@ __global__ __launch_bounds__(256) void k_absmax(const float *__restrict__ c, int
     }
 }
 
-template <int W, int MODE, int TZ>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void
+// NV vectors of strengths in one pass over the tile's records.  What bounds
+// the pass is the serial chain of a k-block (records -> weights -> LDS ->
+// split operands), not the matrix cores, so two vectors share it: the search
+// of the records, the weight tables and the A operands are formed once and
+// each vector adds its B operand and its products.  Two vectors' accumulators
+// take 128 registers, which leaves 2 waves per SIMD instead of 3; four would
+// leave one.  16 vectors of 4.2e6 radial points on 512^3: the whole type 1
+// 29.6 ms with one vector a pass, 27.2 ms with two.
+template <int W, int MODE, int TZ, int NV>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(NV == 1 ? 3 : 2))) void
 k_spread_mfma3(
     GridParams g, SpreadParams sp, const uint32_t *__restrict__ offsets,
     const float *__restrict__ rec_off,
-    const float *__restrict__ c_sorted, int64_t M, const uint32_t *__restrict__ totals,
+    const float *__restrict__ c_sorted, int64_t M, int64_t v0, int64_t vectors,
+    const uint32_t *__restrict__ totals,
     const uint32_t *__restrict__ parts, const uint32_t *__restrict__ item_off,
     const uint32_t *__restrict__ heavy_base, const uint32_t *__restrict__ ctrl,
     const uint32_t *__restrict__ cmax, float *__restrict__ grid, float *__restrict__ partial)
@@ -115,8 +125,8 @@ k_spread_mfma3(
     __shared__ __align__(16) float KX[(kTile + 1) * kPitch];
     __shared__ __align__(16) float KY[(kTile + 1) * kPitch];
     __shared__ __align__(16) float KZ[(kTile + 1) * kPitch];
-    __shared__ __align__(16) float CC[2 * kPitch];
-    __shared__ MfmaRec st[64];
+    __shared__ __align__(16) float CC[2 * NV * kPitch];
+    __shared__ MfmaRec<NV> st[64];
     __shared__ TileRows<NROWS> rows;
 
     const int lane = threadIdx.x;
@@ -128,10 +138,11 @@ k_spread_mfma3(
     const int bxc = r32 >> 1;  // B column: x cell, real (0) or imaginary (1)
     const int bpart = r32 & 1;
 
-    float scale, unscale;
-    strength_scale(cmax + blockIdx.y, &scale, &unscale);
+    const int64_t v = v0 + NV * (int64_t)blockIdx.y;  // first of the NV vectors
+    float scale[NV], unscale[NV];
+#pragma unroll
+    for (int u = 0; u < NV; ++u) strength_scale(cmax + v + u, &scale[u], &unscale[u]);
 
-    const int64_t v = blockIdx.y;
     const UniformPtr<float> panels = panel_coefficients<float>(g);
     const int64_t n_items = ctrl[0];
     const uint32_t part_len_cap = ctrl[3];
@@ -152,18 +163,21 @@ k_spread_mfma3(
         if (xs < 0) xs += n0;
 
         stage_tile_rows<3, kTile, TZ, W, NROWS>(rows, lane, y0, z0, rx, g, offsets);
-        f32x16 acc[kBlocks];
+        f32x16 acc[NV][kBlocks];
 #pragma unroll
-        for (int m = 0; m < kBlocks; ++m) acc[m] = f32x16{};
+        for (int u = 0; u < NV; ++u)
+#pragma unroll
+            for (int m = 0; m < kBlocks; ++m) acc[u][m] = f32x16{};
         // records in chunks of 64, the next chunk's loads in flight while
         // the current one is contracted
         const int64_t klo = rlo, khi = rhi;
-        Fetched<float> nx = fetch_record<float, NROWS>(rows, klo + lane, khi, rec_off, cv);
+        Fetched<float, NV> nx =
+            fetch_record<float, NROWS, NV>(rows, klo + lane, khi, rec_off, cv, 2 * M);
         for (int64_t k0 = klo; k0 < khi; k0 += 64) {
-            const Fetched<float> cur = nx;
-            nx = fetch_record<float, NROWS>(rows, k0 + 64 + lane, khi, rec_off, cv);
+            const Fetched<float, NV> cur = nx;
+            nx = fetch_record<float, NROWS, NV>(rows, k0 + 64 + lane, khi, rec_off, cv, 2 * M);
             bool take = false;
-            MfmaRec R{};
+            MfmaRec<NV> R{};
             if (cur.valid) {
                 int64_t ee = (int64_t)cur.sx0 - xs;
                 if (ee < 0) ee += n0;
@@ -174,8 +188,11 @@ k_spread_mfma3(
                 R.ox = cur.off.x;
                 R.oy = cur.off.y;
                 R.oz = cur.off.z;
-                R.cre = cur.c.x * scale;
-                R.cim = cur.c.y * scale;
+#pragma unroll
+                for (int u = 0; u < NV; ++u) {
+                    R.c[u].x = cur.c[u].x * scale[u];
+                    R.c[u].y = cur.c[u].y * scale[u];
+                }
             }
             const uint64_t mask = __ballot(take);
             const int pos = __popcll(mask & ((1ull << lane) - 1ull));
@@ -196,12 +213,12 @@ k_spread_mfma3(
                 if (lane < 48) {
                     const int j = lane & 15, axis = lane >> 4;
                     if (j < kn) {
-                        const MfmaRec &S = st[kb + j];
+                        const MfmaRec<NV> &S = st[kb + j];
                         const int s = axis == 0 ? S.sx : (axis == 1 ? S.sy : S.sz);
                         const float o = axis == 0 ? S.ox : (axis == 1 ? S.oy : S.oz);
                         float *tb = axis == 0 ? KX : (axis == 1 ? KY : KZ);
                         const unsigned lim = axis == 2 ? TZ : kTile;
-es_axis_weights<float, W>(o, (float)g.beta, panels, [&](int t, float wt) {
+                        es_axis_weights<float, W>(o, (float)g.beta, panels, [&](int t, float wt) {
                             const unsigned c = (unsigned)(s + t);
                             const unsigned row = c < lim ? c : (unsigned)kTile;
                             tb[row * kPitch + j] = wt;
@@ -209,8 +226,11 @@ es_axis_weights<float, W>(o, (float)g.beta, panels, [&](int t, float wt) {
                     }
                 } else {
                     const int j = lane - 48;
-                    CC[j] = j < kn ? st[kb + j].cre : 0.0f;
-                    CC[kPitch + j] = j < kn ? st[kb + j].cim : 0.0f;
+#pragma unroll
+                    for (int u = 0; u < NV; ++u) {
+                        CC[2 * u * kPitch + j] = j < kn ? st[kb + j].c[u].x : 0.0f;
+                        CC[(2 * u + 1) * kPitch + j] = j < kn ? st[kb + j].c[u].y : 0.0f;
+                    }
                 }
                 wave_sync();
                 // band of z cells the k-block touches (records in row order)
@@ -220,11 +240,14 @@ es_axis_weights<float, W>(o, (float)g.beta, panels, [&](int t, float wt) {
                 zhi = zhi > TZ - 1 ? TZ - 1 : zhi;
                 const int mlo = zlo >> 1, mhi = zhi >> 1;
 
-                V bh, bl;
+                V bh[NV], bl[NV];
                 {
                     const f32x8 kx = load8(KX + bxc * kPitch + j0);
-                    const f32x8 cc = load8(CC + bpart * kPitch + j0);
-                    Op::split(kx * cc, bh, bl);
+#pragma unroll
+                    for (int u = 0; u < NV; ++u) {
+                        const f32x8 cc = load8(CC + (2 * u + bpart) * kPitch + j0);
+                        Op::split(kx * cc, bh[u], bl[u]);
+                    }
                 }
                 const f32x8 ky = load8(KY + ay * kPitch + j0);
 #pragma unroll
@@ -233,10 +256,13 @@ es_axis_weights<float, W>(o, (float)g.beta, panels, [&](int t, float wt) {
                     const f32x8 kz = load8(KZ + (2 * m + az) * kPitch + j0);
                     V ah, al;
                     Op::split(ky * kz, ah, al);
-                    acc[m] = Op::mma(ah, bh, acc[m]);
-                    if constexpr (kSplit) {
-                        acc[m] = Op::mma(ah, bl, acc[m]);
-                        acc[m] = Op::mma(al, bh, acc[m]);
+#pragma unroll
+                    for (int u = 0; u < NV; ++u) {
+                        acc[u][m] = Op::mma(ah, bh[u], acc[u][m]);
+                        if constexpr (kSplit) {
+                            acc[u][m] = Op::mma(ah, bl[u], acc[u][m]);
+                            acc[u][m] = Op::mma(al, bh[u], acc[u][m]);
+                        }
                     }
                 }
                 wave_sync();
@@ -248,18 +274,20 @@ es_axis_weights<float, W>(o, (float)g.beta, panels, [&](int t, float wt) {
         // the block (y = row % 16, z = 2m + row / 16), column r32
         const int64_t pslot = np > 1 ? (int64_t)heavy_base[b] + p : 0;
 #pragma unroll
-        for (int m = 0; m < kBlocks; ++m) {
+        for (int t = 0; t < NV * kBlocks; ++t) {
+            const int u = t / kBlocks, m = t % kBlocks;
 #pragma unroll
             for (int i = 0; i < 16; ++i) {
                 const int row = 8 * (i >> 2) + 4 * half + (i & 3);
                 const int yy = row & 15, zz = 2 * m + (row >> 4);
-                const float val = acc[m][i] * unscale;
+                const float val = acc[u][m][i] * unscale[u];
                 if (np == 1) {
                     const int64_t gx = x0 + bxc, gy = y0 + yy, gz = z0 + zz;
                     if (gx < n0 && gy < n1 && gz < n2)
-                        grid[2 * (v * g.fine_total + gx + n0 * (gy + n1 * gz)) + bpart] = val;
+                        grid[2 * ((v + u) * g.fine_total + gx + n0 * (gy + n1 * gz)) + bpart] =
+                            val;
                 } else {
-                    partial[partial_index<kTile, kTile, TZ>(pslot, gridDim.y, v, bxc, yy, zz) +
+                    partial[partial_index<kTile, kTile, TZ>(pslot, vectors, v + u, bxc, yy, zz) +
                             bpart] = val;
                 }
             }
@@ -290,7 +318,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_
     __shared__ __align__(16) float KX[(kTile2 + 1) * kPitch];
     __shared__ __align__(16) float KY[(kTile2 + 1) * kPitch];
     __shared__ __align__(16) float CC[2 * kPitch];
-    __shared__ MfmaRec st[64];
+    __shared__ MfmaRec<1> st[64];
     __shared__ TileRows<NROWS> rows;
 
     const int lane = threadIdx.x;
@@ -329,7 +357,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_
             const Fetched<float> cur = nx;
             nx = fetch_record<float, NROWS>(rows, k0 + 64 + lane, khi, rec_off, cv);
             bool take = false;
-            MfmaRec R{};
+            MfmaRec<1> R{};
             if (cur.valid) {
                 int64_t ee = (int64_t)cur.sx0 - xs;
                 if (ee < 0) ee += n0;
@@ -338,8 +366,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_
                 R.sy = cur.q - (W - 1);
                 R.ox = cur.off.x;
                 R.oy = cur.off.y;
-                R.cre = cur.c.x * scale;
-                R.cim = cur.c.y * scale;
+                R.c[0].x = cur.c[0].x * scale;
+                R.c[0].y = cur.c[0].y * scale;
             }
             const uint64_t mask = __ballot(take);
             const int pos = __popcll(mask & ((1ull << lane) - 1ull));
@@ -360,7 +388,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_
                 if (lane < 32) {
                     const int j = lane & 15, axis = lane >> 4;
                     if (j < kn) {
-                        const MfmaRec &S = st[kb + j];
+                        const MfmaRec<1> &S = st[kb + j];
                         const int s0 = axis == 0 ? S.sx : S.sy;
                         const float o = axis == 0 ? S.ox : S.oy;
                         float *tb = axis == 0 ? KX : KY;
@@ -373,8 +401,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_
                     }
                 } else if (lane < 48) {
                     const int j = lane - 32;
-                    CC[j] = j < kn ? st[kb + j].cre : 0.0f;
-                    CC[kPitch + j] = j < kn ? st[kb + j].cim : 0.0f;
+                    CC[j] = j < kn ? st[kb + j].c[0].x : 0.0f;
+                    CC[kPitch + j] = j < kn ? st[kb + j].c[0].y : 0.0f;
                 }
                 wave_sync();
                 V ah, al;
@@ -423,14 +451,23 @@ void launch_kernel(dim3 grid3, const GridParams &g, const SpreadParams &sp,
                    const float *c_sorted, int64_t M, const TileWork &w, float *grid,
                    float *partial, hipStream_t stream)
 {
-    if constexpr (D == 3)
-        k_spread_mfma3<W, MODE, 8><<<grid3, 64, 0, stream>>>(
-            g, sp, offsets, rec_off, c_sorted, M, w.totals, w.parts, w.item_off,
-            w.heavy_base, w.ctrl, w.cmax, grid, partial);
-    else
+    if constexpr (D == 3) {
+        // vectors in pairs, an odd last one by itself: each vector's sums are
+        // the same in either form
+        const int64_t vectors = grid3.y, pairs = vectors / 2;
+        if (pairs)
+            k_spread_mfma3<W, MODE, 8, 2><<<dim3(grid3.x, (unsigned)pairs), 64, 0, stream>>>(
+                g, sp, offsets, rec_off, c_sorted, M, 0, vectors, w.totals, w.parts, w.item_off,
+                w.heavy_base, w.ctrl, w.cmax, grid, partial);
+        if (vectors & 1)
+            k_spread_mfma3<W, MODE, 8, 1><<<dim3(grid3.x), 64, 0, stream>>>(
+                g, sp, offsets, rec_off, c_sorted, M, vectors - 1, vectors, w.totals, w.parts,
+                w.item_off, w.heavy_base, w.ctrl, w.cmax, grid, partial);
+    } else {
         k_spread_mfma2<W, MODE><<<grid3, 64, 0, stream>>>(
             g, sp, offsets, rec_off, c_sorted, M, w.totals, w.parts, w.item_off,
             w.heavy_base, w.ctrl, w.cmax, grid, partial);
+    }
 }
 
 template <int D, int W>
@@ -445,12 +482,12 @@ bool launch_width(SpreadMethod method, dim3 grid3, const GridParams &g, const Sp
                                                         c_sorted, M, w, grid, partial, stream);
         return true;
     case SpreadMethod::MfmaF16x3:
-        launch_kernel<D, W, (int)SpreadMethod::MfmaF16x3>(grid3, g, sp, offsets,                                                           rec_off, c_sorted, M, w, grid, partial,
-                                                          stream);
+        launch_kernel<D, W, (int)SpreadMethod::MfmaF16x3>(grid3, g, sp, offsets, rec_off,
+                                                          c_sorted, M, w, grid, partial, stream);
         return true;
     case SpreadMethod::MfmaBf16x3:
-        launch_kernel<D, W, (int)SpreadMethod::MfmaBf16x3>(grid3, g, sp, offsets,                                                            rec_off, c_sorted, M, w, grid, partial,
-                                                           stream);
+        launch_kernel<D, W, (int)SpreadMethod::MfmaBf16x3>(grid3, g, sp, offsets, rec_off,
+                                                           c_sorted, M, w, grid, partial, stream);
         return true;
     default:
         return false;

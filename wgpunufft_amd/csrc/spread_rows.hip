@@ -152,8 +152,8 @@ __device__ __forceinline__ void rows3_accumulate(Rows3Stage<T> &st, TileRows<NRO
             tile_weights<T, W, TX>(R.kx, ee - (W - 1), (T)cur.off.x, beta, panels, same);
             tile_weights<T, W, TY>(R.ky, cur.q % NRY - (W - 1), (T)cur.off.y, beta, panels, same);
             tile_weights<T, W, TZ>(R.kz, rz, (T)cur.off.z, beta, panels, by_block);
-            R.c[0] = cur.c.x;
-            R.c[1] = cur.c.y;
+            R.c[0] = cur.c[0].x;
+            R.c[1] = cur.c[0].y;
             const int lo = rz > 0 ? rz >> 1 : 0, hi = rz + W - 1 < TZ ? (rz + W - 1) >> 1 : 3;
             st.blocks[pos] = (2u << hi) - (1u << lo);
         }
@@ -365,8 +365,8 @@ __device__ __forceinline__ void rows2_accumulate(Rows2Stage<T> &st, TileRows<NRO
             Row2Rec<T> &R = st.rec[pos];
             tile_weights<T, W, TX>(R.kx, rel, (T)cur.off.x, beta, panels, same);
             tile_weights<T, W, TY>(R.ky, cur.q - (W - 1), (T)cur.off.y, beta, panels, same);
-            R.c[0] = cur.c.x;
-            R.c[1] = cur.c.y;
+            R.c[0] = cur.c[0].x;
+            R.c[1] = cur.c[0].y;
             st.blocks[pos] = (rel < 8 ? 1u : 0u) | (rel + W > 8 ? 2u : 0u);
         }
         if (lane < 7 && nst + lane < 64) st.rec[nst + lane].c[0] = st.rec[nst + lane].c[1] = (T)0;

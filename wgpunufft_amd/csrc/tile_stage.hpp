@@ -93,34 +93,37 @@ struct Vec4Of<double> {
 __device__ inline int record_start_x(float w) { return __float_as_int(w); }
 __device__ inline int record_start_x(double w) { return (int)w; }
 
-// One lane's record of a chunk (the tile's k-th record), with its global
-// loads in flight until used.
-template <typename T>
+// One lane's record of a chunk (the tile's k-th record) with NV vectors of
+// strengths, `stride` values apart, its global loads in flight until used.
+template <typename T, int NV = 1>
 struct Fetched {
     int q, sx0;
     typename Vec4Of<T>::V4 off;
-    typename Vec4Of<T>::V2 c;
+    typename Vec4Of<T>::V2 c[NV];
     bool valid;
 };
 
-template <typename T, int NROWS>
-__device__ inline Fetched<T> fetch_record(const TileRows<NROWS> &rows, int64_t k, int64_t khi,
-                                          const T *__restrict__ rec_off,
-                                          const T *__restrict__ cv)
+template <typename T, int NROWS, int NV = 1>
+__device__ inline Fetched<T, NV> fetch_record(const TileRows<NROWS> &rows, int64_t k, int64_t khi,
+                                              const T *__restrict__ rec_off,
+                                              const T *__restrict__ cv, int64_t stride = 0)
 {
     using V4 = typename Vec4Of<T>::V4;
     using V2 = typename Vec4Of<T>::V2;
-    Fetched<T> f;
+    Fetched<T, NV> f;
     f.valid = k < khi;
     f.q = 0;
     f.sx0 = 0;
     f.off = V4{(T)0, (T)0, (T)0, (T)0};
-    f.c = V2{(T)0, (T)0};
+#pragma unroll
+    for (int u = 0; u < NV; ++u) f.c[u] = V2{(T)0, (T)0};
     if (f.valid) {
         const uint32_t slot = tile_slot<NROWS>(rows, (uint32_t)k, &f.q);
         f.off = *(const V4 *)(rec_off + 4 * (int64_t)slot);
         f.sx0 = record_start_x(f.off.w);
-        f.c = *(const V2 *)(cv + 2 * (int64_t)slot);
+#pragma unroll
+        for (int u = 0; u < NV; ++u)
+            f.c[u] = *(const V2 *)(cv + u * stride + 2 * (int64_t)slot);
     }
     return f;
 }
