@@ -401,34 +401,76 @@ __global__ void k_clear_u32(uint32_t *p, int64_t n)
     if (i < n) p[i] = 0u;
 }
 
+// Targets are counted and placed by box through counters in LDS, one global
+// addition a workgroup and box: a few boxes take all targets, and global
+// additions to one address go one after the other (1e6 targets in 27 boxes:
+// 2.0 ms to count and 2.2 ms to place by one addition a target, 0.015 and
+// 0.048 ms so).
+// Boxes past the LDS counters are added to in global memory; the order of a
+// box's targets is free (each target's sum stands alone).
+constexpr int kBoxSlots = 1024;
+constexpr int kBoxTargets = 8;  // a lane's targets
+
 template <int D, typename T>
 __global__ __launch_bounds__(256) void k_type3_box_count(Type3Boxes bx, int64_t N,
                                                          const T *__restrict__ s,
                                                          uint32_t *__restrict__ box,
                                                          uint32_t *__restrict__ counts)
 {
-    const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= N) return;
-    const uint32_t b = target_box<D, T>(bx, s + k * D);
-    box[k] = b;
-    atomicAdd(counts + b, 1u);
+    __shared__ uint32_t cnt[kBoxSlots];
+    const int slots = bx.count < kBoxSlots ? (int)bx.count : kBoxSlots;
+    for (int t = threadIdx.x; t < slots; t += 256) cnt[t] = 0u;
+    __syncthreads();
+    const int64_t k0 = (int64_t)blockIdx.x * (256 * kBoxTargets) + threadIdx.x;
+#pragma unroll
+    for (int i = 0; i < kBoxTargets; ++i) {
+        const int64_t k = k0 + 256 * i;
+        if (k >= N) break;
+        const uint32_t b = target_box<D, T>(bx, s + k * D);
+        box[k] = b;
+        atomicAdd(b < (uint32_t)kBoxSlots ? cnt + b : counts + b, 1u);
+    }
+    __syncthreads();
+    for (int t = threadIdx.x; t < slots; t += 256)
+        if (cnt[t]) atomicAdd(counts + t, cnt[t]);
 }
 
 template <int D, typename T>
-__global__ __launch_bounds__(256) void k_type3_box_scatter(int64_t N, const T *__restrict__ s,
+__global__ __launch_bounds__(256) void k_type3_box_scatter(int64_t N, int64_t nbox,
+                                                           const T *__restrict__ s,
                                                            const uint32_t *__restrict__ box,
                                                            const uint32_t *__restrict__ offsets,
                                                            uint32_t *__restrict__ cursor,
                                                            uint32_t *__restrict__ perm,
                                                            T *__restrict__ s_sorted)
 {
-    const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= N) return;
-    const uint32_t b = box[k];
-    const int64_t pos = (int64_t)offsets[b] + atomicAdd(cursor + b, 1u);
-    perm[pos] = (uint32_t)k;
+    __shared__ uint32_t cnt[kBoxSlots];
+    const int slots = nbox < kBoxSlots ? (int)nbox : kBoxSlots;
+    for (int t = threadIdx.x; t < slots; t += 256) cnt[t] = 0u;
+    __syncthreads();
+    const int64_t k0 = (int64_t)blockIdx.x * (256 * kBoxTargets) + threadIdx.x;
+    uint32_t b[kBoxTargets], rank[kBoxTargets];
 #pragma unroll
-    for (int a = 0; a < D; ++a) s_sorted[pos * D + a] = s[k * D + a];
+    for (int i = 0; i < kBoxTargets; ++i) {
+        const int64_t k = k0 + 256 * i;
+        b[i] = k < N ? box[k] : 0u;
+        if (k < N) rank[i] = atomicAdd(b[i] < (uint32_t)kBoxSlots ? cnt + b[i] : cursor + b[i], 1u);
+    }
+    __syncthreads();
+    // from a box's count in this workgroup to its first place
+    for (int t = threadIdx.x; t < slots; t += 256)
+        if (cnt[t]) cnt[t] = offsets[t] + atomicAdd(cursor + t, cnt[t]);
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kBoxTargets; ++i) {
+        const int64_t k = k0 + 256 * i;
+        if (k >= N) break;
+        const int64_t pos =
+            (int64_t)rank[i] + (b[i] < (uint32_t)kBoxSlots ? cnt[b[i]] : offsets[b[i]]);
+        perm[pos] = (uint32_t)k;
+#pragma unroll
+        for (int a = 0; a < D; ++a) s_sorted[pos * D + a] = s[k * D + a];
+    }
 }
 
 // ---------------------------------------------------------------------
@@ -626,7 +668,8 @@ bool type3_box_count(const Type3Boxes &bx, int64_t N, const T *s, uint32_t *box,
 {
     k_clear_u32<<<grid_for(bx.count, 256), 256, 0, stream>>>(counts, bx.count);
     if (N > 0)
-        k_type3_box_count<D, T><<<grid_for(N, 256), 256, 0, stream>>>(bx, N, s, box, counts);
+        k_type3_box_count<D, T><<<grid_for(N, 256 * kBoxTargets), 256, 0, stream>>>(bx, N, s, box,
+                                                                                   counts);
     return hip_ok(hipGetLastError(), "type-3 box count launch");
 }
 
@@ -637,8 +680,8 @@ bool type3_box_scatter(const Type3Boxes &bx, int64_t N, const T *s, const uint32
 {
     k_clear_u32<<<grid_for(bx.count, 256), 256, 0, stream>>>(cursor, bx.count);
     if (N > 0)
-        k_type3_box_scatter<D, T><<<grid_for(N, 256), 256, 0, stream>>>(N, s, box, offsets, cursor,
-                                                                       perm, s_sorted);
+        k_type3_box_scatter<D, T><<<grid_for(N, 256 * kBoxTargets), 256, 0, stream>>>(
+            N, bx.count, s, box, offsets, cursor, perm, s_sorted);
     return hip_ok(hipGetLastError(), "type-3 box scatter launch");
 }
 
