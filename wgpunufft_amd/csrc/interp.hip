@@ -391,8 +391,8 @@ __device__ __forceinline__ void interp_tile3(typename Complex2<T>::type *tile, c
             }
         }
         T *dst = out_v + 2 * (int64_t)idx;
-        dst[0] = sre;
-        dst[1] = sim;
+        dst[0] = reach ? sre : (T)0;
+        dst[1] = reach ? sim : (T)0;
     }
     __syncthreads();
 }
@@ -592,7 +592,7 @@ __global__ __launch_bounds__(kWide3Threads) void k_interp_wide3(
             }
             sre = quad_add_xor<2>(quad_add_xor<1>(sre));
             sim = quad_add_xor<2>(quad_add_xor<1>(sim));
-            if (j < 2) out_v[2 * (int64_t)idx + j] = j == 0 ? sre : sim;
+            if (j < 2) out_v[2 * (int64_t)idx + j] = reach ? (j == 0 ? sre : sim) : 0.0;
         }
         __syncthreads();
     }
@@ -731,8 +731,8 @@ __global__ __launch_bounds__(THREADS) void k_interp_tiled2(
                 }
             }
             T *dst = out + 2 * (vo + (int64_t)idx);
-            dst[0] = sre;
-            dst[1] = sim;
+            dst[0] = reach ? sre : (T)0;
+            dst[1] = reach ? sim : (T)0;
         }
         __syncthreads();
     }
@@ -788,8 +788,8 @@ __global__ __launch_bounds__(64) void k_interp_direct2(int64_t M, const T *__res
         sim += wt[1][dy] * rim;
     }
     T *dst = out + 2 * (v * M + idx);
-    dst[0] = sre;
-    dst[1] = sim;
+    dst[0] = reach ? sre : (T)0;
+    dst[1] = reach ? sim : (T)0;
 }
 
 constexpr int kTile2Threads = 128;

@@ -499,6 +499,10 @@ __device__ inline void es_axis_weights_any(int w, T off, T beta, UniformPtr<T> c
 {
     constexpr int NE = sizeof(T) == 4 ? kPanelEven32 : kPanelEven64;
     constexpr int NO = sizeof(T) == 4 ? kPanelOdd32 : kPanelOdd64;
+    if (!on_support<T>(off)) {
+        for (int t = 0; t < w; ++t) put(t, (T)0);
+        return;
+    }
     put(0, es_weight<T>(off, w, beta));
     put(w - 1, es_weight<T>(off + (T)(w - 1), w, beta));
     const T x = off + (T)0.5 * (T)(w - 1);

@@ -51,11 +51,23 @@ __device__ inline T es_edge_weight(T d, T beta)
     }
 }
 
+// Whether an offset is that of a point's support (at most 1 - w/2, which is
+// at most zero) and not of one out of the fold's reach (kOutsideOffset, the
+// same on every axis), which weighs zero.
+template <typename T>
+__device__ inline bool on_support(T off)
+{
+    return off < (T)1;
+}
+
 // The W weights of one axis of a point, put(t, weight) for cell t of its
 // support, from its offset (start - position, in [-W/2, 1 - W/2)).  Inner
 // cells come in pairs from the panel polynomials (about 5 FMAs a weight in
 // FP32 and 8 in FP64, where sqrt and exp take 30 and 60 instructions),
-// accurate to the type's rounding; the end cells directly.
+// accurate to the type's rounding; the end cells directly.  The polynomials
+// hold on the support alone: an offset that is not on_support is the caller's
+// to leave out (a tile takes no such record, the interpolations write zero:
+// one test a point, where zero weights cost the FP64 tiles 4%).
 template <typename T, int W, typename Put>
 __device__ __forceinline__ void es_axis_weights(T off, T beta, UniformPtr<T> c, Put put)
 {

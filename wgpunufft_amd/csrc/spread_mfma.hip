@@ -181,7 +181,7 @@ k_spread_mfma3(
             if (cur.valid) {
                 int64_t ee = (int64_t)cur.sx0 - xs;
                 if (ee < 0) ee += n0;
-                take = ee < kTile + W - 1;
+                take = ee < kTile + W - 1 && on_support(cur.off.x);
                 R.sx = (int)ee - (W - 1);
                 R.sy = cur.q % NRY - (W - 1);
                 R.sz = cur.q / NRY - (W - 1);

@@ -138,7 +138,7 @@ __device__ __forceinline__ void rows3_accumulate(Rows3Stage<T> &st, TileRows<NRO
         if (cur.valid) {
             int64_t e64 = (int64_t)cur.sx0 - xs;
             if (e64 < 0) e64 += n0;
-            take = e64 < TX + W - 1;
+            take = e64 < TX + W - 1 && on_support<T>(cur.off.x);
             ee = (int)e64;
         }
         const uint64_t mask = __ballot(take);
@@ -353,7 +353,7 @@ __device__ __forceinline__ void rows2_accumulate(Rows2Stage<T> &st, TileRows<NRO
         if (cur.valid) {
             int64_t e64 = (int64_t)cur.sx0 - xs;
             if (e64 < 0) e64 += n0;
-            take = e64 < TX + W - 1;
+            take = e64 < TX + W - 1 && on_support<T>(cur.off.x);
             ee = (int)e64;
         }
         const uint64_t mask = __ballot(take);
