@@ -310,6 +310,14 @@ int tile_replay_edge(int dim, int edge2, int width, const int64_t *fine, const i
     return 0;
 }
 
+// The 1D blocks' staged range of a lane (k_spread of one dimension).
+void replay_staged_range(int64_t ka, int64_t ke, int64_t k0, int m, int *range)
+{
+    const StagedRange r = staged_range(ka, ke, k0, m);
+    range[0] = r.lo;
+    range[1] = r.hi;
+}
+
 int tile_replay(int dim, int width, const int64_t *fine, const int64_t *side,
                 const uint32_t *offsets, int64_t M, uint32_t light_limit, uint32_t min_part,
                 int64_t budget_bytes, int64_t vectors, int64_t *report)

@@ -137,3 +137,27 @@ def test_replay_catches_a_planted_offset_fault(replay_lib):
     off[len(off) // 2:] += 5000
     bad = _run(replay_lib, 2, w, fine, side, off, M)
     assert bad["violations"] > 0 and bad["code"] in (2, 3)
+
+
+def test_staged_range_of_large_blocks(replay_lib):
+    """1D blocks: the records a lane takes from the 64 staged ones, for lane
+    ranges anywhere in a block of up to 2^32 - 2 records (differences past
+    31 bits in both directions): inside the staged ones, and exactly the
+    intersection."""
+    L = replay_lib
+    L.replay_staged_range.argtypes = [ctypes.c_int64] * 3 + [ctypes.c_int, ctypes.c_void_p]
+    top = (1 << 32) - 2
+    marks = sorted({min(max(b + d, 0), top) for b in (0, 64, 1 << 30, 1 << 31, 3 << 30, top)
+                    for d in (-65, -64, -1, 0, 1, 63, 64, 100)})
+    got = (ctypes.c_int * 2)()
+    for k0 in marks:
+        m = min(64, top - k0)
+        for ka in marks:
+            for ke in (e for e in marks if e >= ka):
+                L.replay_staged_range(ka, ke, k0, m, got)
+                lo, hi = max(ka, k0) - k0, min(ke, k0 + m) - k0
+                where = (ka, ke, k0, m, got[0], got[1])
+                if lo < hi:
+                    assert (got[0], got[1]) == (lo, hi), where
+                else:
+                    assert got[0] >= got[1] and 0 <= got[0] <= m and 0 <= got[1] <= m, where

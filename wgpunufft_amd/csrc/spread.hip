@@ -577,10 +577,9 @@ __device__ __forceinline__ void spread_block(Spread1Shared<T, R> &sh, const Grid
         __syncthreads();
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
-            const int lo = (int)(ka[i] > k0 ? ka[i] - k0 : 0);
-            const int hi = (int)(ke[i] - k0 < m ? ke[i] - k0 : m);
+            const StagedRange in = staged_range(ka[i], ke[i], k0, m);
 #pragma unroll 2
-            for (int q = lo; q < hi; ++q) {
+            for (int q = in.lo; q < in.hi; ++q) {
                 const Staged1<T, R> &S = st[q];
                 int64_t e = x0 - S.s;
                 if (e < 0) e += n;

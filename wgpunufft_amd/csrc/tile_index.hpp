@@ -186,6 +186,19 @@ __host__ __device__ inline TileItem tile_item(int64_t item, int64_t block_count,
     return t;
 }
 
+// The staged records [lo, hi) that lie in a lane's range [ka, ke) of a block's
+// records, where records [k0, k0 + m) are staged.  Clamped before it narrows:
+// a block may hold up to 2^32 records.
+struct StagedRange {
+    int lo, hi;
+};
+
+__host__ __device__ inline StagedRange staged_range(int64_t ka, int64_t ke, int64_t k0, int m)
+{
+    const int64_t lo = ka - k0, hi = ke - k0;
+    return StagedRange{(int)(lo < 0 ? 0 : (lo < m ? lo : m)), (int)(hi < 0 ? 0 : (hi < m ? hi : m))};
+}
+
 // Problem of a batch's combined element t (work item, partial slot, heavy
 // tile): the last problem q whose base[4q + k] <= t.
 __host__ __device__ inline int batch_problem_of(const int64_t *__restrict__ base, int nprob, int k,
