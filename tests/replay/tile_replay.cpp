@@ -310,6 +310,23 @@ int tile_replay_edge(int dim, int edge2, int width, const int64_t *fine, const i
     return 0;
 }
 
+// Coefficients of the panel polynomials of a kernel of `width` cells as the
+// plans of a precision hold them (at most `cap` written); returns the even
+// part's count, *odd the odd part's, *n the total.
+int replay_panels(int width, double beta, int f64, double *coef, int cap, int *odd,
+                  int *n)
+{
+    EsKernel k{};
+    k.width = width;
+    k.beta = beta;
+    const int even = panel_even(f64 != 0, width);
+    *odd = panel_odd(f64 != 0, width);
+    const std::vector<double> c = es_panel_coefficients(k, even, *odd);
+    *n = (int)c.size();
+    for (int i = 0; i < *n && i < cap; ++i) coef[i] = c[(size_t)i];
+    return even;
+}
+
 // The 1D blocks' staged range of a lane (k_spread of one dimension).
 void replay_staged_range(int64_t ka, int64_t ke, int64_t k0, int m, int *range)
 {

@@ -76,11 +76,11 @@ bool es_kernel_for_tolerance(double eps, double sigma, EsKernel *out)
 
 std::vector<double> es_panel_coefficients(const EsKernel &k, int even, int odd)
 {
-    // Chebyshev interpolation of every panel on 20 nodes in long double, cut
+    // Chebyshev interpolation of every panel on 24 nodes in long double, cut
     // at the degree kept (near-minimax: the series falls geometrically, the
     // kernel's singularities lying at least one panel away), then rewritten
     // in powers of x.
-    constexpr int nodes = 20, terms = 16;
+    constexpr int nodes = 24, terms = 20;
     struct Tables {
         long double cosine[4 * nodes];    // cos(pi i / (2 nodes))
         long double power[terms][terms];  // T_j(2 x) = sum_i power[j][i] x^i

@@ -199,12 +199,14 @@ bool Plan::init_common()
     panel_off = (int64_t)table.size();
     if (precision == Precision::F32) {
         const std::vector<double> pc =
-            es_panel_coefficients(kernel, kPanelEven32, kPanelOdd32);
+            es_panel_coefficients(kernel, panel_even(false, kernel.width),
+                                  panel_odd(false, kernel.width));
         const std::vector<float> pf(pc.begin(), pc.end());
         table.resize(table.size() + (pf.size() + 1) / 2);
         if (!pf.empty()) std::memcpy(table.data() + panel_off, pf.data(), 4 * pf.size());
     } else {
-        for (double v : es_panel_coefficients(kernel, kPanelEven64, kPanelOdd64))
+        for (double v : es_panel_coefficients(kernel, panel_even(true, kernel.width),
+                                              panel_odd(true, kernel.width)))
             table.push_back(v);
     }
     if (!hip_ok(hipMalloc(&d_inv_phihat, sizeof(double) * table.size()), "amplitude table"))

@@ -493,12 +493,12 @@ struct Spread1Shared {
 };
 
 // The weights of a support of w cells (w known at run time), as
-// es_axis_weights.
-template <typename T, typename Put>
+// es_axis_weights with the coefficients of width WC; zero for a point out of
+// the fold's reach.
+template <int WC, typename T, typename Put>
 __device__ inline void es_axis_weights_any(int w, T off, T beta, UniformPtr<T> c, Put put)
 {
-    constexpr int NE = sizeof(T) == 4 ? kPanelEven32 : kPanelEven64;
-    constexpr int NO = sizeof(T) == 4 ? kPanelOdd32 : kPanelOdd64;
+    constexpr int NE = panel_even(sizeof(T) == 8, WC), NO = panel_odd(sizeof(T) == 8, WC);
     if (!on_support<T>(off)) {
         for (int t = 0; t < w; ++t) put(t, (T)0);
         return;
@@ -571,8 +571,16 @@ __device__ __forceinline__ void spread_block(Spread1Shared<T, R> &sh, const Grid
             S.s = rec_start[slot].x;
             S.cre = cv[2 * slot];
             S.cim = cv[2 * slot + 1];
-            es_axis_weights_any<T>(w, rec_off[4 * slot], beta, panels,
-                                   [&](int t, T v) { S.kx[R - 1 + t] = v; });
+            const auto put = [&](int t, T v) { S.kx[R - 1 + t] = v; };
+            const T off = rec_off[4 * slot];
+            if (w <= 4)
+                es_axis_weights_any<4>(w, off, beta, panels, put);
+            else if (w <= 6)
+                es_axis_weights_any<6>(w, off, beta, panels, put);
+            else if (w <= 8)
+                es_axis_weights_any<8>(w, off, beta, panels, put);
+            else
+                es_axis_weights_any<kMaxWidth>(w, off, beta, panels, put);
         }
         __syncthreads();
 #pragma unroll

@@ -71,8 +71,7 @@ __device__ inline bool on_support(T off)
 template <typename T, int W, typename Put>
 __device__ __forceinline__ void es_axis_weights(T off, T beta, UniformPtr<T> c, Put put)
 {
-    constexpr int NE = sizeof(T) == 4 ? kPanelEven32 : kPanelEven64;
-    constexpr int NO = sizeof(T) == 4 ? kPanelOdd32 : kPanelOdd64;
+    constexpr int NE = panel_even(sizeof(T) == 8, W), NO = panel_odd(sizeof(T) == 8, W);
     const T x = off + (T)(0.5 * (W - 1));
     const T x2 = x * x;
     put(0, es_edge_weight<T, W>(off, beta));
