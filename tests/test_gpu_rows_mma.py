@@ -58,3 +58,35 @@ def test_rows_sum_few_records(dim, prec, eps):
         rows, blocks = _both(prec, eps, n_modes, x, c)
         d = rel_l2(rows, blocks)
         assert d <= bound, f"dim {dim} {prec} w {w} M {M}: {d:.3e}"
+
+
+@pytest.mark.parametrize("sigma", [2.0, 1.25])
+@pytest.mark.parametrize("dim", [2, 3])
+@pytest.mark.parametrize("eps", [10.0 ** -e for e in range(1, 8)])
+def test_fp32_rows_are_as_exact_as_the_blocks(eps, dim, sigma):
+    """FP32 rows and blocks against the same kernel's FP64 transform: the
+    rows' weights carry no more rounding than sqrtf and expf, at the narrow
+    widths of end cells alone too (one record at a time, so that no error
+    averages out; a tenth for the spread of 400 records)."""
+    import torch
+    import wgpunufft_amd as W
+    n_modes = [20, 18, 17][:dim]
+    rng = np.random.default_rng(dim)
+    cfg = W.NufftConfig(n_modes, eps).with_sigma(sigma)
+    exact = W.NufftPlan.type1_gpu(cfg.with_precision(W.F64))
+    info = exact.info()
+    if info["width"] > 8:
+        pytest.skip("beyond the FP32 row tiles")
+    err = {}
+    x = _points(400, [2 * n for n in n_modes], dim, np.float32, rng)
+    for rows in (True, False):
+        plan = W.NufftPlan.type1_gpu(cfg).set_bin_tuning(0, rows)
+        assert plan.info()["width"] == info["width"]
+        one = torch.ones(1, dtype=torch.complex64, device="cuda")
+        got, ref = [], []
+        for p in x:
+            xt = torch.from_numpy(p[None]).cuda()
+            got.append(plan.encode_gpu(xt, one).clone())
+            ref.append(exact.encode_gpu(xt.double(), one.to(torch.complex128)).clone())
+        err[rows] = rel_l2(torch.stack(got).cpu().numpy(), torch.stack(ref).cpu().numpy())
+    assert err[True] <= 1.1 * err[False]

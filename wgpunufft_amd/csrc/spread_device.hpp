@@ -32,10 +32,14 @@ __device__ inline UniformPtr<T> panel_coefficients(const GridParams &g)
     return (UniformPtr<T>)(uintptr_t)g.panels;
 }
 
-// The weight of a support's first or last cell, at distance d: directly,
-// for W known (no division), FP32 on the hardware square root and base-2
-// exponential (these cells' weights are small from width 4 on, so the
-// cancellation in sqrt(q) - 1 does not show).
+// The weight of a support's first or last cell, at distance d: directly, for
+// W known (no division).  FP32 takes the hardware square root and base-2
+// exponential, up to width 4 of -beta s^2 / (1 + sqrt q), which does not
+// cancel near the centre; wider kernels weigh these cells so little that the
+// cancellation in sqrt(q) - 1 stays below the rounding of the other cells.
+// Largest errors at upsampling factor 2, es_weight / sqrt(q) - 1 on the
+// hardware units / this: width 2 18e-8 / 18e-8 / 8e-8, 3 24e-8 / 28e-8 /
+// 10e-8, 4 14e-8 / 17e-8 / 6e-8, 5 7e-8 / 7e-8, 6 2e-8 / 4e-8, 7 1e-8 / 1e-8.
 template <typename T, int W>
 __device__ inline T es_edge_weight(T d, T beta)
 {
@@ -43,9 +47,13 @@ __device__ inline T es_edge_weight(T d, T beta)
     const T q = (T)1 - s * s;
     if constexpr (sizeof(T) == 4) {
         const float bl = 1.44269504f * beta;
-        const float e = __builtin_amdgcn_exp2f(
-            __builtin_fmaf(__builtin_amdgcn_sqrtf(q), bl, -bl));
-        return q > 0.0f ? e : 0.0f;
+        float e;
+        if constexpr (W <= 4)
+            e = -bl * (s * s) *
+                __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_sqrtf(fmaxf(q, 0.0f)));
+        else
+            e = __builtin_fmaf(__builtin_amdgcn_sqrtf(q), bl, -bl);
+        return q > 0.0f ? __builtin_amdgcn_exp2f(e) : 0.0f;
     } else {
         return q > 0.0 ? exp(beta * (sqrt(q) - 1.0)) : 0.0;
     }
