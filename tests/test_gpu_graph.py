@@ -116,3 +116,50 @@ def test_encode_with_binning_captured_in_a_graph():
         assert torch.equal(g2.view(torch.float32).view(torch.int32),
                            e2.view(torch.float32).view(torch.int32)), f"type-2 replay {r}"
         print(f"GRAPH encode replay {r} bitwise equal", flush=True)
+
+
+@pytest.mark.parametrize("n_modes,prec,warm,count,step", [
+    ([20, 18, 17], "f32", 500, 40_000, "execute"),     # gathered, then 3D tiles
+    ([20, 18, 17], "f64", 500, 40_000, "execute"),
+    ([104, 97, 110], "f32", 300_000, 200, "execute"),  # tiles, then marked rows
+    ([104, 97, 110], "f32", 300_000, 200, "encode"),
+    ([61, 40], "f32", 140_000, 160_000, "encode"),     # unsorted, then sorted (within the slack)
+])
+def test_type2_capture_after_a_warm_up_on_another_count(n_modes, prec, warm, count, step):
+    """Which interpolation a type-2 plan runs depends on the point count; a
+    captured call may take another than the warm-up did, and finds its
+    buffers sized all the same (a plan's point buffers have a quarter of
+    slack)."""
+    import torch
+    import wgpunufft_amd as W
+    f64 = prec == "f64"
+    real, cplx = (torch.float64, torch.complex128) if f64 else (torch.float32, torch.complex64)
+    gen = torch.Generator(device="cuda").manual_seed(count)
+    x = [((2 * torch.rand(n, len(n_modes), generator=gen, device="cuda", dtype=torch.float64) - 1)
+          * 3.14159).to(real) for n in (warm, count)]
+    fm = torch.randn(int(np.prod(n_modes)), generator=gen, device="cuda", dtype=cplx)
+    out = [torch.empty(n, dtype=cplx, device="cuda") for n in (warm, count)]
+    cfg = W.NufftConfig(n_modes, 1e-6)
+    plan = W.NufftPlan.type2_gpu(cfg.with_precision(W.F64) if f64 else cfg)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        plan.encode_gpu(x[0], fm, out=out[0])
+        if step == "execute":
+            plan.set_points_gpu(x[1])
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        if step == "execute":
+            plan.execute_gpu(fm, out=out[1])
+        else:
+            plan.encode_gpu(x[1], fm, out=out[1])
+    torch.cuda.synchronize()
+    for _ in range(3):
+        fm.copy_(torch.randn(fm.numel(), generator=gen, device="cuda", dtype=cplx))
+        graph.replay()
+        torch.cuda.synchronize()
+        got = out[1].clone()
+        want = plan.encode_gpu(x[1], fm)
+        assert torch.equal(torch.view_as_real(got), torch.view_as_real(want))

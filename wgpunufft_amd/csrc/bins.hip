@@ -1278,7 +1278,7 @@ bool BinSorter::ensure(int64_t nbins, int64_t M, bool need_sort_scratch)
     }
     if (!ctrl_ && !alloc_u32(&ctrl_, 4, "bin sort counters")) return false;
     if (M > points_cap_) {
-        const int64_t cap = M + M / 4 + 1024;
+        const int64_t cap = point_capacity(M);
         // 64-bit sort keys (canonical order), else 32-bit
         if (!alloc_u32(&keys_, 2 * cap, "point keys")) return false;
         if (!alloc_u32(&keys_b_, 2 * cap, "point keys")) return false;

@@ -51,6 +51,11 @@ public:
     // Bytes bind_external needs for M points and nbins bins.
     static size_t external_bytes(int64_t nbins, int64_t M);
 
+    // Sizes the buffers of an index-order or grouped sort without sorting.
+    bool reserve(int64_t nbins, int64_t M) { return ensure(nbins, M, false); }
+    // Points that the buffers of a sort of M points take (a quarter of slack).
+    static int64_t point_capacity(int64_t M) { return M + M / 4 + 1024; }
+
     const uint32_t *sorted() const { return sorted_; }
     const uint32_t *offsets() const { return offsets_; }
     int64_t nbins() const { return nbins_; }

@@ -416,35 +416,58 @@ bool Plan::ensure_items(int64_t n)
     if (n <= item_cap) return true;
     if (item_off) (void)hipFree(item_off);
     item_off = nullptr;
+    item_cap = 0;
     if (!hip_ok(hipMalloc(&item_off, sizeof(uint32_t) * n), "interpolation items")) return false;
     item_cap = n;
     return true;
 }
 
-bool Plan::ensure_row_bits(int64_t n)
+void Plan::ensure_row_bits(int64_t n)
 {
-    if (n <= row_bits_cap) return true;
+    if (n <= row_bits_cap) return;
     if (row_bits) (void)hipFree(row_bits);
     row_bits = nullptr;
     row_bits_cap = 0;
-    if (!hip_ok(hipMalloc(&row_bits, sizeof(uint32_t) * n), "row marks")) return false;
-    row_bits_cap = n;
+    if (hipMalloc(&row_bits, sizeof(uint32_t) * n) == hipSuccess) {
+        row_bits_cap = n;
+    } else {
+        row_bits = nullptr;
+        (void)hipGetLastError();
+    }
+}
+
+// The scratch of every interpolation the plan may take, whatever the count of
+// the points now set: a later call with another count may be captured.
+bool Plan::ensure_interp_scratch()
+{
+    // bin item offsets of the tiles and the scratch of their scan
+    const int64_t bins = gp.nbins + 1;
+    if ((tiled_interp() || wide3_interp()) && !ensure_items(bins + scan_tiles(bins) + 1))
+        return false;
+    // (without its marks the last pass writes every row)
+    if (rows_grid()) ensure_row_bits(line_fft->rows_groups() * line_fft->rows_words());
     return true;
 }
 
+// Whether the grid is one that sparse_rows can hold for: 64 MB, about 14 us of
+// writes, pay for the two launches that mark the rows.
+bool Plan::rows_grid() const
+{
+    return type == 2 && dim == 3 && use_line_fft() && line_fft &&
+           2.0 * (double)real_bytes() * (double)fine_total >= 64e6;
+}
+
 // A type 2 whose gathered points read less than half of the grid's rows (of
-// rows_lines() cells along x) writes only those in the FFT's last pass, when
-// the grid is large enough (64 MB, about 14 us of writes) to pay for the two
-// launches that mark them.  900^3 FP64 cells and 37000 points of width 11
-// read 9% of the rows: last pass 5.8 -> 3.7 ms.  The tiled interpolations
+// rows_lines() cells along x) writes only those in the FFT's last pass, on a
+// large enough grid (rows_grid).  900^3 FP64 cells and 37000 points of width
+// 11 read 9% of the rows: last pass 5.8 -> 3.7 ms.  The tiled interpolations
 // read whole tiles and take the whole grid.
 bool Plan::sparse_rows(int64_t M) const
 {
-    if (type != 2 || dim != 3 || !use_line_fft() || !line_fft) return false;
+    if (!rows_grid() || !row_bits) return false;
     if (binned_interp != Interp::Unsorted && binned_interp != Interp::Gather) return false;
     const double w = kernel.width, cells = (double)fine_total;
-    return 2.0 * (double)real_bytes() * cells >= 64e6 &&
-           (double)M * w * w * (w + line_fft->rows_lines() - 1.0) < 0.5 * cells;
+    return (double)M * w * w * (w + line_fft->rows_lines() - 1.0) < 0.5 * cells;
 }
 
 bool Plan::ensure_strengths(int64_t M, int64_t vectors)
@@ -710,6 +733,10 @@ bool Plan::set_points_t(int64_t M, const T *pts, hipStream_t stream)
             mark(kStageSort, false, stream);
             if (!sorter.sort<D, T>(M, pts, gp, BinOrder::Grouped, stream)) return false;
             mark(kStageSort, true, stream);
+        } else if (!unsorted(interp_kind(BinSorter::point_capacity(M))) &&
+                   !sorter.reserve(gp.nbins, M)) {
+            // (a count within the slack may sort, and may be captured)
+            return false;
         }
     }
     points_set = true;
@@ -722,6 +749,7 @@ bool Plan::execute_t(int64_t active, const T *in, T *out, hipStream_t stream, bo
     if (fresh_marks) reset_marks();
     const int64_t M = point_count;
     if (!ensure_grid(active) || (!spread_only && !ensure_fft(active))) return false;
+    if (type == 2 && !ensure_interp_scratch()) return false;
     ModeParams mp = mode_params();
     if (type == 1) {
         if (M == 0) return fill_zero<T>(out, 2 * mode_total * active, stream);
@@ -778,8 +806,7 @@ bool Plan::execute_t(int64_t active, const T *in, T *out, hipStream_t stream, bo
                 if (sparse_rows(M)) {
                     const int words = line_fft->rows_words();
                     const int64_t groups = line_fft->rows_groups();
-                    if (!ensure_row_bits(groups * words) ||
-                        !mark_rows<T>(M, (const T *)points, gp, line_fft->rows_lines(), words,
+                    if (!mark_rows<T>(M, (const T *)points, gp, line_fft->rows_lines(), words,
                                       groups, row_bits, stream))
                         return false;
                     rows = row_bits;
@@ -795,13 +822,10 @@ bool Plan::execute_t(int64_t active, const T *in, T *out, hipStream_t stream, bo
         }
         mark_between(kStageFft, kStageInterp, stream);
         if (D == 3 && binned_interp == Interp::Tiled3) {
-            // bin item offsets and the scratch of their scan
-            if (!ensure_items(gp.nbins + 1 + scan_tiles(gp.nbins + 1) + 1)) return false;
             if (!interpolate_tiled3<T>(M, active, sorter.sorted(), sorter.offsets(), item_off,
                                        (const T *)points, gp, (const T *)grid, out, stream))
                 return false;
         } else if (D == 3 && sizeof(T) == 8 && binned_interp == Interp::Wide3) {
-            if (!ensure_items(gp.nbins + 1 + scan_tiles(gp.nbins + 1) + 1)) return false;
             if (!interpolate_wide3(M, active, sorter.sorted(), sorter.offsets(), item_off,
                                    (const double *)points, gp, (const double *)grid,
                                    (double *)out, stream))
@@ -1400,12 +1424,18 @@ bool execute_type2_many_t(int64_t count, Plan *const *plans, const int64_t *M,
     if (!head.batch_sorter) head.batch_sorter = std::make_unique<BinSorter>();
     BinSorter &bs = *head.batch_sorter;
     if (!bs.sort_many<D, float>(m_off, head.batch_table, (int)count, bins, stream)) return false;
+    if constexpr (D == 3) {
+        // work-item offsets of the combined bins and their scan scratch
+        // (whatever the counts, as ensure_interp_scratch)
+        const int64_t nb = (int64_t)bins;
+        bool tiles = false;
+        for (int64_t i = 0; i < count; ++i) tiles = tiles || plans[i]->tiled_interp();
+        if (tiles && !head.ensure_items(nb + 1 + scan_tiles(nb + 1) + 1)) return false;
+    }
     if (!widths.empty()) {
         if constexpr (D == 3) {
-            // work-item offsets of the combined bins and their scan scratch
             const int64_t nb = (int64_t)bins;
-            if (!head.ensure_items(nb + 1 + scan_tiles(nb + 1) + 1) ||
-                !interpolate_tiled3_many(bs.sorted(), bs.offsets(), head.item_off, nb,
+            if (!interpolate_tiled3_many(bs.sorted(), bs.offsets(), head.item_off, nb,
                                          head.batch_table, (int)count, widths.data(),
                                          bin_lo.data(), bin_hi.data(), class_points.data(),
                                          (int)widths.size(), stream))

@@ -123,8 +123,10 @@ struct Plan {
     int64_t item_cap = 0;
     uint32_t *row_bits = nullptr;  // cells a sparse type 2 reads (LineFft rows)
     int64_t row_bits_cap = 0;
+    bool rows_grid() const;
     bool sparse_rows(int64_t M) const;
-    bool ensure_row_bits(int64_t n);
+    bool ensure_interp_scratch();
+    void ensure_row_bits(int64_t n);
     std::map<int64_t, std::unique_ptr<FftPlan>> ffts;
     // 3D grids: the pruned line-transform FFT (fft_engine 0, where the grid
     // qualifies) or rocFFT's 3D plan (fft_engine 1).
