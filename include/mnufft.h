@@ -99,7 +99,9 @@ int mnufft_execute(mnufft_plan plan, int64_t active_batch, const void *d_in, voi
                    void *stream);
 
 /* set_points + execute: NufftPlan::encode_type{1,2}_gpu_batch
- * (src/plan.rs:808-872, 1090-1177). */
+ * (src/plan.rs:808-872, 1090-1177).  The same results; a type-2 plan may leave
+ * the points of one execute unsorted where it sorts points that are kept (set,
+ * or executed again). */
 int mnufft_encode(mnufft_plan plan, int64_t active_batch, int64_t M, const void *d_points,
                   const void *d_in, void *d_out, void *stream);
 

@@ -284,12 +284,8 @@ class NufftPlan(_PlanBase):
             raise ValueError("output tensor has the wrong type, layout or size")
         return out
 
-    def execute_gpu(self, values, out=None, active_batch=None):
-        """Type 1: strengths (active x M) -> modes; type 2: modes -> values at
-        the points (src/plan.rs:931-977, 1180-1229)."""
-        if self._points is None:
-            raise NufftError(1, "points must be set before executing")
-        M = self._points.shape[0]
+    def _vectors(self, M, values, out, active_batch):
+        """Vectors of an execution at M points, and its output."""
         modes = self.config.mode_count()
         per = M if self.kind == 1 else modes
         active = active_batch or max(1, values.numel() // max(per, 1))
@@ -297,14 +293,31 @@ class NufftPlan(_PlanBase):
             raise ValueError("values must be a contiguous tensor of the plan's complex type")
         if values.numel() < active * per:
             raise ValueError("too few input values for the active batch")
-        out = self._out(active, out, modes if self.kind == 1 else M)
+        return active, self._out(active, out, modes if self.kind == 1 else M)
+
+    def execute_gpu(self, values, out=None, active_batch=None):
+        """Type 1: strengths (active x M) -> modes; type 2: modes -> values at
+        the points (src/plan.rs:931-977, 1180-1229)."""
+        if self._points is None:
+            raise NufftError(1, "points must be set before executing")
+        active, out = self._vectors(self._points.shape[0], values, out, active_batch)
         check(lib().mnufft_execute(self._handle, active, _ptr(values), _ptr(out), _stream_ptr()))
         return out
 
     def encode_gpu(self, points, values, out=None, active_batch=None):
-        """set_points_gpu + execute_gpu (src/plan.rs:808-872, 1090-1108)."""
-        self.set_points_gpu(points)
-        return self.execute_gpu(values, out, active_batch)
+        """set_points_gpu + execute_gpu (src/plan.rs:808-872, 1090-1108), the
+        points binned for the one execution (same results)."""
+        self._check_points(points)
+        M = points.shape[0]
+        try:
+            active, out = self._vectors(M, values, out, active_batch)
+        except ValueError:
+            self.set_points_gpu(points)  # the points are set all the same
+            raise
+        self._points = points
+        check(lib().mnufft_encode(self._handle, active, M, _ptr(points), _ptr(values), _ptr(out),
+                                  _stream_ptr()))
+        return out
 
     execute_type1_gpu = execute_gpu
     execute_type2_gpu = execute_gpu

@@ -217,7 +217,9 @@ void mnufft_destroy(mnufft_plan plan)
     }
 }
 
-int mnufft_set_points(mnufft_plan plan, int64_t M, const void *d_points, void *stream)
+// once: the vectors of an encode's execute, 0 for kept points
+static int set_points_for(mnufft_plan plan, int64_t M, const void *d_points, int64_t once,
+                          void *stream)
 {
     return guarded([&] {
         if (!plan || (M > 0 && !d_points) || M < 0) {
@@ -229,9 +231,15 @@ int mnufft_set_points(mnufft_plan plan, int64_t M, const void *d_points, void *s
             return MNUFFT_ERROR_INVALID_ARGUMENT;
         }
         if (!mnufft::point_count_ok(M, "point")) return MNUFFT_ERROR_PLAN;
-        if (!plan->plan->set_points(M, d_points, (hipStream_t)stream)) return MNUFFT_ERROR_GPU;
+        if (!plan->plan->set_points(M, d_points, (hipStream_t)stream, once))
+            return MNUFFT_ERROR_GPU;
         return MNUFFT_SUCCESS;
     });
+}
+
+int mnufft_set_points(mnufft_plan plan, int64_t M, const void *d_points, void *stream)
+{
+    return set_points_for(plan, M, d_points, 0, stream);
 }
 
 int mnufft_execute(mnufft_plan plan, int64_t active_batch, const void *d_in, void *d_out,
@@ -266,7 +274,7 @@ int mnufft_execute(mnufft_plan plan, int64_t active_batch, const void *d_in, voi
 int mnufft_encode(mnufft_plan plan, int64_t active_batch, int64_t M, const void *d_points,
                   const void *d_in, void *d_out, void *stream)
 {
-    int rc = mnufft_set_points(plan, M, d_points, stream);
+    int rc = set_points_for(plan, M, d_points, active_batch > 0 ? active_batch : 1, stream);
     if (rc) return rc;
     return mnufft_execute(plan, active_batch, d_in, d_out, stream);
 }

@@ -321,27 +321,42 @@ bool Plan::tiled2_interp() const
     return true;
 }
 
-Plan::Interp Plan::interp_kind(int64_t M) const
+Plan::Interp Plan::interp_kind(int64_t M, int64_t once) const
 {
     // Unsorted while the gather's cache-line traffic (w^(d-1) rows of w cells
     // and a line of slack) stays below 128 MB, in 1D on any grid of at most
-    // 64 MB: the bin sort costs 45 to 65 us and earns the gather less.  Whole
-    // encodes / executes, sorted against unsorted: 2D w7 on 1024^2 cells, 1e5
-    // points 127 / 58 against 62 / 52 us, 4e5 160 / 60 against 88 / 78; 3D w7
-    // on 256^3, 2e4 points 237 / 170 against 181 / 171, 16e4 347 / 264 against
-    // 339 / 330; 1D w7 on 1e5 cells, 3e6 points 278 / 142 against 128 / 119.
+    // 64 MB: the bin sort costs 45 to 65 us, more than one execute gains by
+    // it.  Encodes sorted / unsorted: 2D w7 on 1024^2 cells, 1.5e5 points 122
+    // / 59 us; 3D w7 on 200^3, 2.1e4 points 162 / 102; 1D w7 on 1e5 cells, 3e6
+    // points 259 / 102.
     if (dim <= 3) {
         double rows = 1.0;
         for (int a = 1; a < dim; ++a) rows *= kernel.width;
         const double bytes = (double)M * rows * (2.0 * real_bytes() * kernel.width + 64.0);
-        if (bytes <= 128e6 || (dim == 1 && 2.0 * real_bytes() * (double)fine_total <= 64e6))
-            return tiled2_interp() ? Interp::Direct2 : Interp::Unsorted;
+        if (bytes <= 128e6 || (dim == 1 && 2.0 * real_bytes() * (double)fine_total <= 64e6)) {
+            // Points kept for many executes, and one encode of many vectors,
+            // are sorted where that gives the same sums sooner.  2D tiles of 8
+            // points and more, executes sorted / unsorted: w7 on 1024^2, 1e5
+            // points (6 a tile) 50 / 52 us, 1.5e5 (9) 50 / 59; on 184 x 136, 8
+            // vectors of 5e4 33 / 55, of 1.5e5 45 / 107.  An encode loses at
+            // most 8 us a vector at 128 MB.  3D sets, which are gathered either
+            // way, from 4 vectors on and a grid of 2 MB: 8 vectors, w7 on 200^3
+            // 685 / 700, on 64^3 95 / 112 (one vector 98 / 102 and 43 / 38), FP64
+            // on 40^3 (1 MB) 90 / 82.  1D sets gain nothing: 1e5 cells, 3e6
+            // points 126 / 102.
+            const bool many = !once || (double)once * bytes > 1e9;
+            if (dim == 2 && tiled2_interp())
+                return many && (double)M >= 8.0 * (double)type2_geometry().nbins ? Interp::Tiled2
+                                                                                 : Interp::Direct2;
+            return dim == 3 && !once && batch >= 4 && 2.0 * real_bytes() * (double)fine_total >= 2e6
+                       ? Interp::Gather
+                       : Interp::Unsorted;
+        }
     }
     // A 3D tile costs the loads of its halo, as much as gathering 20 points:
     // executes gathered against tiled, w7 on 256^3 (32768 tiles) 3.2e5 points
     // 309 against 431, 6.4e5 397 / 434, 1.3e6 599 / 450; FP64 w10 on 128^3
-    // (4096 tiles) 4e4 points 153 against 211, 8e4 230 / 216.  (A 2D tile
-    // 12 points; the sets below that are unsorted already.)
+    // (4096 tiles) 4e4 points 153 against 211, 8e4 230 / 216.
     const double tiles = (double)type2_geometry().nbins;
     if ((double)M >= 20.0 * tiles) {
         if (tiled_interp()) return Interp::Tiled3;
@@ -701,7 +716,7 @@ void Plan::reset_marks() { (void)begin_call(); }
 // Type 1 and type 2.
 // ----------------------------------------------------------------------
 template <int D, typename T>
-bool Plan::set_points_t(int64_t M, const T *pts, hipStream_t stream)
+bool Plan::set_points_t(int64_t M, const T *pts, hipStream_t stream, int64_t once)
 {
     if (!point_count_ok(M, "point")) return false;
     reset_marks();
@@ -728,12 +743,13 @@ bool Plan::set_points_t(int64_t M, const T *pts, hipStream_t stream)
         mark(kStagePrepare, true, stream);
     } else {
         gp = type2_geometry();
-        binned_interp = interp_kind(M);
+        binned_interp = interp_kind(M, once);
+        executed_once = false;
         if (!unsorted(binned_interp)) {
             mark(kStageSort, false, stream);
             if (!sorter.sort<D, T>(M, pts, gp, BinOrder::Grouped, stream)) return false;
             mark(kStageSort, true, stream);
-        } else if (!unsorted(interp_kind(BinSorter::point_capacity(M))) &&
+        } else if (!unsorted(interp_kind(BinSorter::point_capacity(M), once)) &&
                    !sorter.reserve(gp.nbins, M)) {
             // (a count within the slack may sort, and may be captured)
             return false;
@@ -749,7 +765,19 @@ bool Plan::execute_t(int64_t active, const T *in, T *out, hipStream_t stream, bo
     if (fresh_marks) reset_marks();
     const int64_t M = point_count;
     if (!ensure_grid(active) || (!spread_only && !ensure_fft(active))) return false;
-    if (type == 2 && !ensure_interp_scratch()) return false;
+    if (type == 2) {
+        // the points of an encode, executed again: kept after all (captured
+        // calls leave them, as every replay would sort them)
+        if (executed_once && unsorted(binned_interp) && !unsorted(interp_kind(M, 0))) {
+            hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+            if (hipStreamIsCapturing(stream, &capture) == hipSuccess &&
+                capture == hipStreamCaptureStatusNone &&
+                !set_points_t<D, T>(M, (const T *)points, stream))
+                return false;
+        }
+        executed_once = true;
+        if (!ensure_interp_scratch()) return false;
+    }
     ModeParams mp = mode_params();
     if (type == 1) {
         if (M == 0) return fill_zero<T>(out, 2 * mode_total * active, stream);
@@ -1109,7 +1137,7 @@ bool Plan::execute_type3_t(int64_t active, int64_t M, const T *x, const T *c, in
         if (!type3_source<D, T>(t3, M, active, x, c, (T *)t3_xr, (T *)t3_cp, stream)) return false;
         if (!spread_type3_sources<D, T>(active, M, (const T *)t3_cp, true, stream)) return false;
         if (!type3_target<D, T>(t3, N, s, (T *)t3_sr, (double *)t3_factor, stream)) return false;
-        if (!inner->set_points_t<D, T>(N, (const T *)t3_sr, stream)) return false;
+        if (!inner->set_points_t<D, T>(N, (const T *)t3_sr, stream, active)) return false;
         if (!inner->execute_t<D, T>(active, (const T *)outer->grid, (T *)t3_interp, stream, false))
             return false;
         if (!type3_final<T>(N, active, (const T *)t3_interp, (const double *)t3_factor, out,
@@ -1173,7 +1201,7 @@ bool Plan::execute_type3_t(int64_t active, int64_t M, const T *x, const T *c, in
         const T *sb = (const T *)t3_s_sorted + off * D;
         if (!type3_target<D, T>(tp, nb, sb, (T *)t3_sr, (double *)t3_factor, stream))
             return false;
-        if (!inner->set_points_t<D, T>(nb, (const T *)t3_sr, stream)) return false;
+        if (!inner->set_points_t<D, T>(nb, (const T *)t3_sr, stream, active)) return false;
         if (!inner->execute_t<D, T>(active, (const T *)outer->grid, (T *)t3_interp, stream, false))
             return false;
         if (!type3_final<T>(nb, active, (const T *)t3_interp, (const double *)t3_factor, out,
@@ -1203,9 +1231,9 @@ bool Plan::execute_type3_t(int64_t active, int64_t M, const T *x, const T *c, in
         }                                                                                         \
     } while (0)
 
-bool Plan::set_points(int64_t M, const void *pts, hipStream_t stream)
+bool Plan::set_points(int64_t M, const void *pts, hipStream_t stream, int64_t once)
 {
-#define SP(D, T) set_points_t<D, T>(M, (const T *)pts, stream)
+#define SP(D, T) set_points_t<D, T>(M, (const T *)pts, stream, once)
     MNUFFT_DISPATCH(*this, SP, SP);
 #undef SP
 }
@@ -1339,7 +1367,7 @@ bool execute_type2_many_t(int64_t count, Plan *const *plans, const int64_t *M,
     std::vector<int64_t> order((size_t)count);
     for (int64_t i = 0; i < count; ++i) order[(size_t)i] = i;
     auto tiled_w = [&](int64_t i) {
-        const Plan::Interp kind = plans[i]->interp_kind(M[i]);
+        const Plan::Interp kind = plans[i]->interp_kind(M[i], 1);
         const bool tiled = kind == Plan::Interp::Tiled2 || kind == Plan::Interp::Direct2 ||
                            kind == Plan::Interp::Tiled3;
         return tiled ? plans[i]->kernel.width : 1000;

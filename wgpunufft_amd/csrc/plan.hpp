@@ -100,11 +100,14 @@ struct Plan {
     // sums, so a batch takes its 2D plans' small sets through the tiles.
     enum class Interp { Unsorted, Direct2, Gather, Tiled3, Wide3, Tiled2 };
     static bool unsorted(Interp k) { return k == Interp::Unsorted || k == Interp::Direct2; }
-    Interp interp_kind(int64_t M) const;
+    // (for points of one encode of `once` vectors, 0: kept for many executes;
+    // a point's sum does not depend on `once`)
+    Interp interp_kind(int64_t M, int64_t once) const;
     const void *points = nullptr;
     int64_t point_count = 0;
     bool points_set = false;
     Interp binned_interp = Interp::Gather;  // type 2: of the points set
+    bool executed_once = false;             // type 2: since the points were set
     GridParams gp{};
     int geometry_index = 0;
 
@@ -206,7 +209,9 @@ struct Plan {
     void mark_between(int done, int next, hipStream_t stream);
     void reset_marks();
 
-    bool set_points(int64_t M, const void *pts, hipStream_t stream);
+    // once: the vectors of the one execute that follows (an encode), or 0 for
+    // points kept for any number of executes.
+    bool set_points(int64_t M, const void *pts, hipStream_t stream, int64_t once = 0);
     bool execute(int64_t active, const void *in, void *out, hipStream_t stream);
     // Scratch of a multi-plan type-2 execution led by this plan: the
     // combined bin sort and the device table of the problems.
@@ -230,7 +235,7 @@ struct Plan {
     bool stage_times(double *ms, int n, int64_t *calls);
 
     template <int D, typename T>
-    bool set_points_t(int64_t M, const T *pts, hipStream_t stream);
+    bool set_points_t(int64_t M, const T *pts, hipStream_t stream, int64_t once = 0);
     template <int D, typename T>
     bool execute_t(int64_t active, const T *in, T *out, hipStream_t stream, bool fresh_marks);
     template <int D, typename T>
