@@ -70,16 +70,22 @@ GridParams make_grid(int dim, int width, const int64_t *fine, const int64_t *sid
     return g;
 }
 
-// k_plan restated: the light limit doubled until the heavy blocks fit half
+// k_plan on one thread: the split rule (for an automatic plan from the
+// records in reach), the light limit doubled until the heavy blocks fit half
 // the part slots, the part length from the heavy records over the spare
 // slots, then the ordered scans of items and heavy parts.
-void plan_items(const std::vector<uint32_t> &totals, uint32_t light_limit, uint32_t min_part,
+void plan_items(const std::vector<uint32_t> &totals, SplitRule rule, bool auto_split,
                 int64_t part_capacity, std::vector<uint32_t> &parts,
                 std::vector<uint32_t> &item_off, std::vector<uint32_t> &heavy_base,
                 std::vector<uint32_t> &heavy_list, uint32_t ctrl[4], Report &rep)
 {
     const int64_t nb = (int64_t)totals.size();
-    uint32_t limit = light_limit;
+    if (auto_split) {
+        uint64_t records = 0;
+        for (uint32_t t : totals) records += t;
+        rule = auto_split_rule(records, rule);
+    }
+    uint32_t limit = rule.light_limit;
     uint64_t heavy_records = 0;
     uint32_t heavy_blocks = 0;
     for (;;) {
@@ -93,26 +99,15 @@ void plan_items(const std::vector<uint32_t> &totals, uint32_t light_limit, uint3
         if ((int64_t)heavy_blocks * 2 <= part_capacity || limit >= 0x7fffffffu) break;
         limit *= 2;
     }
-    uint64_t spare = part_capacity > (int64_t)heavy_blocks
-                         ? (uint64_t)(part_capacity - heavy_blocks)
-                         : 1ull;
-    uint64_t part = (heavy_records + spare - 1) / spare;
-    if (part < min_part) part = min_part;
-    const uint32_t part32 = (uint32_t)(part > 0xffffffffull ? 0xffffffffull : part);
+    const uint32_t part32 = part_length(heavy_records, heavy_blocks, part_capacity, rule.min_part);
     parts.assign(nb, 0);
     item_off.assign(nb + 1, 0);
     heavy_base.assign(nb + 1, 0);
     heavy_list.clear();
     uint64_t items = 0, hparts = 0;
     for (int64_t b = 0; b < nb; ++b) {
-        uint32_t np = 1, hp = 0;
-        if (totals[b] > limit) {
-            np = (uint32_t)((totals[b] + (uint64_t)part32 - 1) / part32);
-            if (np > 1)
-                hp = np;
-            else
-                np = 1;
-        }
+        const uint32_t np = block_parts(totals[b], limit, part32);
+        const uint32_t hp = np > 1 ? np : 0;
         parts[b] = np;
         item_off[b] = (uint32_t)items;
         heavy_base[b] = (uint32_t)hparts;
@@ -130,8 +125,7 @@ void plan_items(const std::vector<uint32_t> &totals, uint32_t light_limit, uint3
 
 template <int D, int TX, int TY, int TZ, int W>
 void replay(const GridParams &g, const SpreadParams &sp, const uint32_t *offsets, int64_t M,
-            uint32_t light_limit, uint32_t min_part, int64_t budget_bytes, int64_t vectors,
-            Report &rep)
+            SplitRule rule, bool auto_split, int64_t budget_bytes, int64_t vectors, Report &rep)
 {
     constexpr int NRY = TY + W - 1;
     constexpr int NROWS = D == 3 ? NRY * (TZ + W - 1) : NRY;
@@ -161,7 +155,7 @@ void replay(const GridParams &g, const SpreadParams &sp, const uint32_t *offsets
     rep.partial_floats = part_capacity * per_part * chunk / (int64_t)sizeof(float);
     std::vector<uint32_t> parts, item_off, heavy_base, heavy_list;
     uint32_t ctrl[4];
-    plan_items(totals, light_limit, min_part, part_capacity, parts, item_off, heavy_base,
+    plan_items(totals, rule, auto_split, part_capacity, parts, item_off, heavy_base,
                heavy_list, ctrl, rep);
     rep.items = ctrl[0];
     rep.heavy_parts = ctrl[1];
@@ -171,7 +165,11 @@ void replay(const GridParams &g, const SpreadParams &sp, const uint32_t *offsets
     TileRows<NROWS> rows;
     for (int64_t item = 0; item < (int64_t)ctrl[0]; ++item) {
         const TileItem ti = tile_item(item, nb, item_off.data(), parts.data(), totals.data(),
-                                      ctrl[3]);
+                                      ctrl[3], ctrl[0]);
+        // (the bounded search finds the unbounded one's tile)
+        const TileItem all = tile_item(item, nb, item_off.data(), parts.data(), totals.data(),
+                                       ctrl[3]);
+        if (ti.b != all.b || ti.p != all.p) rep.fail(kItem, item);
         if (ti.b < 0 || ti.b >= nb || ti.p < 0 || ti.p >= (int64_t)ti.np || ti.rlo > ti.rhi) {
             rep.fail(kItem, item);
             continue;
@@ -252,13 +250,13 @@ void replay(const GridParams &g, const SpreadParams &sp, const uint32_t *offsets
 
 template <int D, int TX, int TY, int TZ>
 bool replay_width(int W, const GridParams &g, const SpreadParams &sp, const uint32_t *offsets,
-                  int64_t M, uint32_t light_limit, uint32_t min_part, int64_t budget,
-                  int64_t vectors, Report &rep)
+                  int64_t M, SplitRule rule, bool auto_split, int64_t budget, int64_t vectors,
+                  Report &rep)
 {
     switch (W) {
 #define REPLAY_W(w)                                                                           \
     case w:                                                                                   \
-        replay<D, TX, TY, TZ, w>(g, sp, offsets, M, light_limit, min_part, budget, vectors, rep); \
+        replay<D, TX, TY, TZ, w>(g, sp, offsets, M, rule, auto_split, budget, vectors, rep);      \
         return true;
         REPLAY_W(2) REPLAY_W(3) REPLAY_W(4) REPLAY_W(5) REPLAY_W(6) REPLAY_W(7) REPLAY_W(8)
 #undef REPLAY_W
@@ -276,12 +274,13 @@ extern "C" {
 // bin offsets of the row geometry `side`.  report (16 values): violations,
 // first violation code, its work item, items, heavy tiles, heavy parts, part
 // length, largest slot, largest partial index, partial floats, records
-// visited, largest tile total, largest offsets index, nbins.  Returns -1 for
-// an unsupported shape.
-int tile_replay_edge(int dim, int edge2, int width, const int64_t *fine, const int64_t *side,
-                     const uint32_t *offsets, int64_t M, uint32_t light_limit, uint32_t min_part,
-                     int64_t budget_bytes, int64_t vectors, int64_t *report)
+// visited, largest tile total, largest offsets index, nbins.  auto_split: the
+// engine's own split (a plan's default).  Returns -1 for an unsupported shape.
+int tile_replay_split(int dim, int edge2, int width, const int64_t *fine, const int64_t *side,
+                      const uint32_t *offsets, int64_t M, uint32_t light_limit, uint32_t min_part,
+                      int auto_split, int64_t budget_bytes, int64_t vectors, int64_t *report)
 {
+    const SplitRule rule{light_limit, min_part};
     if (dim == 2 && edge2 != 16 && edge2 != 32) return -1;
     GridParams g = make_grid(dim, width, fine, side);
     SpreadParams sp{};
@@ -294,12 +293,12 @@ int tile_replay_edge(int dim, int edge2, int width, const int64_t *fine, const i
     }
     Report rep;
     bool ok = dim == 2 && edge2 == 32
-                  ? replay_width<2, 32, 32, 1>(width, g, sp, offsets, M, light_limit, min_part,
+                  ? replay_width<2, 32, 32, 1>(width, g, sp, offsets, M, rule, auto_split != 0,
                                                budget_bytes, vectors, rep)
-              : dim == 2 ? replay_width<2, 16, 16, 1>(width, g, sp, offsets, M, light_limit,
-                                                      min_part, budget_bytes, vectors, rep)
-              : dim == 3 ? replay_width<3, 16, 16, 8>(width, g, sp, offsets, M, light_limit,
-                                                      min_part, budget_bytes, vectors, rep)
+              : dim == 2 ? replay_width<2, 16, 16, 1>(width, g, sp, offsets, M, rule,
+                                                      auto_split != 0, budget_bytes, vectors, rep)
+              : dim == 3 ? replay_width<3, 16, 16, 8>(width, g, sp, offsets, M, rule,
+                                                      auto_split != 0, budget_bytes, vectors, rep)
                          : false;
     if (!ok) return -1;
     const int64_t v[14] = {rep.violations,  rep.first_code,    rep.first_item, rep.items,
@@ -308,6 +307,29 @@ int tile_replay_edge(int dim, int edge2, int width, const int64_t *fine, const i
                            rep.max_offset_index, g.nbins};
     for (int i = 0; i < 14; ++i) report[i] = v[i];
     return 0;
+}
+
+int tile_replay_edge(int dim, int edge2, int width, const int64_t *fine, const int64_t *side,
+                     const uint32_t *offsets, int64_t M, uint32_t light_limit, uint32_t min_part,
+                     int64_t budget_bytes, int64_t vectors, int64_t *report)
+{
+    return tile_replay_split(dim, edge2, width, fine, side, offsets, M, light_limit, min_part, 0,
+                             budget_bytes, vectors, report);
+}
+
+// The work plan of nb blocks' totals (defaults of a plan where light_limit or
+// min_part is 0): plan[0] items, [1] heavy parts, [2] heavy blocks, [3] records
+// per part, and the partial slots a batch sizes for `reach` blocks a record.
+int64_t replay_plan(const uint32_t *totals, int64_t nb, uint32_t light_limit, uint32_t min_part,
+                    int auto_split, int64_t capacity, double reach, int64_t M, uint32_t *plan)
+{
+    const SplitRule rule{light_limit ? light_limit : kLightLimit, min_part ? min_part : kMinPart};
+    std::vector<uint32_t> parts, item_off, heavy_base, heavy_list;
+    Report rep;
+    plan_items(std::vector<uint32_t>(totals, totals + nb), rule, auto_split != 0, capacity, parts,
+               item_off, heavy_base, heavy_list, plan, rep);
+    return rep.violations ? -1
+                          : part_slots_bound(nb, reach, M, rule.min_part, auto_split != 0, capacity);
 }
 
 // Coefficients of the panel polynomials of a kernel of `width` cells as the

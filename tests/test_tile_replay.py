@@ -36,22 +36,23 @@ def replay_lib():
     L = ctypes.CDLL(LIB)
     L.tile_replay.restype = ctypes.c_int
     L.tile_replay_edge.restype = ctypes.c_int
-    L.tile_replay_edge.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_void_p,
-                                   ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int64,
-                                   ctypes.c_uint32, ctypes.c_uint32, ctypes.c_int64,
-                                   ctypes.c_int64, ctypes.c_void_p]
+    L.tile_replay_split.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_void_p,
+                                    ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int64,
+                                    ctypes.c_uint32, ctypes.c_uint32, ctypes.c_int, ctypes.c_int64,
+                                    ctypes.c_int64, ctypes.c_void_p]
     return L
 
 
-def _run(L, dim, width, fine, side, offsets, M, vectors=1, edge2=32):
+def _run(L, dim, width, fine, side, offsets, M, vectors=1, edge2=32, auto=False):
     """Light limit 4096 records, parts of at least 1024, 256 MiB of partial
-    sums: the spreader's defaults (spread.hpp)."""
+    sums: the spreader's defaults (spread.hpp), split further where they leave
+    the chip idle with `auto`."""
     f = np.asarray(fine, dtype=np.int64)
     s = np.asarray(side, dtype=np.int64)
     off = np.ascontiguousarray(offsets, dtype=np.uint32)
     rep = np.zeros(16, dtype=np.int64)
-    rc = L.tile_replay_edge(dim, edge2, width, f.ctypes.data, s.ctypes.data, off.ctypes.data, M,
-                            4096, 1024, 256 << 20, vectors, rep.ctypes.data)
+    rc = L.tile_replay_split(dim, edge2, width, f.ctypes.data, s.ctypes.data, off.ctypes.data, M,
+                             4096, 1024, int(auto), 256 << 20, vectors, rep.ctypes.data)
     assert rc == 0
     return dict(zip(FIELDS, rep.tolist()))
 
@@ -112,6 +113,18 @@ def test_replay_2d_plain_row_tiles_at_5e7_points(replay_lib):
     r = _run(replay_lib, 2, w, fine, side, _offsets(fine, w, side, x), M, edge2=16)
     print("REPLAY 2D rows clustered", r)
     assert r["violations"] == 0, r
+
+
+@pytest.mark.parametrize("M", [100_000, 1_000_000])
+def test_replay_automatic_split(replay_lib, M):
+    """Small sets on 256^2 cells, tiles cut into the automatic split's parts:
+    every index in bounds, and more waves of work than tiles."""
+    fine, w = [256, 256], 7
+    side = _row_side(fine)
+    x = S.uniform_coords(S.config_seed(3, 1), M, 2)
+    r = _run(replay_lib, 2, w, fine, side, _offsets(fine, w, side, x), M, edge2=16, auto=True)
+    assert r["violations"] == 0, r
+    assert r["heavy_tiles"] == 256 and 1000 <= r["items"] <= 256 + 2048
 
 
 def test_replay_3d_tiles_at_1e7_clustered_points(replay_lib):

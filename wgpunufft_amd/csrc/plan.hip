@@ -1567,11 +1567,7 @@ bool execute_type1_many_t(int64_t count, Plan *const *plans, const int64_t *M,
         q.light_limit = p.spreader.light_limit;
         q.min_part = p.spreader.min_part;
         q.auto_split = p.spreader.auto_split ? 1u : 0u;
-        // partial slots the problem's heavy parts can take: at most its
-        // capacity, and at most a part per heavy block plus its records in
-        // reach (each record counted by at most `reach` blocks) over the
-        // smallest part, with a factor two of margin, or (the automatic
-        // split) kAutoWaves parts of an even share
+        // blocks that may count one record of the problem
         double reach = 1.0;
         for (int a = 0; a < D; ++a) {
             const int64_t B = sp.block[a], n = p.fine[a];
@@ -1582,10 +1578,8 @@ bool execute_type1_many_t(int64_t count, Plan *const *plans, const int64_t *M,
                                   ? all
                                   : std::min<int64_t>(all, (side + p.kernel.width + 2 * B - 3) / B + 1));
         }
-        double most = 2.0 * reach * (double)M[i] / (double)std::max<uint32_t>(q.min_part, 1);
-        if (q.auto_split) most = std::max(most, (double)kAutoWaves);
-        const double bound = (double)sp.block_count + most;
-        k.slots += std::min<int64_t>(q.part_capacity, (int64_t)std::min(bound, 9.0e15));
+        k.slots += part_slots_bound(sp.block_count, reach, M[i], q.min_part, q.auto_split != 0,
+                                    q.part_capacity);
         k.blocks += sp.block_count;
         k.p1 = (int)r + 1;
         ModeProblem &mq = mtable[(size_t)r];

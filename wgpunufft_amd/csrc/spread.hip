@@ -55,15 +55,6 @@ __global__ __launch_bounds__(256) void k_classify(GridParams g, SpreadParams sp,
     if (lane == 0) totals[b] = (uint32_t)(total > 0xffffffffull ? 0xffffffffull : total);
 }
 
-// A plan whose split is left to the engine aims at this many waves of work
-// (256 CUs by 4 SIMDs, twice over) while its blocks hold few records: parts
-// of an even share of the records in reach, at least kAutoPart of them (below
-// that a part's fixed cost, its reach rows and its partial sums, outweighs
-// the shorter chain), and blocks of more than two such parts are split.
-// 1e5 points on 256^2 cells (256 tiles of 740 records in reach, one wave
-// each): spread 41 -> 12 us.
-constexpr uint32_t kAutoPart = 128;
-
 // One workgroup plans the work items: a light block is one item, a heavy
 // block as many parts as its records need.  ctrl[0] = items, ctrl[1] = heavy
 // parts, ctrl[2] = heavy blocks, ctrl[3] = records per part.  A thread takes
@@ -97,13 +88,9 @@ __device__ inline void plan_blocks(int64_t nblocks, const uint32_t *__restrict__
         for (int o = 32; o > 0; o >>= 1) mine += __shfl_xor(mine, o, 64);
         if (lane == 0) atomicAdd(&s_records, mine);
         __syncthreads();
-        const unsigned long long share = (s_records + kAutoWaves - 1) / kAutoWaves;
-        const uint32_t part = share > kAutoPart ? (uint32_t)(share < 0x3fffffffull ? share : 0x3fffffffull)
-                                                : kAutoPart;
-        if (2 * part < light_limit) {
-            light_limit = 2 * part;
-            min_part = part < min_part ? part : min_part;
-        }
+        const SplitRule r = auto_split_rule(s_records, SplitRule{light_limit, min_part});
+        light_limit = r.light_limit;
+        min_part = r.min_part;
     }
     // Raise the light limit until the heavy blocks fill at most half of the
     // partial-sum slots, so every heavy block keeps room for several parts.
@@ -137,15 +124,7 @@ __device__ inline void plan_blocks(int64_t nblocks, const uint32_t *__restrict__
         }
         __syncthreads();
     }
-    uint32_t part;
-    {
-        const uint64_t spare = part_capacity > (int64_t)s_heavy_blocks
-                                   ? (uint64_t)(part_capacity - s_heavy_blocks)
-                                   : 1ull;
-        uint64_t len = (s_heavy_records + spare - 1) / spare;
-        if (len < min_part) len = min_part;
-        part = (uint32_t)(len > 0xffffffffull ? 0xffffffffull : len);
-    }
+    const uint32_t part = part_length(s_heavy_records, s_heavy_blocks, part_capacity, min_part);
     // Ordered exclusive scans of items and heavy parts.
     uint32_t carry_items = 0, carry_parts = 0;
     for (int64_t base = 0; base < nblocks; base += (int64_t)blockDim.x * kPlanRun) {
@@ -155,10 +134,9 @@ __device__ inline void plan_blocks(int64_t nblocks, const uint32_t *__restrict__
         for (int j = 0; j < kPlanRun; ++j) {
             np[j] = 0;
             if (b0 + j < nblocks) {
-                const uint32_t t = totals[b0 + j];
                 // a block that fits one part is written directly (np == 1
                 // means light to the tile kernels and the reduction)
-                np[j] = t > light_limit ? (uint32_t)((t + (uint64_t)part - 1) / part) : 1u;
+                np[j] = block_parts(totals[b0 + j], light_limit, part);
             }
             items += np[j];
             heavy += np[j] > 1 ? np[j] : 0u;

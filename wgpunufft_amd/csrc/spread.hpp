@@ -4,6 +4,7 @@
 #include <vector>
 
 #include "nufft_internal.hpp"
+#include "tile_index.hpp"
 
 namespace mnufft {
 
@@ -63,10 +64,6 @@ struct SpreadProblem {
     uint32_t light_limit, min_part;
     uint32_t auto_split;
 };
-
-// Waves of work that a plan with few records in reach is split for (plan_blocks
-// in spread.hip): its heavy parts are then at most this many and one a block.
-constexpr uint32_t kAutoWaves = 2048;
 
 // A class of consecutive problems [p0, p1) of one run length (or of the row
 // tiles and one kernel width): its blocks
@@ -142,8 +139,8 @@ struct Spreader {
     // smallest part; with auto_split both are lowered for point sets that
     // would leave the chip idle (never by a caller's or the autotuner's own
     // values).
-    uint32_t light_limit = 4096;
-    uint32_t min_part = 1024;
+    uint32_t light_limit = kLightLimit;
+    uint32_t min_part = kMinPart;
     bool auto_split = true;
     // Partial-sum slots of one vector, and the scratch a chunk of vectors
     // may take (the chunk is at least one vector).

@@ -143,6 +143,69 @@ __host__ __device__ inline uint32_t tile_slot(const TileRows<NROWS> &rows, uint3
     return j < rows.n0[lo] ? rows.f0[lo] + j : rows.f1[lo] + (j - rows.n0[lo]);
 }
 
+// The split of a type-1 work plan.  A block of more than light_limit records in
+// reach is cut into parts of at least min_part.  A plan whose split is left to
+// the engine aims at kAutoWaves waves of work (256 CUs by 4 SIMDs, twice over)
+// while its blocks hold few records: parts of an even share of the records in
+// reach, at least kAutoPart of them (below that a part's fixed cost, its reach
+// rows and its partial sums, outweighs the shorter chain), and blocks of more
+// than two such parts are split.  1e5 points on 256^2 cells (256 tiles of 740
+// records in reach, one wave each): spread 41 -> 12 us.
+constexpr uint32_t kLightLimit = 4096, kMinPart = 1024;
+constexpr uint32_t kAutoWaves = 2048, kAutoPart = 128;
+
+struct SplitRule {
+    uint32_t light_limit, min_part;
+};
+
+// The rule of an automatic plan with `records` in reach of its blocks.
+__host__ __device__ inline SplitRule auto_split_rule(uint64_t records, SplitRule r)
+{
+    const uint64_t share = (records + kAutoWaves - 1) / kAutoWaves;
+    const uint32_t part =
+        share > kAutoPart ? (uint32_t)(share < 0x3fffffffull ? share : 0x3fffffffull) : kAutoPart;
+    if (2 * part < r.light_limit) {
+        r.light_limit = 2 * part;
+        r.min_part = part < r.min_part ? part : r.min_part;
+    }
+    return r;
+}
+
+// Records per part of a plan whose heavy blocks hold `records`, given the
+// partial-sum slots: every heavy block keeps one.
+__host__ __device__ inline uint32_t part_length(uint64_t records, uint32_t heavy_blocks,
+                                                int64_t capacity, uint32_t min_part)
+{
+    const uint64_t spare =
+        capacity > (int64_t)heavy_blocks ? (uint64_t)(capacity - heavy_blocks) : 1ull;
+    uint64_t len = (records + spare - 1) / spare;
+    if (len < min_part) len = min_part;
+    return (uint32_t)(len > 0xffffffffull ? 0xffffffffull : len);
+}
+
+// Parts of a block: more than one only for a heavy block, whose parts take
+// partial-sum slots.
+__host__ __device__ inline uint32_t block_parts(uint32_t total, uint32_t light_limit,
+                                                uint32_t part)
+{
+    return total > light_limit ? (uint32_t)((total + (uint64_t)part - 1) / part) : 1u;
+}
+
+// Partial slots that a plan's heavy parts can take: at most its capacity, and
+// at most a part per block plus the records in reach (`reach` blocks may count
+// each of M) over the smallest part, with a factor two of margin, or (the
+// automatic split) kAutoWaves parts of an even share.
+inline int64_t part_slots_bound(int64_t blocks, double reach, int64_t M, uint32_t min_part,
+                                bool auto_split, int64_t capacity)
+{
+    double most = 2.0 * reach * (double)M / (double)(min_part > 1 ? min_part : 1);
+    if (auto_split && most < (double)kAutoWaves) most = (double)kAutoWaves;
+    const double bound = (double)blocks + most;
+    return capacity < (int64_t)(bound < 9.0e15 ? bound : 9.0e15)
+               ? capacity
+               : (int64_t)(bound < 9.0e15 ? bound : 9.0e15);
+}
+
 // Work item -> (tile, part, record range) of the tile plan.  With the number
 // of items, the search starts from the tiles that can hold the item: every
 // tile has an item, so tile b starts between item b and item b plus the
