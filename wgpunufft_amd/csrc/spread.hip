@@ -551,11 +551,12 @@ __device__ __forceinline__ void spread_block(Spread1Shared<T, R> &sh, const Grid
             S.cim = cv[2 * slot + 1];
             const auto put = [&](int t, T v) { S.kx[R - 1 + t] = v; };
             const T off = rec_off[4 * slot];
-            if (w <= 4)
+            // (FP32: one count of coefficients for every width)
+            if (sizeof(T) == 8 && w <= 4)
                 es_axis_weights_any<4>(w, off, beta, panels, put);
-            else if (w <= 6)
+            else if (sizeof(T) == 8 && w <= 6)
                 es_axis_weights_any<6>(w, off, beta, panels, put);
-            else if (w <= 8)
+            else if (sizeof(T) == 8 && w <= 8)
                 es_axis_weights_any<8>(w, off, beta, panels, put);
             else
                 es_axis_weights_any<kMaxWidth>(w, off, beta, panels, put);
