@@ -280,8 +280,12 @@ int mnufft_set_point_order(mnufft_plan plan, int32_t order);
  * parts of at least min_part records, with partial sums in slots of at most
  * part_budget_bytes per vector (the light limit is raised until the heavy
  * tiles fit half the slots).  Zero keeps a knob's current value (defaults
- * 4096, 1024, 256 MiB).  Results stay bitwise repeatable for fixed knobs;
- * other knobs change the summation order of heavy tiles only.
+ * 4096, 1024, 256 MiB).  While both the light limit and the smallest part are
+ * at their defaults, whether set or not, point sets that would leave the chip
+ * idle are split further: into parts of an even share of the records over 2048
+ * waves, at least 128 records each, from tiles of more than two such parts.
+ * Results stay bitwise repeatable for fixed knobs; other knobs change the
+ * summation order of heavy tiles only.
  */
 int mnufft_set_spread_tuning(mnufft_plan plan, int64_t light_limit, int64_t min_part,
                              int64_t part_budget_bytes);

@@ -142,7 +142,8 @@ class _PlanBase:
     def set_spread_tuning(self, light_limit=0, min_part=0, part_budget_bytes=0):
         """Work-plan knobs of the type-1 spread (0 keeps the current value):
         records above which a tile is split into parts, the smallest part,
-        and the partial-sum budget per vector in bytes."""
+        and the partial-sum budget per vector in bytes.  With the first two
+        at their defaults, small point sets are split further."""
         check(lib().mnufft_set_spread_tuning(self._handle, int(light_limit), int(min_part),
                                              int(part_budget_bytes)))
         return self

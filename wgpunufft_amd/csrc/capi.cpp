@@ -712,7 +712,9 @@ int mnufft_set_spread_tuning(mnufft_plan plan, int64_t light_limit, int64_t min_
     Plan &q = p.type == 3 && p.outer ? *p.outer : p;
     if (light_limit) q.spreader.light_limit = (uint32_t)light_limit;
     if (min_part) q.spreader.min_part = (uint32_t)min_part;
-    if (light_limit || min_part) q.spreader.auto_split = false;
+    // the automatic split is the default values' own
+    q.spreader.auto_split = q.spreader.light_limit == mnufft::kLightLimit &&
+                            q.spreader.min_part == mnufft::kMinPart;
     if (part_budget_bytes) q.spreader.budget_bytes = part_budget_bytes;
     return MNUFFT_SUCCESS;
 }

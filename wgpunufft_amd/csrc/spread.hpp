@@ -136,9 +136,8 @@ struct Spreader {
     int64_t vmax_cap = 0;
     int64_t part_capacity = 0;
     // Records in reach above which a block is split into parts, and the
-    // smallest part; with auto_split both are lowered for point sets that
-    // would leave the chip idle (never by a caller's or the autotuner's own
-    // values).
+    // smallest part; with auto_split (both at their defaults) both are
+    // lowered for point sets that would leave the chip idle.
     uint32_t light_limit = kLightLimit;
     uint32_t min_part = kMinPart;
     bool auto_split = true;
