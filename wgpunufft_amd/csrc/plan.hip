@@ -406,23 +406,30 @@ bool Plan::ensure_grid(int64_t vectors)
     return true;
 }
 
-bool Plan::ensure_records(int64_t M)
+// Records of M points; their starts only for plans that read them.
+bool Plan::ensure_records(int64_t M, bool starts)
 {
-    if (M <= rec_cap) return true;
-    if (rec_start) (void)hipFree(rec_start);
-    if (rec_off) (void)hipFree(rec_off);
-    if (rec_perm) (void)hipFree(rec_perm);
-    rec_start = nullptr;
-    rec_off = nullptr;
-    rec_perm = nullptr;
-    int64_t cap = M + M / 4 + 64;
-    const size_t quads = dim <= 3 ? 1 : 2;  // rec_quads of the plan's rank
-    if (!hip_ok(hipMalloc(&rec_start, sizeof(int4) * quads * cap), "prepared starts"))
-        return false;
-    if (!hip_ok(hipMalloc(&rec_off, 4 * quads * real_bytes() * cap), "prepared offsets"))
-        return false;
-    if (!hip_ok(hipMalloc(&rec_perm, sizeof(uint32_t) * cap), "record permutation")) return false;
-    rec_cap = cap;
+    const int64_t quads = dim <= 3 ? 1 : 2;  // rec_quads of the plan's rank
+    if (M > rec_cap) {
+        if (rec_off) (void)hipFree(rec_off);
+        if (rec_perm) (void)hipFree(rec_perm);
+        rec_off = nullptr;
+        rec_perm = nullptr;
+        rec_cap = 0;
+        const int64_t cap = M + M / 4 + 64;
+        if (!hip_ok(hipMalloc(&rec_off, 4 * quads * real_bytes() * cap), "prepared offsets") ||
+            !hip_ok(hipMalloc(&rec_perm, sizeof(uint32_t) * cap), "record permutation"))
+            return false;
+        rec_cap = cap;
+    }
+    if (starts && M > start_cap) {
+        if (rec_start) (void)hipFree(rec_start);
+        rec_start = nullptr;
+        start_cap = 0;
+        if (!hip_ok(hipMalloc(&rec_start, sizeof(int4) * quads * rec_cap), "prepared starts"))
+            return false;
+        start_cap = rec_cap;
+    }
     return true;
 }
 
@@ -730,15 +737,16 @@ bool Plan::set_points_t(int64_t M, const T *pts, hipStream_t stream, int64_t onc
         binned_order = point_order;
         binned_dense = sizeof(T) == 4 ? dense_threshold(gp) : 0u;
         mark(kStageSort, false, stream);
-        if (!ensure_records(M)) return false;
+        // the row tiles read no starts; the blocks and the dense windows do
+        const bool starts = !gp_rows || binned_dense;
+        if (!ensure_records(M, starts)) return false;
         if (!sorter.sort<D, T>(M, pts, gp, point_order, stream)) return false;
         mark_between(kStageSort, kStagePrepare, stream);
         if (binned_dense && !dense.classify(gp, spread_params(), sorter.offsets(), stream))
             return false;
-        // the row tiles read no starts; the blocks and the dense windows do
-        int4 *starts = gp_rows && !binned_dense ? nullptr : rec_start;
-        if (!sorter.prepare<D, T>(M, pts, gp, point_order, starts, (T *)rec_off, rec_perm,
-                                  stream, binned_dense ? dense.before : nullptr))
+        if (!sorter.prepare<D, T>(M, pts, gp, point_order, starts ? rec_start : nullptr,
+                                  (T *)rec_off, rec_perm, stream,
+                                  binned_dense ? dense.before : nullptr))
             return false;
         mark(kStagePrepare, true, stream);
     } else {
@@ -887,8 +895,10 @@ bool Plan::bin_sort_t(int64_t M, const T *pts, uint32_t *sorted, uint32_t *offse
     reset_marks();
     mark(kStageSort, false, stream);
     if (!sorter.sort<D, T>(M, pts, g, BinOrder::Index, stream)) return false;
-    if (!ensure_records(M)) return false;
-    if (!sorter.prepare<D, T>(M, pts, g, BinOrder::Index, rec_start, (T *)rec_off, sorted, stream))
+    // (only the permutation is wanted; the records of ranks above 3 hold both)
+    if (!ensure_records(M, D > 3)) return false;
+    if (!sorter.prepare<D, T>(M, pts, g, BinOrder::Index, D > 3 ? rec_start : nullptr,
+                              (T *)rec_off, sorted, stream))
         return false;
     mark(kStageSort, true, stream);
     if (offsets &&
@@ -1606,7 +1616,7 @@ bool execute_type1_many_t(int64_t count, Plan *const *plans, const int64_t *M,
         bool blocks = false;  // a class on the output-stationary blocks reads the starts
         for (const SpreadClass &k : classes) blocks = blocks || k.run != 0;
         if (!bs.sort_many<D, T>(m_off, head.batch_table, (int)count, bins, stream) ||
-            !head.ensure_records(m_off) || !head.ensure_strengths(m_off, 1) ||
+            !head.ensure_records(m_off, blocks) || !head.ensure_strengths(m_off, 1) ||
             !prepare_many<D, T>(m_off, bs.sorted(), head.batch_table, (int)count,
                                 blocks ? head.rec_start : nullptr, (T *)head.rec_off,
                                 head.rec_perm, stream) ||

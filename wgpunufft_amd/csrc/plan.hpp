@@ -119,7 +119,7 @@ struct Plan {
     int4 *rec_start = nullptr;
     void *rec_off = nullptr;
     uint32_t *rec_perm = nullptr;  // original index of every record slot (type 1)
-    int64_t rec_cap = 0;
+    int64_t rec_cap = 0, start_cap = 0;
     void *c_sorted = nullptr;
     size_t c_sorted_bytes = 0;
     uint32_t *item_off = nullptr;  // work items of the tiled interpolation
@@ -193,7 +193,7 @@ struct Plan {
     ModeParams mode_params() const;
     size_t real_bytes() const;
     bool ensure_grid(int64_t vectors);
-    bool ensure_records(int64_t M);
+    bool ensure_records(int64_t M, bool starts);
     bool ensure_strengths(int64_t M, int64_t vectors);
     bool ensure_items(int64_t n);
     bool tiled_interp() const;
