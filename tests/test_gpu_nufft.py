@@ -569,3 +569,23 @@ def test_batch_beyond_2_32_values():
     sel = torch.arange(0, M, 97, device="cuda")
     r2 = W.reference_type2_f64(n_modes, x.double(), fm.to(torch.complex128), points=sel)
     assert rel_l2(cb[B - 1][sel].cpu().numpy(), r2.cpu().numpy()) <= 32e-6
+
+
+@pytest.mark.parametrize("n_modes", [[40, 30], [200]])
+def test_bin_sort_of_other_points_leaves_the_kept_ones(n_modes):
+    """bin_sort works in the plan's own scratch: an execute after it runs on
+    the points that were set, whatever was sorted meanwhile."""
+    torch, W, O, S = _setup()
+    d = len(n_modes)
+    x = torch.from_numpy(S.uniform_coords(S.config_seed(1, 95), 3000, d)).cuda()
+    c = torch.from_numpy(S.complex_normal(S.config_seed(1, 96), 3000)).cuda()
+    plan = W.NufftPlan.type1_gpu(W.NufftConfig(n_modes, 1e-6))
+    want = plan.encode_gpu(x, c).clone()
+    order = plan.points_permutation()[0].clone()
+    for M in (500, 20000):
+        other = torch.from_numpy(S.uniform_coords(S.config_seed(1, M), M, d)).cuda()
+        plan.bin_sort(other)
+        got = plan.execute_gpu(c)
+        assert torch.equal(torch.view_as_real(got), torch.view_as_real(want))
+        plan.bin_sort(other)
+        assert torch.equal(plan.points_permutation()[0], order)

@@ -430,6 +430,10 @@ int mnufft_points_permutation(mnufft_plan plan, uint32_t *d_sorted, uint32_t *d_
             return MNUFFT_ERROR_INVALID_ARGUMENT;
         }
         Plan &p = *plan->plan;
+        // (a bin_sort since works in the same scratch: binned again)
+        if (p.points_set && !p.records_set &&
+            !p.set_points(p.point_count, p.points, (hipStream_t)stream))
+            return MNUFFT_ERROR_GPU;
         if (!p.points_set || p.binned_dense != 0u) {
             set_error(p.points_set ? "dense bins keep their records apart from the bin order"
                                    : "no points are binned");

@@ -730,6 +730,7 @@ bool Plan::set_points_t(int64_t M, const T *pts, hipStream_t stream, int64_t onc
     points = pts;
     point_count = M;
     points_set = false;
+    records_set = false;
     if (type == 1) {
         gp = spread_geometry(M, &geometry_index);
         gp_rows = rows_geometry();
@@ -748,6 +749,7 @@ bool Plan::set_points_t(int64_t M, const T *pts, hipStream_t stream, int64_t onc
                                   (T *)rec_off, rec_perm, stream,
                                   binned_dense ? dense.before : nullptr))
             return false;
+        records_set = true;
         mark(kStagePrepare, true, stream);
     } else {
         gp = type2_geometry();
@@ -789,9 +791,9 @@ bool Plan::execute_t(int64_t active, const T *in, T *out, hipStream_t stream, bo
     ModeParams mp = mode_params();
     if (type == 1) {
         if (M == 0) return fill_zero<T>(out, 2 * mode_total * active, stream);
-        // a spread method that needs other bins, or another in-bin order,
-        // re-bins the kept points
-        if ((gp_rows != rows_geometry() || binned_order != point_order ||
+        // a spread method that needs other bins, another in-bin order or a
+        // sort of other points (bin_sort) re-bins the kept points
+        if ((!records_set || gp_rows != rows_geometry() || binned_order != point_order ||
              binned_side0 != rows_side0 ||
              binned_dense != (sizeof(T) == 4 ? dense_threshold(gp) : 0u)) &&
             !set_points_t<D, T>(M, (const T *)points, stream))
@@ -892,6 +894,7 @@ bool Plan::bin_sort_t(int64_t M, const T *pts, uint32_t *sorted, uint32_t *offse
 {
     if (!point_count_ok(M, "point")) return false;
     GridParams g = type1_geometry(M, nullptr);
+    records_set = false;  // the sort and the records are these points' now
     reset_marks();
     mark(kStageSort, false, stream);
     if (!sorter.sort<D, T>(M, pts, g, BinOrder::Index, stream)) return false;

@@ -106,6 +106,7 @@ struct Plan {
     const void *points = nullptr;
     int64_t point_count = 0;
     bool points_set = false;
+    bool records_set = false;  // type 1: the records are those of the points set
     Interp binned_interp = Interp::Gather;  // type 2: of the points set
     bool executed_once = false;             // type 2: since the points were set
     GridParams gp{};
