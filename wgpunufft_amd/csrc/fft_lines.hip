@@ -380,13 +380,15 @@ __device__ __forceinline__ void for_kept(const LineFftKept &m, int i, int nb, in
 //
 // What bounds the passes: HBM for FP32 (512^3, 4 vectors: x 1.55 ms, y 0.75
 // ms, 4.1 and 4.3 TB/s where a copy reaches 4.6), HBM latency on the short
-// rows of long FP64 axes (900^3: x 1.6, y 2.3, z 6.4 ms, 2.7 to 3.7 TB/s).
-// The vector ALU bounded them before (x 2.1, y 1.0 ms; 900^3 1.8, 2.7, 7.1
-// ms): an address product, a window test and index divisions for every
-// element, divisions of the pass constants in every thread and five small
-// radices at 900 took 124 (FP32) and 156 (FP64) instructions an element; now
-// one 64-bit pointer a butterfly stepped by a uniform stride, windows as
-// masks over t, constants from the host and the largest radices: 56 and 77.
+// rows of long FP64 axes (900^3: x 1.5, y 2.2 ms, z 5.8 ms for every row, 3.7
+// ms for the marked ones of a sparse type 2).  The vector ALU bounded them
+// before (x 2.1, y 1.0 ms; 900^3 1.8, 2.7, 7.1 ms): an address product, a
+// window test and index divisions for every element, divisions of the pass
+// constants in every thread and five small radices at 900 took 124 (FP32) and
+// 156 (FP64) instructions an element; now one 64-bit pointer a butterfly
+// stepped by a uniform stride, windows as masks over t, constants from the
+// host and the largest radices: 56 and 77.
+
 // One butterfly index of the workgroup: line c, butterfly i of the line.
 template <typename T>
 __device__ inline void butterfly(const LineFftAxis &P, const LineFftPass &ps, int b, int *c, int *i)
@@ -764,10 +766,6 @@ LineFftKept kept_masks(int r, int n, int hi, int lo)
     return m;
 }
 
-// Lines per workgroup: the lines and the twiddle table fit the LDS array;
-// along the contiguous axis a line per thread at least, else few enough
-// lines for about 2048 workgroups (`count` lines in all), small groups
-// sharing a CU.
 // Whether the line kernels may take the wide LDS budget (set once).
 bool wide_lds()
 {
@@ -789,7 +787,10 @@ bool wide_lds()
     return ok;
 }
 
-// `wide`: the 80 KB budget, else 64 KB (the support test uses 64 KB).
+// Lines per workgroup: the lines and the twiddle table fit the LDS array
+// (`wide`: the 80 KB budget, else 64 KB); along the contiguous axis an element
+// per thread at least and few enough groups for about 2048 workgroups (`count`
+// lines in all), small groups sharing a CU.
 bool group_lines(int n, bool line_major, bool f64, int64_t count, bool wide, LineFftAxis *ax)
 {
     const int lds = f64 ? (wide ? LdsElems<double>::value : LdsElems<double>::base)

@@ -742,7 +742,7 @@ __global__ __launch_bounds__(THREADS) void k_interp_tiled2(
 // the sums of k_interp_tiled2 (cell by cell along x, then row by row: the
 // same bits) with the rows read from the grid, which a set this small leaves
 // in the caches.  No sort and no tile: 1e4 points on 184 x 136 cells at width
-// 6 take one launch where sort and tiles took eight (encode 85 -> 27 us with
+// 6 take one launch where sort and tiles took eight (encode 85 -> 30 us with
 // the FFT's own changes).
 template <typename T, int W>
 __global__ __launch_bounds__(64) void k_interp_direct2(int64_t M, const T *__restrict__ coords,
