@@ -40,7 +40,10 @@ __device__ inline UniformPtr<T> panel_coefficients(const GridParams &g)
 // Largest errors at upsampling factor 2, es_weight / sqrt(q) - 1 on the
 // hardware units / this: width 2 18e-8 / 18e-8 / 8e-8, 3 24e-8 / 28e-8 /
 // 10e-8, 4 14e-8 / 17e-8 / 6e-8, 5 7e-8 / 7e-8, 6 2e-8 / 4e-8, 7 1e-8 / 1e-8.
-template <typename T, int W>
+// SPLIT: weights that become FP16 or BF16 operands, rounded to 2^-21 at best,
+// take the shorter form at every width (width 4, 9.3e6 points: an execute 873
+// us, 884 with the other).
+template <typename T, int W, bool SPLIT>
 __device__ inline T es_edge_weight(T d, T beta)
 {
     const T s = d * (T)(2.0 / W);
@@ -48,7 +51,7 @@ __device__ inline T es_edge_weight(T d, T beta)
     if constexpr (sizeof(T) == 4) {
         const float bl = 1.44269504f * beta;
         float e;
-        if constexpr (W <= 4)
+        if constexpr (W <= 4 && !SPLIT)
             e = -bl * (s * s) *
                 __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_sqrtf(fmaxf(q, 0.0f)));
         else
@@ -76,14 +79,14 @@ __device__ inline bool on_support(T off)
 // hold on the support alone: an offset that is not on_support is the caller's
 // to leave out (a tile takes no such record, the interpolations write zero:
 // one test a point, where zero weights cost the FP64 tiles 4%).
-template <typename T, int W, typename Put>
+template <typename T, int W, bool SPLIT = false, typename Put>
 __device__ __forceinline__ void es_axis_weights(T off, T beta, UniformPtr<T> c, Put put)
 {
     constexpr int NE = panel_even(sizeof(T) == 8, W), NO = panel_odd(sizeof(T) == 8, W);
     const T x = off + (T)(0.5 * (W - 1));
     const T x2 = x * x;
-    put(0, es_edge_weight<T, W>(off, beta));
-    put(W - 1, es_edge_weight<T, W>(off + (T)(W - 1), beta));
+    put(0, es_edge_weight<T, W, SPLIT>(off, beta));
+    put(W - 1, es_edge_weight<T, W, SPLIT>(off + (T)(W - 1), beta));
 #pragma unroll
     for (int t = 1; t <= (W - 1) / 2; ++t) {
         UniformPtr<T> e = c + (t - 1) * (NE + NO), o = e + NE;

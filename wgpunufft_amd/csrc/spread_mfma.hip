@@ -218,7 +218,8 @@ k_spread_mfma3(
                         const float o = axis == 0 ? S.ox : (axis == 1 ? S.oy : S.oz);
                         float *tb = axis == 0 ? KX : (axis == 1 ? KY : KZ);
                         const unsigned lim = axis == 2 ? TZ : kTile;
-                        es_axis_weights<float, W>(o, (float)g.beta, panels, [&](int t, float wt) {
+                        es_axis_weights<float, W, true>(o, (float)g.beta, panels,
+                                                        [&](int t, float wt) {
                             const unsigned c = (unsigned)(s + t);
                             const unsigned row = c < lim ? c : (unsigned)kTile;
                             tb[row * kPitch + j] = wt;
