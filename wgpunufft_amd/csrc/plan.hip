@@ -475,8 +475,8 @@ bool Plan::ensure_interp_scratch()
 // writes, pay for the two launches that mark the rows.
 bool Plan::rows_grid() const
 {
-    return type == 2 && dim == 3 && use_line_fft() && line_fft &&
-           2.0 * (double)real_bytes() * (double)fine_total >= 64e6;
+    return type == 2 && dim == 3 && line_fft &&
+           2.0 * (double)real_bytes() * (double)fine_total >= 64e6 && use_line_fft();
 }
 
 // A type 2 whose gathered points read less than half of the grid's rows (of
