@@ -16,7 +16,8 @@ pytestmark = pytest.mark.gpu
     ([40, 40], 20_000, 8, True, False),
     ([40, 40], 20_000, 96, True, True),   # an encode of over 1e9 bytes of gathers
     ([32, 36, 35], 3000, 1, False, False), ([32, 36, 35], 3000, 4, True, False),
-    ([16, 18, 17], 3000, 4, False, False)])
+    ([16, 18, 17], 3000, 4, False, False),
+    ([104, 97, 110], 300, 4, True, False)])   # the last FFT pass on marked rows
 def test_kept_points_give_the_bits_of_encodes(n_modes, M, batch, kept_sorted, encode_sorted, prec,
                                               eps):
     import torch

@@ -22,7 +22,7 @@ def test_row_tile_plans_hold_no_starts():
     plan.set_points_gpu(x)
     rows = _used(torch)
     plan.set_points_gpu(x)
-    assert _used(torch) == rows
+    assert _used(torch) <= rows + margin
     plan.set_bin_tuning(0, False)  # the output-stationary blocks read them
     plan.set_points_gpu(x)
     assert _used(torch) - rows >= 16 * M - margin
