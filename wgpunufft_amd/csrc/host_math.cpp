@@ -74,13 +74,16 @@ bool es_kernel_for_tolerance(double eps, double sigma, EsKernel *out)
     return true;
 }
 
-std::vector<double> es_panel_coefficients(const EsKernel &k, int even, int odd)
+namespace {
+
+// Chebyshev interpolation of every panel on `nodes` nodes in long double, cut
+// at the degree kept (near-minimax: the series falls geometrically, the
+// kernel's singularities lying at least one panel away), then rewritten in
+// powers of x.
+template <int nodes>
+std::vector<double> fit_panels(const EsKernel &k, int even, int odd)
 {
-    // Chebyshev interpolation of every panel on 24 nodes in long double, cut
-    // at the degree kept (near-minimax: the series falls geometrically, the
-    // kernel's singularities lying at least one panel away), then rewritten
-    // in powers of x.
-    constexpr int nodes = 24, terms = 20;
+    constexpr int terms = 20;
     struct Tables {
         long double cosine[4 * nodes];    // cos(pi i / (2 nodes))
         long double power[terms][terms];  // T_j(2 x) = sum_i power[j][i] x^i
@@ -120,6 +123,16 @@ std::vector<double> es_panel_coefficients(const EsKernel &k, int even, int odd)
         for (int i = 0; i < odd; ++i) out.push_back(middle ? 0.0 : power(2 * i + 1));
     }
     return out;
+}
+
+}  // namespace
+
+std::vector<double> es_panel_coefficients(const EsKernel &k, int even, int odd)
+{
+    // three nodes more than the degree: what they alias is below its rounding
+    const int degree = std::max(2 * even - 2, 2 * odd - 1);
+    return degree <= 10 ? fit_panels<14>(k, even, odd)
+                        : degree <= 15 ? fit_panels<19>(k, even, odd) : fit_panels<22>(k, even, odd);
 }
 
 // Lengths rocFFT runs with its own radix kernels: prime factors 2..13.
